@@ -391,20 +391,21 @@ int device_cus() {
   return n;
 }
 
-// Split count of a decode launch: enough splits to give every CU kDecodeWGsPerCU work-groups
-// (each split walks cps consecutive 128-key chunks), at most decode_splits_max.
-struct DecodeSplit {
-  int nChunks, cps, nSplits;
-};
-DecodeSplit decode_split(int batch, int heads_kv, int seq_kv) {
-  DecodeSplit d{};
-  d.nChunks = static_cast<int>(decode_chunks(seq_kv));
+// Split count of a decode launch over equal lengths: an equal run of 128-key chunks for each of
+// kDecodeWGsPerCU work-groups per CU (decode_cps), at most decode_splits_max.  One split needs no
+// merge launch, which costs as much as two to three more chunks in one work-group's walk: 8.5
+// against 10.4 us at 2 chunks, 11.2 against 11.9 at 3 and 13.4 against 12.0 at 4 (B1, Hq32/Hkv8,
+// D128, bf16; B16: 9.8 against 13.2 at 2, 14.1 against 15.7 at 4).
+constexpr int kDecodeDirectChunks = 3;
+constexpr int kDecodeRaggedSplits = 4;
+int decode_splits(int batch, int heads_kv, int seq_kv, int slots) {
+  const int chunks = static_cast<int>(decode_chunks(seq_kv));
   const long long units = static_cast<long long>(batch) * heads_kv;
-  const long long want = (static_cast<long long>(coalibi::kDecodeWGsPerCU) * device_cus() + units - 1) / units;
-  const int splits = static_cast<int>(std::max(1LL, std::min<long long>(want, decode_splits_max(seq_kv))));
-  d.cps = (d.nChunks + splits - 1) / splits;
-  d.nSplits = (d.nChunks + d.cps - 1) / d.cps;
-  return d;
+  if (chunks <= kDecodeDirectChunks || units >= slots) return 1;
+  const int cps = coalibi::decode_cps(units * chunks, chunks, slots, coalibi::kMaxDecodeSplits,
+                                      [&](int c) { return units * ((chunks + c - 1) / c); });
+  const int n = (chunks + cps - 1) / cps, own = (chunks + n - 1) / n;
+  return (chunks + own - 1) / own;  // in equal runs
 }
 
 // Bytes of split-K partials for `parts` (batch, query head, split) triples: the maximum, the sum
@@ -469,9 +470,10 @@ int decode_impl(const char* fn, bool scratch_ws, int dtype, const void* q, const
                                      std::to_string(coalibi::kMaxDecodeChunks * coalibi::kDecodeChunkKeys));
   // The workspace size first: it depends on the shape only, and a decode whose partials do not fit
   // is refused before any pointer is looked at.
-  const DecodeSplit sp = decode_split(batch, heads_kv, seq_kv);
+  const int slots = coalibi::kDecodeWGsPerCU * device_cus();
+  int splits = decode_splits(batch, heads_kv, seq_kv, slots);
   const size_t rows = static_cast<size_t>(batch) * heads_q;
-  const size_t parts = rows * (scratch_ws ? static_cast<size_t>(sp.nSplits) : decode_splits_max(seq_kv));
+  size_t parts = rows * (scratch_ws ? static_cast<size_t>(splits) : decode_splits_max(seq_kv));
   const size_t need = decode_partials_bytes(parts, head_dim);
   if (workspace_bytes < need) {
     if (scratch_ws)
@@ -488,6 +490,17 @@ int decode_impl(const char* fn, bool scratch_ws, int dtype, const void* q, const
     return rc;
   if (!std::isfinite(sm_scale)) return fail(CO_ALIBI_EINVAL, std::string(fn) + ": sm_scale must be finite");
 
+  if (seq_lens != nullptr && splits > 1) {
+    // Lengths below seq_kv leave work-groups to the longer sequences, up to kDecodeRaggedSplits
+    // times as many splits each, where their partials fit.
+    const size_t most = std::min(static_cast<size_t>(splits) * kDecodeRaggedSplits, decode_splits_max(seq_kv));
+    for (size_t n = most; n > static_cast<size_t>(splits); n = n / 2)
+      if (decode_partials_bytes(rows * n, head_dim) <= workspace_bytes) {
+        splits = static_cast<int>(n);
+        break;
+      }
+    if (scratch_ws) parts = rows * splits;
+  }
   const size_t stat_bytes = round_up(parts * sizeof(float), 256);
   char* ws = static_cast<char*>(workspace);
   coalibi::DecodeArgs a{};
@@ -508,9 +521,9 @@ int decode_impl(const char* fn, bool scratch_ws, int dtype, const void* q, const
   a.G = heads_q / heads_kv;
   a.L = seq_kv;
   a.cap = kv_capacity;
-  a.nChunks = sp.nChunks;
-  a.cps = sp.cps;
-  a.nSplits = sp.nSplits;
+  a.nSplits = splits;
+  a.cps = static_cast<int>((decode_chunks(seq_kv) + splits - 1) / splits);
+  a.slots = slots;
   a.sc2 = sm_scale * coalibi::kLog2eHost;
   hipStream_t st = static_cast<hipStream_t>(stream);
   hipError_t e;

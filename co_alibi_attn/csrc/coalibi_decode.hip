@@ -15,7 +15,7 @@
 //      accumulator rows, the group's query heads on the columns), z from the sigma
 //      suffix inside the split only, the split's softmax partial (max, sum, O = P V on
 //      MFMA) and its sigma total.
-//   2. merge: per (batch, query head).  The keys after chunk c add the same amount
+//   2. merge (not with one split per sequence): per (batch, query head).  The keys after chunk c add the same amount
 //      off_c = sum_{c' > c} sigma_total[c'] to z_j of every key of chunk c, which
 //      shifts a_j of the whole chunk by -slope*log2(e)*off_c and leaves its sum and
 //      O partial unchanged once the maximum is shifted by the same amount.  The
@@ -24,6 +24,8 @@
 // K and V go to per-wavefront LDS tiles by buffer-to-LDS DMA, each issued one chunk ahead
 // as soon as its tile has been read; K is read back as the MFMA A operand, V as the k-major
 // B operand of P V.
+#include <algorithm>
+
 #include "coalibi_common.h"
 #include "coalibi_kernels.h"
 
@@ -34,7 +36,79 @@ namespace {
 constexpr int kDecWaves = 4;
 constexpr int kDecWaveKeys = 32;  // keys per wavefront: one 32-key MFMA tile
 constexpr int kDecMergeThreads = 256;
-static_assert(kDecWaves * kDecWaveKeys == kDecodeChunkKeys, "chunk = the work-group's keys");
+
+__device__ __forceinline__ int decode_chunks_of(int len) { return (len + kDecodeChunkKeys - 1) / kDecodeChunkKeys; }
+
+template <typename V, typename F>
+__device__ __forceinline__ V wave_reduce(V x, const F& f) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) x = f(x, __shfl_xor(x, off, 64));
+  return x;
+}
+
+// The filled rows of sequence b: per-sequence lengths are clamped to [0, L].
+__device__ __forceinline__ int seq_len_of(const DecodeArgs& a, int b) {
+  return a.seq_lens == nullptr ? a.L : min(max(a.seq_lens[b], 0), a.L);
+}
+
+// Chunks per split of a launch with a length per sequence (every wavefront computes the same): the
+// splits share out the batch's real chunks, so that every work-group streams an equal part of the
+// caches.  Splits sized by the longest sequence leave the work-groups past a shorter one's end
+// idle, and the longest one's walk on alone: 16 sequences of 1024 to 8192 keys (Hq32/Hkv8, D128,
+// bf16) take 60.8 us, against 69.3 that way.
+__device__ __forceinline__ int chunks_per_split(const DecodeArgs& a, int lane) {
+  int total = 0, longest = 0;
+  for (int b = lane; b < a.B; b += 64) {
+    const int n = decode_chunks_of(seq_len_of(a, b));
+    total += n;
+    longest = max(longest, n);
+  }
+  total = wave_reduce(total, [](int x, int y) { return x + y; });
+  longest = wave_reduce(longest, [](int x, int y) { return max(x, y); });
+  return decode_cps(static_cast<long long>(total) * a.Hkv, longest, a.slots, a.nSplits, [&](int c) {
+    int n = 0;
+    for (int b = lane; b < a.B; b += 64) n += (decode_chunks_of(seq_len_of(a, b)) + c - 1) / c;
+    return static_cast<long long>(wave_reduce(n, [](int x, int y) { return x + y; })) * a.Hkv;
+  });
+}
+
+// A sequence's own splits: as many as cps chunks each make, then of equal length; `used` hold keys.
+struct SeqSplits {
+  int n, cps, used;
+};
+__device__ __forceinline__ SeqSplits seq_splits(int chunks, int cps) {
+  const int n = max((chunks + cps - 1) / cps, 1), own = max((chunks + n - 1) / n, 1);
+  return {n, own, (chunks + own - 1) / own};
+}
+
+// The (batch, kv head, split) of a work-group of a launch with a length per sequence: the ids run
+// over the sequences' own splits, split fastest, and ids past the last one have none (bhk < 0).
+struct SplitItem {
+  int bhk, split;
+};
+__device__ __forceinline__ SplitItem split_item(const DecodeArgs& a, int cps, int lane) {
+  int before = 0;  // ids of the sequences passed
+  const int id = blockIdx.x;
+  for (int b0 = 0; b0 < a.B; b0 += 64) {
+    const int b = b0 + lane;
+    const int n = b < a.B ? seq_splits(decode_chunks_of(seq_len_of(a, b)), cps).n : 0;
+    int incl = n * a.Hkv;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int o = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += o;
+    }
+    const unsigned long long in = __ballot(id < before + incl);
+    if (in != 0) {
+      const int l = __ffsll(in) - 1;
+      const int splits = __shfl(n, l, 64), at = id - before - (__shfl(incl, l, 64) - splits * a.Hkv);
+      const int hkv = at / splits;
+      return {__builtin_amdgcn_readfirstlane((b0 + l) * a.Hkv + hkv), __builtin_amdgcn_readfirstlane(at - hkv * splits)};
+    }
+    before += __shfl(incl, 63, 64);
+  }
+  return {-1, 0};
+}
 
 template <typename T, int D>
 struct DecCfg {
@@ -133,7 +207,12 @@ __device__ __forceinline__ void ld_k_fragments(typename Mfma<T>::vec8 (&f)[KS], 
 constexpr int vmcnt_imm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
 constexpr int kLgkmcnt0 = 15 | (3 << 14) | (7 << 4);
 
-template <typename T, int D>
+// How a launch splits its sequences: evenly, by a plan over a length per sequence (RAGGED), or not
+// at all (DIRECT, nSplits == 1): the work-group then writes o and lse itself and no merge is
+// launched.
+enum class Split { kEven, kRagged, kDirect };
+
+template <typename T, int D, Split SPLIT>
 __global__ __launch_bounds__(kDecWaves * 64, (D > 128 || sizeof(T) == 4) ? 1 : 2) void coalibi_decode_split_kernel(
     DecodeArgs a) {
   using M = Mfma<T>;
@@ -151,22 +230,28 @@ __global__ __launch_bounds__(kDecWaves * 64, (D > 128 || sizeof(T) == 4) ? 1 : 2
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int hl = lane & 31, hh = lane >> 5;
-  const int split = blockIdx.x, bhk = blockIdx.y;
+  constexpr bool kRagged = SPLIT == Split::kRagged, kDirect = SPLIT == Split::kDirect;
+  // Without a plan: a (split, b * Hkv + hkv) grid.
+  SplitItem item{(int)blockIdx.y, (int)blockIdx.x};
+  int cps = a.cps;
+  if constexpr (kRagged) {
+    cps = chunks_per_split(a, lane);
+    item = split_item(a, cps, lane);
+    if (item.bhk < 0) return;
+  }
+  const int split = item.split, bhk = item.bhk;
   const int G = a.G, nS = a.nSplits;
   const int b = bhk / a.Hkv, hkv = bhk - b * a.Hkv;
-  // This sequence's cache length (per-sequence lengths clamped to [0, L]).
-  const int L = a.seq_lens == nullptr ? a.L : min(max(a.seq_lens[b], 0), a.L);
+  const int L = SPLIT == Split::kEven ? a.L : seq_len_of(a, b);  // kEven: no lengths
   const int hq0 = hkv * G;  // first query head of the group
   const size_t bh0 = (size_t)b * a.Hq + hq0;
-  const int c_first = split * a.cps;
-  const int c_last = min(c_first + a.cps, (L + kDecodeChunkKeys - 1) / kDecodeChunkKeys) - 1;
-  if (c_last < c_first) {  // the split lies past this sequence's length: an empty partial
-    for (int i = tid; i < G * D; i += kDecWaves * 64) a.pout[((bh0 + i / D) * nS + split) * D + i % D] = 0.f;
-    if (tid < G) {
-      const size_t pi = (bh0 + tid) * nS + split;
-      a.pmax[pi] = kNegInf;
-      a.psum[pi] = 0.f;
-      a.psig[pi] = 0.f;
+  if constexpr (kRagged) cps = seq_splits(decode_chunks_of(L), cps).cps;
+  const int c_first = split * cps;
+  const int c_last = min(c_first + cps, decode_chunks_of(L)) - 1;
+  if (c_last < c_first) {  // an empty sequence: no partial (the merge reads none)
+    if constexpr (kDirect) {
+      for (int i = tid; i < G * D; i += kDecWaves * 64) static_cast<T*>(a.o)[bh0 * D + i] = T(0);
+      if (tid < G && a.lse != nullptr) a.lse[bh0 + tid] = kNegInf;
     }
     return;
   }
@@ -339,10 +424,15 @@ __global__ __launch_bounds__(kDecWaves * 64, (D > 128 || sizeof(T) == 4) ? 1 : 2
       sScale[w][h] = f;
       l += f * sSum[w][h];
     }
-    const size_t pi = (bh0 + h) * nS + split;
-    a.pmax[pi] = m;  // finite: the split's first key is below this sequence's length
-    a.psum[pi] = l;
-    a.psig[pi] = carry;
+    if constexpr (kDirect) {  // the whole sequence: normalise here, as the merge does
+      sSum[0][h] = l;
+      if (a.lse != nullptr) a.lse[bh0 + h] = l > 0.f ? (m + log2f(l)) * kLn2 : kNegInf;
+    } else {
+      const size_t pi = (bh0 + h) * nS + split;
+      a.pmax[pi] = m;  // finite: the split's first key is below this sequence's length
+      a.psum[pi] = l;
+      a.psig[pi] = carry;
+    }
   }
   __syncthreads();  // sScale ready; every wavefront is done with its tiles (no DMA in flight)
 
@@ -365,7 +455,12 @@ __global__ __launch_bounds__(kDecWaves * 64, (D > 128 || sizeof(T) == 4) ? 1 : 2
     float s = 0.f;
 #pragma unroll
     for (int w = 0; w < kDecWaves; ++w) s += o_row(w, h)[d];
-    a.pout[((bh0 + h) * nS + split) * D + d] = s;
+    if constexpr (kDirect) {
+      const float l = sSum[0][h];
+      static_cast<T*>(a.o)[(bh0 + h) * D + d] = static_cast<T>(l > 0.f ? s / l : 0.f);
+    } else {
+      a.pout[((bh0 + h) * nS + split) * D + d] = s;
+    }
   }
 }
 
@@ -391,7 +486,7 @@ __device__ __forceinline__ float wave_sum(float x) {
 }
 
 // O and LSE of one (batch, query head) from its split partials.
-template <typename T, int D>
+template <typename T, int D, bool RAGGED>
 __global__ __launch_bounds__(kDecMergeThreads) void coalibi_decode_merge_kernel(DecodeArgs a) {
   constexpr int NW = kDecMergeThreads / 64;
   constexpr int PARTS = kDecMergeThreads / D;
@@ -400,11 +495,14 @@ __global__ __launch_bounds__(kDecMergeThreads) void coalibi_decode_merge_kernel(
   __shared__ float sAcc[PARTS][D];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const size_t bh = blockIdx.x;
-  const int nS = a.nSplits;
   const float lam2 = a.slopes[bh % a.Hq] * kLog2e;
-  const float* pmax = a.pmax + bh * nS;
-  const float* psum = a.psum + bh * nS;
-  const float* psig = a.psig + bh * nS;
+  // The splits that wrote a partial.
+  int nS = a.nSplits;
+  if constexpr (RAGGED)
+    nS = seq_splits(decode_chunks_of(seq_len_of(a, bh / a.Hq)), chunks_per_split(a, lane)).used;
+  const float* pmax = a.pmax + bh * a.nSplits;
+  const float* psum = a.psum + bh * a.nSplits;
+  const float* psig = a.psig + bh * a.nSplits;
 
   // Exclusive suffix sums of the split sigma totals, 256 splits at a time from the end; the
   // maximum of split s moves by -slope*log2(e) times the sigma of every later split.
@@ -438,8 +536,7 @@ __global__ __launch_bounds__(kDecMergeThreads) void coalibi_decode_merge_kernel(
 #pragma unroll
   for (int w = 0; w < NW; ++w) m = fmaxf(m, sRed[w]);
   __syncthreads();
-  // Empty splits (past a sequence's length) have maximum -inf and weight 0; a sequence
-  // of length 0 has no split with a key: O = 0 and LSE = -inf.
+  // A sequence of length 0 has no split: O = 0 and LSE = -inf.
   const float mref = m == kNegInf ? 0.f : m;
   float l = 0.f;
   for (int c = tid; c < nS; c += kDecMergeThreads) {
@@ -456,7 +553,7 @@ __global__ __launch_bounds__(kDecMergeThreads) void coalibi_decode_merge_kernel(
 
   // O: thread (part, d) sums the splits part, part + PARTS, ... with eight loads in flight.
   const int d = tid % D, part = tid / D;
-  const float* po = a.pout + bh * nS * D + d;
+  const float* po = a.pout + bh * a.nSplits * D + d;
   float acc[8];
 #pragma unroll
   for (int u = 0; u < 8; ++u) acc[u] = 0.f;
@@ -481,11 +578,27 @@ __global__ __launch_bounds__(kDecMergeThreads) void coalibi_decode_merge_kernel(
 
 template <typename T, int D>
 hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream) {
-  hipLaunchKernelGGL((coalibi_decode_split_kernel<T, D>), dim3(a.nSplits, a.B * a.Hkv), dim3(kDecWaves * 64), 0,
-                     stream, a);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((coalibi_decode_merge_kernel<T, D>), dim3(a.B * a.Hq), dim3(kDecMergeThreads), 0, stream, a);
+  const dim3 threads(kDecWaves * 64), merge_grid(a.B * a.Hq), merge_threads(kDecMergeThreads);
+  const dim3 even(a.nSplits, a.B * a.Hkv);
+  if (a.nSplits == 1) {
+    hipLaunchKernelGGL((coalibi_decode_split_kernel<T, D, Split::kDirect>), even, threads, 0, stream, a);
+    return hipGetLastError();
+  }
+  if (a.seq_lens == nullptr) {
+    hipLaunchKernelGGL((coalibi_decode_split_kernel<T, D, Split::kEven>), even, threads, 0, stream, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((coalibi_decode_merge_kernel<T, D, false>), merge_grid, merge_threads, 0, stream, a);
+  } else {
+    // At most one round of work-groups and a rounded-up split per sequence and kv head (decode_cps
+    // shares the chunks out over `slots`).
+    const long long units = static_cast<long long>(a.B) * a.Hkv;
+    const dim3 grid(static_cast<unsigned>(std::min(units * a.nSplits, a.slots + units)));
+    hipLaunchKernelGGL((coalibi_decode_split_kernel<T, D, Split::kRagged>), grid, threads, 0, stream, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((coalibi_decode_merge_kernel<T, D, true>), merge_grid, merge_threads, 0, stream, a);
+  }
   return hipGetLastError();
 }
 

@@ -179,9 +179,10 @@ struct BwdArgs {
 
 // Decode: q/o (B, Hq, D); the caches k/v are (B, Hkv, cap, D) with the first L rows
 // of every head valid (or the first seq_lens[b] rows of sequence b, at most L).  The
-// keys form nChunks chunks of kDecodeChunkKeys; split s of a head covers chunks
-// [s*cps, (s+1)*cps).  Split-K partials per (b*Hq + h, split): pmax / psum / psig
-// (B*Hq, nSplits) and pout (B*Hq, nSplits, D), fp32.
+// keys of a sequence form chunks of kDecodeChunkKeys; split s of a head covers chunks
+// [s*cps, (s+1)*cps), with cps from decode_cps below.  Split-K partials per (b*Hq + h, split):
+// pmax / psum / psig (B*Hq, nSplits) and pout (B*Hq, nSplits, D), fp32; unused with one split,
+// whose work-group writes o and lse itself.
 constexpr int kDecodeChunkKeys = 128;
 constexpr int kMaxDecodeGroup = 32;     // query heads per kv head (MFMA tile columns)
 constexpr int kMaxDecodeChunks = 16384;  // bounds seq_kv (2^21 keys)
@@ -199,12 +200,29 @@ struct DecodeArgs {
   float* psig;
   float* pout;
   const int* seq_lens;  // (B,) per-sequence cache lengths, or NULL (all L)
-  int B, Hq, Hkv, G, L, cap, nChunks, cps, nSplits;
+  int B, Hq, Hkv, G, L, cap;
+  int nSplits;  // most splits of any sequence: the partials' stride
+  int cps;      // chunks per split without seq_lens (with them the kernels share the chunks out)
+  int slots;    // resident work-groups the splits are sized for
   float sc2;
 };
 
 // Split-K work-groups the decode aims at per CU: one round of the two that are resident.
 constexpr int kDecodeWGsPerCU = 2;
+
+// Chunks per split of a decode over sequences with `work` chunks in all (summed over the kv heads;
+// `longest` in the longest one): an equal share of `work` per resident work-group, or up to
+// half as much again where that brings groups(c), the work-groups that c chunks per split make,
+// into one round of `slots`.  At most `max_splits` splits per sequence.  The same rule on the host
+// (one length) and in the kernels (a length per sequence), so equal lengths split alike.
+template <typename F>
+__host__ __device__ inline int decode_cps(long long work, int longest, int slots, int max_splits, const F& groups) {
+  const int share = static_cast<int>((work + slots - 1) / slots), fit = (longest + max_splits - 1) / max_splits;
+  const int c0 = share > fit ? (share > 1 ? share : 1) : (fit > 1 ? fit : 1);
+  for (int c = c0; c <= c0 + c0 / 2 + 1; c += 1 + c / 16)
+    if (groups(c) <= slots) return c;
+  return c0;
+}
 
 // Forward; with a.knorm (the tail skip) it first launches the key-norm kernel that fills it.
 template <typename T, int D, bool CAUSAL>

@@ -220,3 +220,44 @@ def test_decode_random_batches(case):
         ro, rlse = oracle_decode(q[b:b + 1], k[b:b + 1], v[b:b + 1], n)
         check(f"o[{b}] (len {n})", o[b:b + 1], ro, TOL[dtype])
         check(f"lse[{b}] (len {n})", lse[b:b + 1], rlse, TOL[dtype])
+
+
+# Ragged batches at the edges of the split plan: more sequences than a wavefront's lanes, empty ones
+# first and last, one long sequence among empty ones (its splits are capped), lengths around the
+# chunk of 128, and batches with a work-group per head (one split, no merge launch).
+PLAN_CASES = [
+    ("B70", [0] + [130 * i % 1500 for i in range(68)] + [0], 8, 2, 1500, 64),
+    ("one_long", [0, 0, 20000, 0, 0], 8, 2, 20000, 64),
+    ("chunk_edges", [127, 128, 129, 255, 256, 257, 384, 385], 6, 3, 2000, 32),
+    ("all_empty", [0, 0, 0], 4, 4, 1000, 64),
+    ("direct", [384, 1, 0, 129, 383], 16, 4, 384, 128),
+    ("head_each", [700, 0, 1, 900], 128, 128, 900, 32),
+]
+
+
+@pytest.mark.parametrize("case", PLAN_CASES, ids=lambda c: c[0])
+def test_decode_split_plan(case):
+    _, lens, Hq, Hkv, cap, D = case
+    print(f"case {case[0]}", flush=True)
+    q, k, v = cache_inputs(len(lens), Hq, Hkv, cap, cap, D, torch.float16, seed=31)
+    for b, n in enumerate(lens):
+        k[b, :, n:] = 100.0
+        v[b, :, n:] = -1000.0
+    seq = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    o, lse = co_alibi_decode(q.to(DEV), k.to(DEV), v.to(DEV), seq_len=seq, return_lse=True)
+    torch.cuda.synchronize()
+    for b, n in enumerate(lens):
+        if n == 0:
+            assert not o[b].any() and torch.isneginf(lse[b]).all()
+            continue
+        ro, rlse = oracle_decode(q[b:b + 1], k[b:b + 1], v[b:b + 1], n)
+        check(f"o[{b}] (len {n})", o[b:b + 1], ro, TOL[torch.float16])
+        check(f"lse[{b}] (len {n})", lse[b:b + 1], rlse, TOL[torch.float16])
+
+
+@pytest.mark.parametrize("L", [384, 385, 1100, 8200])
+def test_decode_equal_lengths_split_alike(L):
+    """A batch of equal lengths gives the same bits with and without a length tensor."""
+    q, k, v = (t.to(DEV) for t in cache_inputs(3, 8, 2, L, L, 64, torch.bfloat16, seed=7))
+    seq = torch.full((3,), L, dtype=torch.int64, device=DEV)
+    assert torch.equal(co_alibi_decode(q, k, v, seq_len=seq), co_alibi_decode(q, k, v))
