@@ -184,6 +184,7 @@ int fwd_impl(const char* fn, int dtype, const void* q, const void* k, const void
   a.o = o;
   a.lse = lse;
   const bool skip = g_tail_skip.load() != 0;
+  a.every_key = !skip;
   if (stats != nullptr) {  // header, kstart, knorm and the work orders (coalibi_kernels.h)
     const StatsLayout l = stats_layout(batch, heads_q, seq_q, seq_kv);
     int* words = reinterpret_cast<int*>(stats);

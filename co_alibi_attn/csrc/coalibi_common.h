@@ -481,3 +481,102 @@ __device__ __forceinline__ float sum8(f32x8 v, float acc) {
 }
 
 }  // namespace coalibi
+
+// One wavefront with 32 keys of its own (the decode and the kernels that split a row block's keys
+// over their wavefronts): its K and V tiles are private, so it loads and waits alone.
+namespace coalibi {
+
+constexpr int kWaveKeys = 32;  // keys per wavefront: one 32-key MFMA tile
+
+// Buffer-to-LDS DMA of the kWaveKeys rows row0.. of a row-major [nrows][D] matrix into
+// one wavefront's tile (the layout of DmaTile<T, D, kWaveKeys, LD, 1, PERM>): every
+// instruction reads 64 consecutive 16-byte chunks.  STREAM: non-temporal, for data read once.
+// Rows past nrows, pad chunks and the tail after the last row land as zeros.  The source offsets
+// are recomputed from an opaque copy of the lane index at every issue; hoisted out of the chunk
+// loop they would hold a register per instruction for the whole kernel.
+template <typename T, int D, int LD, bool PERM, bool STREAM>
+__device__ __forceinline__ void dma_wave_rows(const T* base, int row0, int nrows, T* lds, int lane) {
+  using Tile = DmaTile<T, D, kWaveKeys, LD, 1, PERM>;
+  const __amdgpu_buffer_rsrc_t r = tile_rsrc(base + (size_t)row0 * D, min(max(nrows - row0, 0), kWaveKeys) * D);
+  int ln;
+  asm volatile("v_mov_b32 %0, %1" : "=v"(ln) : "v"(lane));
+#pragma unroll
+  for (int m = 0; m < Tile::NINSTR; ++m) {
+    const int ch = m * 64 + ln, row = ch / Tile::CPR, j = ch - row * Tile::CPR;
+    const int src = PERM ? (row & ~31) + kRowOfReg(row & 31) : row;
+    const bool in_tile = row < kWaveKeys && j < D / Tile::CH;
+    const int off = in_tile ? (src * D + j * Tile::CH) * (int)sizeof(T) : 0x40000000;
+    if constexpr (STREAM)
+      dma16_to_lds_nt(r, lds + m * 64 * Tile::CH, off);
+    else
+      dma16_to_lds(r, lds + m * 64 * Tile::CH, off);
+  }
+}
+
+// k-major operand: lane l receives tile[rbase + (l/32)*khs + e][col0 + l%32], e = 0..7 (through
+// perm_row when PERM).  Transpose reads for 16-bit; fp32 reads the eight elements one by one.
+template <typename T, bool PERM>
+__device__ __forceinline__ typename Mfma<T>::vec8 ld_kmajor_any(const T* tile, int ld, int rbase, int khs, int col0,
+                                                                int lane) {
+  if constexpr (sizeof(T) == 2) {
+    return ld_kmajor<T, PERM>(tile, ld, rbase, khs, col0, lane);
+  } else {
+    const T* p = tile + col0 + (lane & 31);
+    const int r0 = rbase + (lane >> 5) * khs;
+    typename Mfma<T>::vec8 v;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = p[(PERM ? perm_row(r0 + e) : r0 + e) * ld];
+    return v;
+  }
+}
+
+// The KS fragments (16 bytes each, 32 bytes apart) of one K row of a 16-bit tile, read by
+// inline assembly, four per statement, each statement waiting for its own reads before its
+// results are used.  Compiled LDS reads of the tile would make the compiler wait, before
+// them, for every buffer-to-LDS DMA in flight, the V tile's included; the explicit vmcnt
+// waits of the caller already order these reads after the K tile's DMA.
+template <typename T, int KS>
+__device__ __forceinline__ void ld_k_fragments(typename Mfma<T>::vec8 (&f)[KS], const T* row) {
+  static_assert(sizeof(T) == 2 && KS % 2 == 0, "16-bit tiles, an even number of fragments");
+  const unsigned a = (unsigned)(size_t)(const __attribute__((address_space(3))) T*)row;  // LDS byte address
+  u32x4 u[KS];
+#pragma unroll
+  for (int g = 0; g + 4 <= KS; g += 4)
+    asm volatile(
+        "ds_read_b128 %0, %4 offset:%5\n\t"
+        "ds_read_b128 %1, %4 offset:%6\n\t"
+        "ds_read_b128 %2, %4 offset:%7\n\t"
+        "ds_read_b128 %3, %4 offset:%8\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(u[g]), "=&v"(u[g + 1]), "=&v"(u[g + 2]), "=&v"(u[g + 3])
+        : "v"(a), "i"(32 * g), "i"(32 * (g + 1)), "i"(32 * (g + 2)), "i"(32 * (g + 3))
+        : "memory");
+  if constexpr (KS % 4 == 2)
+    asm volatile(
+        "ds_read_b128 %0, %2 offset:%3\n\t"
+        "ds_read_b128 %1, %2 offset:%4\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(u[KS - 2]), "=&v"(u[KS - 1])
+        : "v"(a), "i"(32 * (KS - 2)), "i"(32 * (KS - 1))
+        : "memory");
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) f[ks] = __builtin_bit_cast(typename Mfma<T>::vec8, u[ks]);
+}
+
+// Waits until at most N vector-memory operations of the wavefront are outstanding.  The memory
+// clobber keeps LDS reads of what untracked DMA wrote behind it.
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  static_assert(N < 64, "vmcnt has 6 bits");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
+}
+
+// Waits until the wavefront's LDS reads have returned (before DMA may write over what they read).
+__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+// s_waitcnt immediates (gfx9 encoding: vmcnt in bits 3:0 and 15:14, expcnt 6:4, lgkmcnt
+// 11:8): at most n vector-memory operations outstanding, or no LDS operation outstanding.
+constexpr int vmcnt_imm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
+constexpr int kLgkmcnt0 = 15 | (3 << 14) | (7 << 4);
+
+}  // namespace coalibi

@@ -34,7 +34,6 @@ namespace coalibi {
 namespace {
 
 constexpr int kDecWaves = 4;
-constexpr int kDecWaveKeys = 32;  // keys per wavefront: one 32-key MFMA tile
 constexpr int kDecMergeThreads = 256;
 
 __device__ __forceinline__ int decode_chunks_of(int len) { return (len + kDecodeChunkKeys - 1) / kDecodeChunkKeys; }
@@ -120,8 +119,8 @@ struct DecCfg {
   // a stride of 16 (mod 32) dwords; fp32 reads V element by element.
   static constexpr int LDK = D + CH;
   static constexpr int LDV = kTr ? D + 2 * ((48 - (D / 2) % 32) % 32) : D + CH;
-  using KTile = DmaTile<T, D, kDecWaveKeys, LDK, 1, true>;
-  using VTile = DmaTile<T, D, kDecWaveKeys, LDV, 1, false>;
+  using KTile = DmaTile<T, D, kWaveKeys, LDK, 1, true>;
+  using VTile = DmaTile<T, D, kWaveKeys, LDV, 1, false>;
   static constexpr int K_ELEMS = KTile::LDS_ELEMS;  // a wavefront's K tile
   static constexpr int V_ELEMS = VTile::LDS_ELEMS;  // a wavefront's V tile
   static constexpr int KS = D / 16;  // k16 steps over the head dim
@@ -131,81 +130,6 @@ struct DecCfg {
                     kMaxDecodeGroup / 2 * D * 4 <= V_ELEMS * (int)sizeof(T),
                 "O partials alias the tiles");
 };
-
-// Buffer-to-LDS DMA of the kDecWaveKeys rows row0.. of a row-major [nrows][D] matrix into
-// one wavefront's tile (the layout of DmaTile<T, D, kDecWaveKeys, LD, 1, PERM>): every
-// instruction reads 64 consecutive 16-byte chunks, non-temporal (the cache is read once per
-// step).  Rows past nrows, pad chunks and the tail after the last row land as zeros.  The source offsets are recomputed from an opaque
-// copy of the lane index at every issue; hoisted out of the chunk loop they would hold a
-// register per instruction for the whole kernel.
-template <typename T, int D, int LD, bool PERM>
-__device__ __forceinline__ void dma_wave_rows(const T* base, int row0, int nrows, T* lds, int lane) {
-  using Tile = DmaTile<T, D, kDecWaveKeys, LD, 1, PERM>;
-  const __amdgpu_buffer_rsrc_t r = tile_rsrc(base + (size_t)row0 * D, min(max(nrows - row0, 0), kDecWaveKeys) * D);
-  int ln;
-  asm volatile("v_mov_b32 %0, %1" : "=v"(ln) : "v"(lane));
-#pragma unroll
-  for (int m = 0; m < Tile::NINSTR; ++m) {
-    const int ch = m * 64 + ln, row = ch / Tile::CPR, j = ch - row * Tile::CPR;
-    const int src = PERM ? (row & ~31) + kRowOfReg(row & 31) : row;
-    const bool in_tile = row < kDecWaveKeys && j < D / Tile::CH;
-    dma16_to_lds_nt(r, lds + m * 64 * Tile::CH, in_tile ? (src * D + j * Tile::CH) * (int)sizeof(T) : 0x40000000);
-  }
-}
-
-// k-major operand: lane l receives tile[rbase + (l/32)*khs + e][col0 + l%32], e = 0..7.
-// Transpose reads for 16-bit; fp32 reads the eight elements one by one.
-template <typename T>
-__device__ __forceinline__ typename Mfma<T>::vec8 ld_kmajor_dec(const T* tile, int ld, int rbase, int khs,
-                                                                  int col0, int lane) {
-  if constexpr (sizeof(T) == 2) {
-    return ld_kmajor<T, false>(tile, ld, rbase, khs, col0, lane);
-  } else {
-    const T* p = tile + (rbase + (lane >> 5) * khs) * ld + col0 + (lane & 31);
-    typename Mfma<T>::vec8 v;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = p[e * ld];
-    return v;
-  }
-}
-
-// The KS fragments (16 bytes each, 32 bytes apart) of one K row of a 16-bit tile, read by
-// inline assembly, four per statement, each statement waiting for its own reads before its
-// results are used.  Compiled LDS reads of the tile would make the compiler wait, before
-// them, for every buffer-to-LDS DMA in flight, the V tile's included; the explicit vmcnt
-// waits of the chunk loop already order these reads after the K tile's DMA.
-template <typename T, int KS>
-__device__ __forceinline__ void ld_k_fragments(typename Mfma<T>::vec8 (&f)[KS], const T* row) {
-  static_assert(sizeof(T) == 2 && KS % 2 == 0, "16-bit tiles, an even number of fragments");
-  const unsigned a = (unsigned)(size_t)(const __attribute__((address_space(3))) T*)row;  // LDS byte address
-  u32x4 u[KS];
-#pragma unroll
-  for (int g = 0; g + 4 <= KS; g += 4)
-    asm volatile(
-        "ds_read_b128 %0, %4 offset:%5\n\t"
-        "ds_read_b128 %1, %4 offset:%6\n\t"
-        "ds_read_b128 %2, %4 offset:%7\n\t"
-        "ds_read_b128 %3, %4 offset:%8\n\t"
-        "s_waitcnt lgkmcnt(0)"
-        : "=&v"(u[g]), "=&v"(u[g + 1]), "=&v"(u[g + 2]), "=&v"(u[g + 3])
-        : "v"(a), "i"(32 * g), "i"(32 * (g + 1)), "i"(32 * (g + 2)), "i"(32 * (g + 3))
-        : "memory");
-  if constexpr (KS % 4 == 2)
-    asm volatile(
-        "ds_read_b128 %0, %2 offset:%3\n\t"
-        "ds_read_b128 %1, %2 offset:%4\n\t"
-        "s_waitcnt lgkmcnt(0)"
-        : "=&v"(u[KS - 2]), "=&v"(u[KS - 1])
-        : "v"(a), "i"(32 * (KS - 2)), "i"(32 * (KS - 1))
-        : "memory");
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) f[ks] = __builtin_bit_cast(typename Mfma<T>::vec8, u[ks]);
-}
-
-// s_waitcnt immediates (gfx9 encoding: vmcnt in bits 3:0 and 15:14, expcnt 6:4, lgkmcnt
-// 11:8): at most n vector-memory operations outstanding, or no LDS operation outstanding.
-constexpr int vmcnt_imm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
-constexpr int kLgkmcnt0 = 15 | (3 << 14) | (7 << 4);
 
 // How a launch splits its sequences: evenly, by a plan over a length per sequence (RAGGED), or not
 // at all (DIRECT, nSplits == 1): the work-group then writes o and lse itself and no merge is
@@ -268,10 +192,10 @@ __global__ __launch_bounds__(kDecWaves * 64, (D > 128 || sizeof(T) == 4) ? 1 : 2
   // the rate).  K rows are permuted (LDS row R holds key kRowOfReg(R)) so that register r of
   // lane l of S^T holds key 16*(l/32) + r of the wavefront.
   auto issue_k = [&](int c) {
-    dma_wave_rows<T, D, C::LDK, true>(kbase, c * kDecodeChunkKeys + wave * kDecWaveKeys, L, sKw, lane);
+    dma_wave_rows<T, D, C::LDK, true, true>(kbase, c * kDecodeChunkKeys + wave * kWaveKeys, L, sKw, lane);
   };
   auto issue_v = [&](int c) {
-    dma_wave_rows<T, D, C::LDV, false>(vbase, c * kDecodeChunkKeys + wave * kDecWaveKeys, L, sVw, lane);
+    dma_wave_rows<T, D, C::LDV, false, true>(vbase, c * kDecodeChunkKeys + wave * kWaveKeys, L, sVw, lane);
   };
   issue_k(c_last);
   issue_v(c_last);
@@ -297,7 +221,7 @@ __global__ __launch_bounds__(kDecWaves * 64, (D > 128 || sizeof(T) == 4) ? 1 : 2
 
   int par = 0;
   for (int c = c_last; c >= c_first; --c) {
-    const int row0 = c * kDecodeChunkKeys + wave * kDecWaveKeys;
+    const int row0 = c * kDecodeChunkKeys + wave * kWaveKeys;
     const bool more = c > c_first;
 
     // This chunk's K has landed once at most its V (issued after it) is outstanding.
@@ -399,7 +323,7 @@ __global__ __launch_bounds__(kDecWaves * 64, (D > 128 || sizeof(T) == 4) ? 1 : 2
     for (int j = 0; j < C::DT; ++j)
 #pragma unroll
       for (int s = 0; s < 2; ++s)
-        oacc[j] = M::k16(pa[s], ld_kmajor_dec<T>(sVw, C::LDV, 8 * s, 16, 32 * j, lane), oacc[j]);
+        oacc[j] = M::k16(pa[s], ld_kmajor_any<T, false>(sVw, C::LDV, 8 * s, 16, 32 * j, lane), oacc[j]);
     if (more) {
       __builtin_amdgcn_s_waitcnt(kLgkmcnt0);  // the V tile has been read
       issue_v(c - 1);

@@ -24,6 +24,8 @@
 // processed: backward pass 1 rebuilds z from it.  R is summed in fp64 over 32-key block
 // totals, exactly the totals pass 1 computes (the same sigmoids summed in the same order), so
 // the difference pass 1 takes is exact up to one rounding.
+#include <algorithm>
+
 #include "coalibi_common.h"
 #include "coalibi_kernels.h"
 
@@ -404,26 +406,22 @@ __global__ __launch_bounds__(256) void coalibi_key_norm_kernel(const T* __restri
   }
 }
 
+// One 128-row block (bh, qb) by a work-group of 4 wavefronts, 32 rows each, over tiles in sK and sV.
 // SKIP: the tail skip (args.knorm holds the key norms); without it every key is processed and
-// the kernel carries none of the skip's per-tile test.
+// the code carries none of the skip's per-tile test.
 template <typename T, int D, bool CAUSAL, bool SKIP>
-__global__ __launch_bounds__(256, (sizeof(T) == 4 || D > 128) ? 1 : 2) void coalibi_fwd_kernel(FwdArgs args) {
+__device__ __forceinline__ void fwd_row_block(const FwdArgs& args, int bh, int qb, T* __restrict__ sK,
+                                              T* __restrict__ sV) {
   using C = FwdCfg<T, D>;
   using M = Mfma<T>;
   using vec8 = typename M::vec8;
   using KTile = TileLoader<T, D, kFwdBN>;
   using VTile = TileLoader<T, D, kFwdBN, !FwdCfg<T, D>::kTr>;
-  __shared__ __align__(16) T sK[kFwdBN * C::LDK];
-  __shared__ __align__(16) T sV[C::V_ELEMS];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int col = lane & 31, hh = lane >> 5;
   const int Sq = args.Sq, Skv = args.Skv;
   const int nQB = (Sq + kFwdBM - 1) / kFwdBM;
-  const WorkItem item = args.row_order ? table_item(args.row_order, blockIdx.x, args.B * args.Hq, gridDim.x)
-                                       : lpt_item(blockIdx.x, args.B * args.Hq, 1);
-  const int bh = item.head;
-  const int qb = nQB - 1 - item.rank;  // rank 0: the longest causal rows
   const int b = bh / args.Hq, hq = bh - b * args.Hq;
   const int hkv = hq / (args.Hq / args.Hkv);
   const T* __restrict__ Qp = static_cast<const T*>(args.q) + (size_t)bh * Sq * D;
@@ -433,7 +431,7 @@ __global__ __launch_bounds__(256, (sizeof(T) == 4 || D > 128) ? 1 : 2) void coal
   const float lam2 = args.slopes[hq] * kLog2e;
   const float sc2 = args.sc2;
   if constexpr (D < C::DP) {  // the padding columns of V stay zero: tiles only write the D real ones
-    lds_zero(sV, (int)sizeof(sV), tid, 256);
+    lds_zero(sV, C::V_ELEMS * (int)sizeof(T), tid, 256);
   }
 
   const int q0 = qb * kFwdBM;
@@ -595,6 +593,301 @@ __global__ __launch_bounds__(256, (sizeof(T) == 4 || D > 128) ? 1 : 2) void coal
   }
 }
 
+template <typename T, int D, bool CAUSAL, bool SKIP>
+__global__ __launch_bounds__(256, (sizeof(T) == 4 || D > 128) ? 1 : 2) void coalibi_fwd_kernel(FwdArgs args) {
+  using C = FwdCfg<T, D>;
+  __shared__ __align__(16) T sK[kFwdBN * C::LDK];
+  __shared__ __align__(16) T sV[C::V_ELEMS];
+  const int nQB = (args.Sq + kFwdBM - 1) / kFwdBM;
+  const WorkItem item = args.row_order ? table_item(args.row_order, blockIdx.x, args.B * args.Hq, gridDim.x)
+                                       : lpt_item(blockIdx.x, args.B * args.Hq, 1);
+  // rank 0: the longest causal rows
+  fwd_row_block<T, D, CAUSAL, SKIP>(args, item.head, nQB - 1 - item.rank, sK, sV);
+}
+
+// ---------------------------------------------------------------------------
+// Small grids.  With fewer row blocks than the GPU has room for, a 128-row block's walk over its
+// keys is the time: one wavefront per SIMD takes about 2.4 us per 64-key tile, whatever the rest
+// of the GPU does.  Here a row block is four work-groups of 32 rows, and a work-group's four
+// wavefronts take the four 32-key tiles of every 128-key step, each from LDS tiles of its own
+// filled by its own DMA (the decode's scheme).  The walk is a quarter as long, over four times the
+// work-groups.  What it costs: K and V are read from L2 four times as often, so it loses where
+// the GPU is full.
+//   Per step each wavefront computes its tile's S^T and sigmoids; the tiles' sigmoid totals go
+// through LDS (one barrier), so that z is absolute in every wavefront; the softmax state is a
+// wavefront's own and the four are combined at the end.
+constexpr int kSplitRows = 32;   // rows per work-group
+constexpr int kSplitWaves = 4;   // key tiles per step
+
+template <typename T, int D>
+struct SplitCfg {
+  static constexpr bool kTr = sizeof(T) == 2;
+  static constexpr int CH = 16 / (int)sizeof(T);
+  static constexpr int DP = D < 32 ? 32 : D;
+  static constexpr int LDK = DP + CH;
+  static constexpr int LDV = kTr ? DP + 2 * CH : DP + CH;
+  using KTile = DmaTile<T, D, kWaveKeys, LDK, 1, true>;
+  using VTile = DmaTile<T, D, kWaveKeys, LDV, 1, false>;
+  static constexpr int K_ELEMS = KTile::LDS_ELEMS;  // a wavefront's K tile
+  static constexpr int V_ELEMS = VTile::LDS_ELEMS;
+  static constexpr int KS = D / 16;
+  static constexpr int DT = DP / 32;
+  // At the end the O partials of rows 0..15 alias a wavefront's K tile, of rows 16..31 its V tile.
+  static constexpr int LDO = DP + 4;  // floats
+  static_assert(16 * LDO * 4 <= K_ELEMS * (int)sizeof(T) && 16 * LDO * 4 <= V_ELEMS * (int)sizeof(T),
+                "O partials alias the tiles");
+  // The whole-block form runs in the same LDS.
+  static_assert(kSplitWaves * K_ELEMS >= kFwdBN * FwdCfg<T, D>::LDK && kSplitWaves * V_ELEMS >= FwdCfg<T, D>::V_ELEMS,
+                "the 64-key tiles fit");
+  static constexpr size_t kLds = (size_t)kSplitWaves * (K_ELEMS + V_ELEMS) * sizeof(T);
+  // fp32 at D = 256 takes 266 KB, above a CU's 160.
+  static constexpr bool kFits = kLds <= 155 * 1024;
+};
+
+// Whether a row block of a head that has `keys` visible keys is split.  A head that the tail skip
+// stops after about window / slope keys walks at most that many in the whole-block form, which then
+// is the shorter one; the tail skip's record is per 128-row block, so the split form has none and
+// records that it processed every key.  With the skip switched off (window infinite) every
+// block is split.
+__device__ __forceinline__ bool split_row_block(int keys, float slope, float window) {
+  return !(slope > 0.f) || (float)keys <= 3.0f * (window / slope) + 192.0f;
+}
+
+template <typename T, int D, bool CAUSAL>
+__device__ __forceinline__ void fwd_split_rows(const FwdArgs& args, int bh, int q0, T* __restrict__ sK,
+                                               T* __restrict__ sV) {
+  using C = SplitCfg<T, D>;
+  using M = Mfma<T>;
+  using vec8 = typename M::vec8;
+  __shared__ float sSig[2][kSplitWaves][kSplitRows];  // the tiles' sigmoid totals, by step parity
+  __shared__ float sMax[kSplitWaves][kSplitRows];
+  __shared__ float sSum[kSplitWaves][kSplitRows];
+  __shared__ float sInv[kSplitRows];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31, hh = lane >> 5;
+  const int Sq = args.Sq, Skv = args.Skv;
+  const int b = bh / args.Hq, hq = bh - b * args.Hq;
+  const int hkv = hq / (args.Hq / args.Hkv);
+  const size_t kvoff = ((size_t)b * args.Hkv + hkv) * (size_t)Skv * D;
+  const T* __restrict__ Kp = static_cast<const T*>(args.k) + kvoff;
+  const T* __restrict__ Vp = static_cast<const T*>(args.v) + kvoff;
+  T* const sKw = sK + wave * C::K_ELEMS;  // this wavefront's tiles
+  T* const sVw = sV + wave * C::V_ELEMS;
+  const float lam2 = args.slopes[hq] * kLog2e;
+  const int row = q0 + col;
+
+  // Tiles n32 - 1 .. 0, four per step from the right; tile t < 0 holds no key (zero rows).
+  const int n32 = (CAUSAL ? min(q0 + kSplitRows - 1, Skv - 1) : Skv - 1) / kWaveKeys + 1;
+  const int steps = (n32 + kSplitWaves - 1) / kSplitWaves;
+  int t = n32 - kSplitWaves + wave;
+  // Untracked DMA: the tiles are this wavefront's own, and the waits below order it.
+  typename C::KTile kdma;
+  typename C::VTile vdma;
+  kdma.init(0, lane);
+  vdma.init(0, lane);
+  const unsigned lds_k = lds_address(sKw), lds_v = lds_address(sVw);
+  auto issue_k = [&](int tt) { kdma.issue_untracked(Kp, max(tt, 0) * kWaveKeys, tt < 0 ? 0 : Skv, lds_k, 0); };
+  auto issue_v = [&](int tt) { vdma.issue_untracked(Vp, max(tt, 0) * kWaveKeys, tt < 0 ? 0 : Skv, lds_v, 0); };
+  vec8 qf[C::KS];
+  {
+    const __amdgpu_buffer_rsrc_t qrs =
+        tile_rsrc(static_cast<const T*>(args.q) + ((size_t)bh * Sq + q0) * D, min(Sq - q0, kSplitRows) * D);
+#pragma unroll
+    for (int ks = 0; ks < C::KS; ++ks)
+      qf[ks] = buffer_load_vec8<vec8>(qrs, (col * D + ks * 16 + hh * 8) * (int)sizeof(T));
+  }
+  issue_k(t);
+  issue_v(t);
+  constexpr bool kPreScaled = sizeof(T) == 2;  // as in fwd_row_block
+  if constexpr (kPreScaled) {
+#pragma unroll
+    for (int ks = 0; ks < C::KS; ++ks) qf[ks] = scale_vec8<T>(qf[ks], args.sc2);
+  }
+  const float sc2 = kPreScaled ? 1.0f : args.sc2;
+
+  f32x16 acc[C::DT];
+#pragma unroll
+  for (int dt = 0; dt < C::DT; ++dt) acc[dt] = f32x16{};
+  float m2 = kNegInf, lsum = 0.f;
+  double zsum = 0.0;  // the sigmoids of the keys right of the step, as fwd_row_block sums them
+
+  for (int s = 0; s < steps; ++s, t -= kSplitWaves) {
+    const bool more = s + 1 < steps;
+    const int key0 = t * kWaveKeys + hh * 16;  // key of register 0
+    // This step's K has landed once at most its V (issued after it) is outstanding.
+    wait_vm<C::VTile::NINSTR>();
+    f32x16 sacc = f32x16{};
+#pragma unroll
+    for (int ks = 0; ks < C::KS; ++ks)
+      sacc = M::k16(ld_vec8(sKw + col * C::LDK + ks * 16 + hh * 8), qf[ks], sacc);
+    if (more) {  // the K tile has been read: the next one lands in it during this step's math
+      wait_lds();
+      issue_k(t - kSplitWaves);
+    }
+    // Register r is a visible key iff r < nvis.
+    const bool masked = t < 0 || (CAUSAL && t * kWaveKeys + kWaveKeys - 1 > q0) || (t + 1) * kWaveKeys > Skv;
+    const int nvis = t < 0 ? 0 : min(Skv, CAUSAL ? row + 1 : Skv) - key0;
+    float loc[16], tot = 0.f;
+    if (masked) {
+#pragma unroll
+      for (int r = 15; r >= 0; --r) loc[r] = tot += r < nvis ? sigmoid_log2(sacc[r] * sc2) : 0.f;
+    } else {
+#pragma unroll
+      for (int r = 15; r >= 0; --r) loc[r] = tot += sigmoid_log2(sacc[r] * sc2);
+    }
+    const float oth = other_half(tot);
+    const float upper = hh ? tot : oth, lower = hh ? oth : tot;  // keys 16..31 and 0..15 of the tile
+    if (hh == 0) sSig[s & 1][wave][col] = upper + lower;
+    lds_barrier();  // the DMA stays in flight
+    float zr = 0.f;
+#pragma unroll
+    for (int w = kSplitWaves - 1; w >= 0; --w) {  // right to left
+      if (w == wave) zr = (float)zsum;
+      zsum += (double)sSig[s & 1][w][col];
+    }
+
+    // As fwd_tile, for one 32-key subtile.
+    const float mb = m2 == kNegInf ? 0.f : m2;
+    const float cst = mb + lam2 * (hh ? zr : zr + upper);
+    float mt = kNegInf;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      sacc[r] = fmaf(-lam2, loc[r], fmaf(sacc[r], sc2, -cst));
+      if (masked) sacc[r] = r < nvis ? sacc[r] : kNegInf;
+      mt = fmaxf(mt, sacc[r]);
+    }
+    mt = fmaxf(mt, other_half(mt));
+    const bool need = m2 == kNegInf ? mt > kNegInf : mt > kRescaleThreshold;
+    if (__any(need)) {
+      const float delta = need ? mt : 0.f;
+      const float alpha = need ? (m2 == kNegInf ? 0.f : fast_exp2(-delta)) : 1.f;
+      m2 = need ? mb + delta : m2;
+      lsum *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < C::DT; ++dt) acc[dt] *= alpha;
+      sacc -= delta;
+    }
+    vec8 pb[2];
+#pragma unroll
+    for (int mh = 0; mh < 2; ++mh) {
+      f32x8 pv;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) pv[e] = fast_exp2(sacc[mh * 8 + e]);
+      pb[mh] = M::pack(pv);
+      lsum = sum8(pb[mh], lsum);
+    }
+    // This step's V has landed once at most the next step's K is outstanding.
+    if (more)
+      wait_vm<C::KTile::NINSTR>();
+    else
+      wait_vm<0>();
+#pragma unroll
+    for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+      for (int mh = 0; mh < 2; ++mh)
+        acc[dt] = M::k16(ld_kmajor_any<T, false>(sVw, C::LDV, mh * 8, 16, dt * 32, lane), pb[mh], acc[dt]);
+    if (more) {
+      wait_lds();  // the V tile has been read
+      issue_v(t - kSplitWaves);
+    }
+  }
+
+  // Combine the four wavefronts' softmax states.
+  const float lown = lsum + other_half(lsum);
+  if (hh == 0) {
+    sMax[wave][col] = m2;
+    sSum[wave][col] = lown;
+  }
+  __syncthreads();
+  float m = kNegInf, l = 0.f;
+#pragma unroll
+  for (int w = 0; w < kSplitWaves; ++w) m = fmaxf(m, sMax[w][col]);
+#pragma unroll
+  for (int w = 0; w < kSplitWaves; ++w) {
+    const float mw = sMax[w][col];
+    l += mw == kNegInf ? 0.f : sSum[w][col] * fast_exp2(mw - m);
+  }
+  const float own = m2 == kNegInf ? 0.f : fast_exp2(m2 - m);
+  auto o_row = [&](int w, int r) {
+    return reinterpret_cast<float*>(r < 16 ? sK + w * C::K_ELEMS : sV + w * C::V_ELEMS) + (r & 15) * C::LDO;
+  };
+  float* const orow = o_row(wave, col);
+#pragma unroll
+  for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<f32x4*>(orow + dt * 32 + g * 8 + hh * 4) =
+          f32x4{acc[dt][g * 4] * own, acc[dt][g * 4 + 1] * own, acc[dt][g * 4 + 2] * own, acc[dt][g * 4 + 3] * own};
+  if (wave == 0 && hh == 0) {
+    sInv[col] = l > 0.f ? 1.0f / l : 0.f;
+    if (row < Sq) {
+      const size_t at = (size_t)bh * Sq + row;
+      if (args.lse != nullptr) args.lse[at] = l > 0.f ? (m + log2f(l)) * kLn2 : kNegInf;
+      if (args.rsum != nullptr) {
+        const float hi = (float)zsum;
+        args.rsum[at] = hi;
+        args.rsum[(size_t)args.B * args.Hq * Sq + at] = (float)(zsum - (double)hi);
+      }
+    }
+  }
+  __syncthreads();
+  const int r = tid >> 3;
+  if (q0 + r < Sq) {
+    using vec4 = typename VecOf<T, 4>::type;
+    T* __restrict__ Orow = static_cast<T*>(args.o) + ((size_t)bh * Sq + q0 + r) * D;
+    const float inv = sInv[r];
+#pragma unroll
+    for (int c = (tid & 7) * 4; c < D; c += 32) {
+      f32x4 v = *reinterpret_cast<const f32x4*>(o_row(0, r) + c);
+#pragma unroll
+      for (int w = 1; w < kSplitWaves; ++w) v += *reinterpret_cast<const f32x4*>(o_row(w, r) + c);
+      *reinterpret_cast<vec4*>(Orow + c) = __builtin_convertvector(v * inv, vec4);
+    }
+  }
+}
+
+// Work-groups 8j .. 8j + 7 of every 32 run on the 8 XCDs: item (id / 32) * 8 + id % 8, so that the
+// four parts of a row block share their K and V in one XCD's L2.
+template <typename T, int D, bool CAUSAL, bool SKIP>
+__global__ __launch_bounds__(256, D * sizeof(T) > 256 ? 1 : 2) void coalibi_fwd_split_kernel(FwdArgs args,
+                                                                                               int items, float window) {
+  using C = SplitCfg<T, D>;
+  __shared__ __align__(16) T sK[kSplitWaves * C::K_ELEMS];
+  __shared__ __align__(16) T sV[kSplitWaves * C::V_ELEMS];
+  const int i = (blockIdx.x >> 5) * 8 + (blockIdx.x & 7), part = (blockIdx.x >> 3) & 3;
+  if (i >= items) return;
+  const WorkItem item = args.row_order ? table_item(args.row_order, i, args.B * args.Hq, items)
+                                       : lpt_item(i, args.B * args.Hq, 1);
+  const int nQB = (args.Sq + kFwdBM - 1) / kFwdBM, qb = nQB - 1 - item.rank;
+  const int q0 = qb * kFwdBM;
+  const float slope = args.slopes[item.head % args.Hq];
+  if (split_row_block(CAUSAL ? min(q0 + kFwdBM, args.Skv) : args.Skv, slope, window)) {
+    if (blockIdx.x == 0 && args.flags != nullptr && threadIdx.x < kStatsHeader)
+      args.flags[threadIdx.x] = threadIdx.x == 0 ? args.order_flags : 0;
+    if (part == 0 && args.kstart != nullptr && threadIdx.x == 0) args.kstart[(size_t)item.head * nQB + qb] = 0;
+    if (q0 + part * kSplitRows < args.Sq) fwd_split_rows<T, D, CAUSAL>(args, item.head, q0 + part * kSplitRows, sK, sV);
+  } else if (part == 0) {
+    fwd_row_block<T, D, CAUSAL, SKIP>(args, item.head, qb, sK, sV);
+  }
+}
+
+// Whether the split form is launched.  It wins where the row blocks leave the GPU room, and longer
+// walks leave more of it (causal: half the work of the longest block on average, and the short
+// blocks' work-groups cost their prologue and merge all the same).  us, whole-block form ->
+// split, fp16 (f = tail skip off):
+//   D 128  n 256: 64 blocks 19.4 -> 13.1 f 13.1 -> 9.2, 128: 19.7 -> 16.5 f 13.3 -> 11.0
+//          n 512: 64 blocks 27.1 -> 20.1 f 20.2 -> 12.2, 128: 27.2 -> 24.4 f 20.3 -> 13.9, 192: 28.2 -> 33.1 f 20.8 -> 22.1
+//          n 1024: 128 blocks 42.6 -> 28.0 f 34.1 -> 21.1, 256: 44.5 -> 44.1 f 35.0 -> 32.8, 320: 46.7 -> 53.2 f 37.5 -> 41.1
+//          n 2048: 128 blocks 73.8 -> 37.6 f 61.5 -> 34.7, 256: 74.9 -> 53.2 f 62.9 -> 52.0, 320: 77.3 -> 61.6 f 66.8 -> 61.9
+//   D 64   n 512: 128 blocks 21.6 -> 19.9 f 14.9 -> 10.4, 192: 22.2 -> 23.1 f 15.2 -> 13.0
+//          n 1024: 256 blocks 34.1 -> 32.7 f 25.3 -> 22.0;  n 2048: 320 blocks 59.5 -> 42.9 f 45.9 -> 40.1
+//   non-causal, D 128: 333 x 2047, 96 blocks 91.0 -> 40.9; 2000 x 3000, 256 blocks 126.2 -> 81.2;
+//          D 64, 1400 x 1400, 352 blocks 43.8 -> 51.8
+//   fp32   D 64: n 1000, 192 blocks 94.7 -> 76.5;  D 128: n 1024, 128 blocks 159.4 -> 105.8
+inline bool split_grid(long long row_blocks, int keys, bool causal) {
+  return row_blocks <= std::max(128, causal ? std::min(keys / 4, 384) : std::min(keys / 8, 256));
+}
+
 }  // namespace
 
 template <typename T, int D, bool CAUSAL>
@@ -623,6 +916,19 @@ hipError_t launch_fwd(const FwdArgs& a, hipStream_t stream) {
   if (a.knorm == nullptr || !rows_sorted) f.row_order = nullptr;  // no sorted table: the fixed order
   const int nQB = (a.Sq + kFwdBM - 1) / kFwdBM;
   const int grid = nQB * a.B * a.Hq;
+  if constexpr (SplitCfg<T, D>::kFits) {
+    if (split_grid(grid, a.Skv, CAUSAL)) {
+      const dim3 parts((grid + 7) / 8 * 32);
+      const float window = a.every_key ? __builtin_inff() : order_window<T>();
+      if (a.knorm != nullptr)
+        hipLaunchKernelGGL((coalibi_fwd_split_kernel<T, D, CAUSAL, true>), parts, dim3(256), 0, stream, f, grid,
+                           window);
+      else
+        hipLaunchKernelGGL((coalibi_fwd_split_kernel<T, D, CAUSAL, false>), parts, dim3(256), 0, stream, f, grid,
+                           window);
+      return hipGetLastError();
+    }
+  }
   if (a.knorm != nullptr)
     hipLaunchKernelGGL((coalibi_fwd_kernel<T, D, CAUSAL, true>), dim3(grid), dim3(256), 0, stream, f);
   else

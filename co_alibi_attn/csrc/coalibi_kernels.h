@@ -113,6 +113,7 @@ struct FwdArgs {
   float* rsum;         // (2, B*Hq, Sq) row sigmoid totals (hi, lo), written when not NULL
   int B, Hq, Hkv, Sq, Skv, nKC;
   float sc2;  // sm_scale * log2(e)
+  bool every_key;  // the tail skip is switched off
   // Work orders (above): written by the key-norm launch when not NULL (key_order only with
   // row_order); the forward follows row_order when it is sorted (row_order_fits).
   int* row_order;
