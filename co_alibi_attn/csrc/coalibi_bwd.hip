@@ -36,6 +36,7 @@
 // Operands whose reduction runs over LDS rows (K^T in pass 1; Q^T, dO^T, s, dP
 // in pass 2) are read with ds_read_b64_tr_b16 from row-major tiles; the fp32
 // validation mode stores transposed copies instead.
+#include <algorithm>
 #include <type_traits>
 
 #include "coalibi_common.h"
@@ -74,22 +75,15 @@ __device__ __forceinline__ bool pair_ok(int key, int row, int Skv, int Sq, bool 
 }
 
 // Elementwise core shared by both passes for one 32-key x 32-query tile held as
-// S^T (lane (col, hh): query q, keys hh*16 + r).  Inputs: sacc = q.k (times sc2 gives
-// log2 units; sc2 = 1 when an operand carries the scale), dacc = dO.v - D (the dS
-// accumulator starts at -D = -dO.O), zb = sum of sigma over keys >= the block start,
-// cb = sum of dA over keys before the block, lse2 = LSE*log2(e).  Outputs the 16
-// values of s and dP packed for the next products; returns the block's dA and sigma totals
-// in `atot_blk` and `ztot_blk` (the same value in both halves of the wavefront).  C is carried multiplied by the slope (lam*C), which makes
-// dP = dA - lam*sigma'*C one fma per key after sigma' = sigma - sigma^2.
-template <typename T, bool MASKED, bool CAUSAL>
-__device__ __forceinline__ void dp_tile(const f32x16& sacc, f32x16& dacc, float zb, float cb, float lse2,
-                                        int key0, int row, int hh, int Skv, int Sq, float sc2, float lam,
-                                        float lam2, typename Mfma<T>::vec8 (&sb)[2],
-                                        typename Mfma<T>::vec8 (&pb)[2], float& atot_blk, float& ztot_blk) {
-  using M = Mfma<T>;
-  // Phase 1: sigma, its inclusive suffix over this run folded into ex = t - lam2*suffix, and
-  // the run's sigma total, summed from the run's last key down as the forward sums it.
-  float sg[16], ex[16];
+// S^T (lane (col, hh): query q, keys hh*16 + r), in three steps so that a caller can exchange the
+// tile's totals between them.
+//
+// dp_sigma: sigma, its inclusive suffix over this run folded into ex = t - lam2*suffix, and
+// the run's sigma total (returned), summed from the run's last key down as the forward sums it.
+// sacc = q.k (times sc2 gives log2 units; sc2 = 1 when an operand carries the scale).
+template <bool MASKED, bool CAUSAL>
+__device__ __forceinline__ float dp_sigma(const f32x16& sacc, int key0, int row, int Skv, int Sq, float sc2,
+                                          float lam2, float (&sg)[16], float (&ex)[16]) {
   float suf = 0.f;
 #pragma unroll
   for (int r = 15; r >= 0; --r) {
@@ -100,14 +94,23 @@ __device__ __forceinline__ void dp_tile(const f32x16& sacc, f32x16& dacc, float 
     suf += s;
     ex[r] = fmaf(-lam2, suf, t);
   }
-  // z = zb - (sigma of the other half's run if it is left of ours) - exclusive prefix, and the
-  // exclusive prefix is the run total minus the inclusive suffix, so
-  // log2 of s = t - lam2*z - lse2 = ex - (lam2*(zb - other - total) + lse2).
-  const float tot = suf;
-  const float oth = other_half(tot);
-  ztot_blk = tot + oth;
-  const float zbase = (zb - (hh ? oth : 0.f)) - tot;
-  const float cst = fmaf(lam2, zbase, lse2);
+  return suf;
+}
+
+// The constant of dp_scores' exponent from the run totals of both halves (tot, oth) and zb, the sum
+// of sigma over keys >= the block start:
+// z = zb - (sigma of the other half's run if it is left of ours) - exclusive prefix, and the
+// exclusive prefix is the run total minus the inclusive suffix, so
+// log2 of s = t - lam2*z - lse2 = ex - (lam2*(zb - other - total) + lse2).
+__device__ __forceinline__ float dp_exponent(float zb, float tot, float oth, int hh, float lam2, float lse2) {
+  return fmaf(lam2, (zb - (hh ? oth : 0.f)) - tot, lse2);
+}
+
+// dp_scores: s packed into sb, and dA = s (dS - D) in place of dacc = dO.v - D (the dS accumulator
+// starts at -D = -dO.O); returns the run's dA total.
+template <typename T, bool MASKED, bool CAUSAL>
+__device__ __forceinline__ float dp_scores(const float (&ex)[16], float cst, f32x16& dacc, int key0, int row, int Skv,
+                                           int Sq, typename Mfma<T>::vec8 (&sb)[2]) {
   float atot = 0.f;
   f32x8 sv[2];
 #pragma unroll
@@ -119,12 +122,17 @@ __device__ __forceinline__ void dp_tile(const f32x16& sacc, f32x16& dacc, float 
     atot += da;
     sv[r >> 3][r & 7] = s;
   }
-  sb[0] = M::pack(sv[0]);
-  sb[1] = M::pack(sv[1]);
-  // lam*C = lam*(cb + (dA of the other half's run if left of ours) + inclusive prefix).
-  const float aoth = other_half(atot);
-  float c = lam * (cb + (hh ? aoth : 0.f));
-  atot_blk = hh ? atot + aoth : aoth + atot;  // same order in both halves
+  sb[0] = Mfma<T>::pack(sv[0]);
+  sb[1] = Mfma<T>::pack(sv[1]);
+  return atot;
+}
+
+// dp_grads: dP packed into pb, from c = lam * (the sum of dA over the keys before this run).  C is
+// carried multiplied by the slope (lam*C), which makes dP = dA - lam*sigma'*C one fma per key
+// after sigma' = sigma - sigma^2.
+template <typename T, bool MASKED, bool CAUSAL>
+__device__ __forceinline__ void dp_grads(const f32x16& dacc, const float (&sg)[16], float c, float lam, int key0,
+                                         int row, int Skv, int Sq, typename Mfma<T>::vec8 (&pb)[2]) {
 #pragma unroll
   for (int mh = 0; mh < 2; ++mh) {
     f32x8 pv;
@@ -138,8 +146,27 @@ __device__ __forceinline__ void dp_tile(const f32x16& sacc, f32x16& dacc, float 
       if (MASKED) dp = pair_ok(key0 + r, row, Skv, Sq, CAUSAL) ? dp : 0.f;
       pv[e] = dp;
     }
-    pb[mh] = M::pack(pv);
+    pb[mh] = Mfma<T>::pack(pv);
   }
+}
+
+// The three in a row, with cb = sum of dA over keys before the block.  Returns the block's dA and
+// sigma totals in `atot_blk` and `ztot_blk` (the same value in both halves of the wavefront).
+template <typename T, bool MASKED, bool CAUSAL>
+__device__ __forceinline__ void dp_tile(const f32x16& sacc, f32x16& dacc, float zb, float cb, float lse2,
+                                        int key0, int row, int hh, int Skv, int Sq, float sc2, float lam,
+                                        float lam2, typename Mfma<T>::vec8 (&sb)[2],
+                                        typename Mfma<T>::vec8 (&pb)[2], float& atot_blk, float& ztot_blk) {
+  float sg[16], ex[16];
+  const float tot = dp_sigma<MASKED, CAUSAL>(sacc, key0, row, Skv, Sq, sc2, lam2, sg, ex);
+  const float oth = other_half(tot);
+  ztot_blk = tot + oth;
+  const float atot =
+      dp_scores<T, MASKED, CAUSAL>(ex, dp_exponent(zb, tot, oth, hh, lam2, lse2), dacc, key0, row, Skv, Sq, sb);
+  // lam*C = lam*(cb + (dA of the other half's run if left of ours) + inclusive prefix).
+  const float aoth = other_half(atot);
+  atot_blk = hh ? atot + aoth : aoth + atot;  // same order in both halves
+  dp_grads<T, MASKED, CAUSAL>(dacc, sg, lam * (cb + (hh ? aoth : 0.f)), lam, key0, row, Skv, Sq, pb);
 }
 
 // ---------------------------------------------------------------------------
@@ -378,6 +405,279 @@ __global__ __launch_bounds__(256, (sizeof(T) == 4 || D > 128) ? 1 : 2) void coal
       }
     }
   }
+}
+
+// ---------------------------------------------------------------------------
+// Pass 1 on small grids: as the forward's split form (coalibi_fwd.hip), a row block is four
+// work-groups of 32 rows, whose four wavefronts take the four 32-key tiles of every 128-key step
+// from LDS tiles of their own.  A 128-row block alone walks its tiles at about 1.5 us each, with one
+// wavefront per SIMD, whatever the rest of the GPU does.
+//   z and C run along the keys, so the step has two exchanges through LDS, each a barrier: the tiles'
+// sigmoid totals (z at a tile's start = z at the step's start minus the totals left of it) and
+// their dA totals (C likewise).  Both are taken off / added in tile order, so s, dA, dP and the
+// records are bit for bit those of the whole-block form.  dQ is the sum of the four wavefronts'.
+constexpr int kSplitRows = 32;
+constexpr int kSplitWaves = 4;
+
+template <typename T, int D>
+struct SplitDqCfg {
+  static constexpr bool kTr = sizeof(T) == 2;
+  static constexpr int CH = 16 / (int)sizeof(T);
+  static constexpr int DP = D < 32 ? 32 : D;
+  static constexpr int LDK = kTr ? DP + 3 * CH : DP + CH;  // read along rows and along keys
+  static constexpr int LDV = DP + CH;
+  using KTile = DmaTile<T, D, kWaveKeys, LDK, 1, true>;
+  using VTile = DmaTile<T, D, kWaveKeys, LDV, 1, true>;
+  static constexpr int K_ELEMS = KTile::LDS_ELEMS;  // a wavefront's K tile
+  static constexpr int V_ELEMS = VTile::LDS_ELEMS;
+  static constexpr int KS = D / 16;
+  static constexpr int DT = DP / 32;
+  static constexpr int LDS = 32 + CH;  // score-store scratch: s and dP as [row][key], in the K tile
+  static constexpr int LDO = DP + 4;   // dQ partials (floats): rows 0..15 in the K tile, 16..31 in the V tile
+  static_assert(16 * LDO * 4 <= K_ELEMS * (int)sizeof(T) && 16 * LDO * 4 <= V_ELEMS * (int)sizeof(T),
+                "dQ partials alias the tiles");
+  // fp32 at D = 256 does not fit a CU's LDS.
+  static constexpr bool kFits = (size_t)kSplitWaves * (K_ELEMS + V_ELEMS) * sizeof(T) <= 155 * 1024;
+};
+
+template <typename T, int D, bool CAUSAL, bool STORE>
+__global__ __launch_bounds__(256, D * sizeof(T) > 256 ? 1 : 2) void coalibi_bwd_dq_split_kernel(BwdArgs args,
+                                                                                               int items) {
+  using C = SplitDqCfg<T, D>;
+  using M = Mfma<T>;
+  using vec8 = typename M::vec8;
+  static_assert(!STORE || 2 * 32 * C::LDS <= C::K_ELEMS, "the score scratch fits the K tile");
+  __shared__ __align__(16) T sK[kSplitWaves * C::K_ELEMS];
+  __shared__ __align__(16) T sV[kSplitWaves * C::V_ELEMS];
+  __shared__ float sSig[kSplitWaves][kSplitRows];  // the tiles' sigmoid totals
+  __shared__ float sDa[kSplitWaves][kSplitRows];   // and dA totals
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31, hh = lane >> 5;
+  const int Sq = args.Sq, Skv = args.Skv;
+  const int nQB = (Sq + kBM - 1) / kBM;
+  // The four parts of a row block run on one XCD (ids 8 apart) and share its K and V in L2.
+  const int i = (blockIdx.x >> 5) * 8 + (blockIdx.x & 7), part = (blockIdx.x >> 3) & 3;
+  if (i >= items) return;
+  // Every block of a head on one XCD: on a grid this small its K and V staying in one L2 counts for
+  // more than an even spread of the heads (n 512 to 2048: up to 15 % faster than the sorted order).
+  const WorkItem item = lpt_item(i, args.B * args.Hq, 1 << 30);
+  const int bh = item.head, qb = nQB - 1 - item.rank;
+  const int q0 = qb * kBM + part * kSplitRows;
+  if (q0 >= Sq) return;
+  const int b = bh / args.Hq, hq = bh - b * args.Hq;
+  const int hkv = hq / (args.Hq / args.Hkv);
+  const size_t qoff = (size_t)bh * Sq * D;
+  const size_t kvoff = ((size_t)b * args.Hkv + hkv) * (size_t)Skv * D;
+  const T* __restrict__ Kp = static_cast<const T*>(args.k) + kvoff;
+  const T* __restrict__ Vp = static_cast<const T*>(args.v) + kvoff;
+  T* const sKw = sK + wave * C::K_ELEMS;  // this wavefront's tiles
+  T* const sVw = sV + wave * C::V_ELEMS;
+  const float lam = args.slopes[hq];
+  const float lam2 = lam * kLog2e;
+  const int row = q0 + col;
+  const bool row_ok = row < Sq;
+  const float tile_sc2 = sizeof(T) == 2 ? 1.0f : args.sc2;  // Q carries the scale in 16-bit types
+
+  // Tiles kt0 .. nkt - 1, four per step; a tile past the last holds no key (zero rows).
+  const int kt0 = valid_kstart(args.kstart[(size_t)bh * nQB + qb], Skv) / kBN;
+  const int nkt = (CAUSAL ? min(q0 + kSplitRows - 1, Skv - 1) : Skv - 1) / kBN + 1;
+  const int steps = (max(nkt - kt0, 0) + kSplitWaves - 1) / kSplitWaves;
+
+  vec8 qf[C::KS], dof[C::KS];
+  float lse2, dpart = 0.f;
+  double zsum;  // z at the next step's start
+  {
+    const int rows = min(Sq - q0, kSplitRows);
+    const size_t blk = qoff + (size_t)q0 * D;
+    const __amdgpu_buffer_rsrc_t qrs = tile_rsrc(static_cast<const T*>(args.q) + blk, rows * D);
+    const __amdgpu_buffer_rsrc_t dors = tile_rsrc(static_cast<const T*>(args.dout) + blk, rows * D);
+    const __amdgpu_buffer_rsrc_t ors = tile_rsrc(static_cast<const T*>(args.o) + blk, rows * D);
+    vec8 of[C::KS];
+#pragma unroll
+    for (int ks = 0; ks < C::KS; ++ks) {
+      const int off = (col * D + hh * 8 + ks * 16) * (int)sizeof(T);
+      qf[ks] = buffer_load_vec8<vec8>(qrs, off);
+      dof[ks] = buffer_load_vec8<vec8>(dors, off);
+      of[ks] = buffer_load_vec8<vec8>(ors, off);
+    }
+    const size_t nrows = (size_t)args.B * args.Hq * Sq, at = (size_t)bh * Sq + q0;
+    auto row_value = [&](const float* p) {
+      return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(tile_rsrc(p, rows), col * 4, 0, 0));
+    };
+    lse2 = row_value(args.lse + at) * kLog2e;
+    zsum = (double)row_value(args.rsum + at) + (double)row_value(args.rsum + nrows + at);
+#pragma unroll
+    for (int ks = 0; ks < C::KS; ++ks) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) dpart += (float)dof[ks][e] * (float)of[ks][e];
+      if constexpr (sizeof(T) == 2) qf[ks] = scale_vec8<T>(qf[ks], args.sc2);
+    }
+  }
+  const float dsum = dpart + other_half(dpart);
+  if (wave == 0 && hh == 0 && row_ok) args.dsum[(size_t)bh * Sq + row] = dsum;
+
+  // Untracked DMA: the tiles are this wavefront's own, and the waits below order it.
+  typename C::KTile kdma;
+  typename C::VTile vdma;
+  kdma.init(0, lane);
+  vdma.init(0, lane);
+  const unsigned lds_k = lds_address(sKw), lds_v = lds_address(sVw);
+  auto issue_k = [&](int t) { kdma.issue_untracked(Kp, t < nkt ? t * kBN : 0, t < nkt ? Skv : 0, lds_k, 0); };
+  auto issue_v = [&](int t) { vdma.issue_untracked(Vp, t < nkt ? t * kBN : 0, t < nkt ? Skv : 0, lds_v, 0); };
+  int t = kt0 + wave;
+  if (steps > 0) {
+    issue_v(t);
+    issue_k(t);
+  }
+
+  f32x16 acc[C::DT];
+#pragma unroll
+  for (int dt = 0; dt < C::DT; ++dt) acc[dt] = f32x16{};
+  float crun = 0.f;
+  float* __restrict__ zb_row = STORE ? nullptr : args.zb + (size_t)bh * args.nZB * Sq + row;
+  float* __restrict__ cb_row = STORE ? nullptr : args.cb + (size_t)bh * args.nZB * Sq + row;
+  const int nQ32 = (Sq + 31) / 32;
+
+  for (int s = 0; s < steps; ++s, t += kSplitWaves) {
+    const bool more = s + 1 < steps, live = t < nkt;
+    const int k0 = t * kBN, key0 = k0 + hh * 16;
+    const bool masked = !live || (CAUSAL && k0 + kBN - 1 > q0) || k0 + kBN > Skv || q0 + kSplitRows > Sq;
+    // The step's K and V; the record stores of the step before, issued after them, may still run.
+    if (STORE && s > 0)
+      wait_vm<4>();
+    else
+      wait_vm<0>();
+    f32x16 sacc = f32x16{}, dacc;
+    float ndsum = -dsum;
+    asm volatile("" : "+v"(ndsum));  // rebuilt every step, as in the whole-block form
+#pragma unroll
+    for (int r = 0; r < 16; ++r) dacc[r] = ndsum;
+#pragma unroll
+    for (int ks = 0; ks < C::KS; ++ks) {
+      sacc = M::k16(ld_vec8(sKw + col * C::LDK + ks * 16 + hh * 8), qf[ks], sacc);
+      dacc = M::k16(ld_vec8(sVw + col * C::LDV + ks * 16 + hh * 8), dof[ks], dacc);
+    }
+    if (more) {  // the V tile has been read: the next one lands in it during this step's math
+      wait_lds();
+      issue_v(t + kSplitWaves);
+    }
+    float sg[16], ex[16];
+    const float tot = masked ? dp_sigma<true, CAUSAL>(sacc, key0, row, Skv, Sq, tile_sc2, lam2, sg, ex)
+                             : dp_sigma<false, CAUSAL>(sacc, key0, row, Skv, Sq, tile_sc2, lam2, sg, ex);
+    const float oth = other_half(tot);
+    if (hh == 0) sSig[wave][col] = tot + oth;
+    lds_barrier();
+    float zb = 0.f;
+#pragma unroll
+    for (int w = 0; w < kSplitWaves; ++w) {
+      if (w == wave) zb = (float)zsum;
+      zsum -= (double)sSig[w][col];
+    }
+    const float cst = dp_exponent(zb, tot, oth, hh, lam2, lse2);
+    vec8 sb[2], pb[2];
+    const float atot = masked ? dp_scores<T, true, CAUSAL>(ex, cst, dacc, key0, row, Skv, Sq, sb)
+                              : dp_scores<T, false, CAUSAL>(ex, cst, dacc, key0, row, Skv, Sq, sb);
+    const float aoth = other_half(atot);
+    if (hh == 0) sDa[wave][col] = aoth + atot;
+    lds_barrier();
+    float cb = 0.f;
+#pragma unroll
+    for (int w = 0; w < kSplitWaves; ++w) {
+      if (w == wave) cb = crun;
+      crun += sDa[w][col];
+    }
+    const float c = lam * (cb + (hh ? aoth : 0.f));
+    if (masked)
+      dp_grads<T, true, CAUSAL>(dacc, sg, c, lam, key0, row, Skv, Sq, pb);
+    else
+      dp_grads<T, false, CAUSAL>(dacc, sg, c, lam, key0, row, Skv, Sq, pb);
+    if constexpr (!STORE) {
+      if (hh == 0 && row_ok && live) {
+        zb_row[(size_t)t * Sq] = zb;
+        cb_row[(size_t)t * Sq] = cb;
+      }
+    }
+#pragma unroll
+    for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+      for (int mh = 0; mh < 2; ++mh)
+        acc[dt] = M::k16(ld_kmajor_any<T, true>(sKw, C::LDK, mh * 8, 16, dt * 32, lane), pb[mh], acc[dt]);
+    if constexpr (STORE) {
+      // As the whole-block form: s and dP through LDS (here the K tile, which has been read) into
+      // the operand order of pass 2.  The next K tile's DMA goes out between the reads and the stores.
+      T* __restrict__ sc = sKw;
+      asm volatile("" ::: "memory");
+      *reinterpret_cast<vec8*>(sc + col * C::LDS + hh * 16) = sb[0];
+      *reinterpret_cast<vec8*>(sc + col * C::LDS + hh * 16 + 8) = sb[1];
+      *reinterpret_cast<vec8*>(sc + (32 + col) * C::LDS + hh * 16) = pb[0];
+      *reinterpret_cast<vec8*>(sc + (32 + col) * C::LDS + hh * 16 + 8) = pb[1];
+      asm volatile("" ::: "memory");
+      u32x4 rec[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+        rec[m] = __builtin_bit_cast(
+            u32x4, ld_kmajor<T, false>(sc + (m >> 1) * 32 * C::LDS, C::LDS, (m & 1) * 16, 8, 0, lane));
+      if (more) {
+        wait_lds();
+        issue_k(t + kSplitWaves);
+      }
+      const size_t at = live ? (size_t)bh * args.score_head + score_record(t, q0 / 32, nQ32, CAUSAL) : 0;
+      const __amdgpu_buffer_rsrc_t rs =
+          tile_rsrc(reinterpret_cast<const u32x4*>(static_cast<const char*>(args.scores) + at * kScoreRecordBytes),
+                    live ? kScoreRecordBytes / 16 : 0);
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+        __builtin_amdgcn_raw_buffer_store_b128(rec[m], rs, (m * 64 + lane) * 16, 0, kCachePolicyNt);
+      asm volatile("" ::: "memory");
+    } else if (more) {
+      wait_lds();
+      issue_k(t + kSplitWaves);
+    }
+  }
+
+  // dQ: the four wavefronts' sums.
+  auto dq_row = [&](int w, int r) {
+    return reinterpret_cast<float*>(r < 16 ? sK + w * C::K_ELEMS : sV + w * C::V_ELEMS) + (r & 15) * C::LDO;
+  };
+  float* const own = dq_row(wave, col);
+#pragma unroll
+  for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<f32x4*>(own + dt * 32 + g * 8 + hh * 4) =
+          f32x4{acc[dt][g * 4], acc[dt][g * 4 + 1], acc[dt][g * 4 + 2], acc[dt][g * 4 + 3]};
+  __syncthreads();
+  const int r = tid >> 3;
+  if (q0 + r < Sq) {
+    using vec4 = typename VecOf<T, 4>::type;
+    T* __restrict__ dQr = static_cast<T*>(args.dq) + qoff + (size_t)(q0 + r) * D;
+    for (int c = (tid & 7) * 4; c < D; c += 32) {
+      f32x4 v = *reinterpret_cast<const f32x4*>(dq_row(0, r) + c);
+#pragma unroll
+      for (int w = 1; w < kSplitWaves; ++w) v += *reinterpret_cast<const f32x4*>(dq_row(w, r) + c);
+      *reinterpret_cast<vec4*>(dQr + c) = __builtin_convertvector(v * args.sm_scale, vec4);
+    }
+  }
+}
+
+// Whether pass 1 takes the split form.  As in the forward (split_grid) it wins where the row blocks
+// leave the GPU room.  At D = 128 in 16-bit types a step waits longer for its own K, whose tile the
+// dQ product reads last, and the limit is lower.  us, whole-block form -> split, fp16 (f = tail
+// skip off):
+//   D 64   n 512: 128 blocks 25.0 -> 17.2 f 25.0 -> 14.5, 192: 25.0 -> 22.1, 256: 25.9 -> 26.7
+//          n 1024: 128 blocks 44.1 -> 21.7, 320: 46.2 -> 36.0 f 46.0 -> 42.8, 384: 46.7 -> 41.0 f 46.7 -> 47.3
+//          n 2048: 128 blocks 82.6 -> 36.9, 384: 84.8 -> 52.4 f 88.2 -> 75.5, 512: 86.1 -> 67.7 f 89.3 -> 95.9
+//   D 128  n 512: 128 blocks 31.3 -> 27.8 f 30.1 -> 23.5, 192: 32.4 -> 34.7
+//          n 1024: 128 blocks 53.8 -> 41.3 f 52.3 -> 37.5, 256: 55.2 -> 55.3
+//          n 2048: 128 blocks 98.2 -> 72.7 f 97.1 -> 69.1, 256: 99.3 -> 82.4 f 100.2 -> 84.7, 320: f 103.3 -> 114.0
+//   non-causal, D 128: 333 x 2047, 96 blocks 103.4 -> 67.7; 2000 x 3000, 256 blocks f 158.0 -> 195.3;
+//          D 64, 1400 x 1400, 352 blocks 64.1 -> 49.5
+//   fp32   D 64: n 1000, 192 blocks 133.9 -> 74.6;  D 128: n 1024, 128 blocks 240.5 -> 109.6
+template <typename T, int D>
+inline bool split_dq_grid(long long row_blocks, int keys, bool causal) {
+  if (sizeof(T) == 2 && D >= 128) return row_blocks <= (causal ? std::max(128, std::min(keys / 5, 256)) : 128);
+  return row_blocks <= std::max(128, causal ? std::min(keys / 3, 384) : std::min(keys / 4, 320));
 }
 
 // Pass 2's rotation of the heads over the XCDs (balanced_item): runs of kLptRotateRanks key
@@ -1196,14 +1496,23 @@ hipError_t launch_bwd(const BwdArgs& a, int stages, hipStream_t stream) {
   const bool store = kStore && a.scores != nullptr;
   static_assert(kStoreBK == kOrderKeyBlock && kPairBK == kOrderKeyBlock, "key_order numbers 64-key blocks");
   if (stages & 1) {
-    const int nQB = (a.Sq + kBM - 1) / kBM;
-    if (store) {
+    const int nQB = (a.Sq + kBM - 1) / kBM, blocks = nQB * a.B * a.Hq;
+    bool split = false;
+    if constexpr (SplitDqCfg<T, D>::kFits) {
+      split = split_dq_grid<T, D>(blocks, a.Skv, CAUSAL);
+      const dim3 parts((blocks + 7) / 8 * 32);
+      if (split && store) {
+        if constexpr (kStore)
+          hipLaunchKernelGGL((coalibi_bwd_dq_split_kernel<T, D, CAUSAL, true>), parts, dim3(256), 0, stream, a, blocks);
+      } else if (split) {
+        hipLaunchKernelGGL((coalibi_bwd_dq_split_kernel<T, D, CAUSAL, false>), parts, dim3(256), 0, stream, a, blocks);
+      }
+    }
+    if (!split && store) {
       if constexpr (kStore)
-        hipLaunchKernelGGL((coalibi_bwd_dq_kernel<T, D, CAUSAL, true>), dim3(nQB * a.B * a.Hq), dim3(256), 0, stream,
-                           a);
-    } else {
-      hipLaunchKernelGGL((coalibi_bwd_dq_kernel<T, D, CAUSAL, false>), dim3(nQB * a.B * a.Hq), dim3(256), 0, stream,
-                         a);
+        hipLaunchKernelGGL((coalibi_bwd_dq_kernel<T, D, CAUSAL, true>), dim3(blocks), dim3(256), 0, stream, a);
+    } else if (!split) {
+      hipLaunchKernelGGL((coalibi_bwd_dq_kernel<T, D, CAUSAL, false>), dim3(blocks), dim3(256), 0, stream, a);
     }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
