@@ -689,7 +689,8 @@ __device__ __forceinline__ int pass2_rotate(const BwdArgs& args) {
 }
 
 // ---------------------------------------------------------------------------
-// Pass 2, fp32 validation mode: dK, dV.  Per wavefront the 32 keys kw0.. of one
+// Pass 2 (recompute path) of 128 keys per work-group, for fp32 and for 16-bit types at D <= 32
+// where the 32-key form below does not take the call: dK, dV.  Per wavefront the 32 keys kw0.. of one
 // 32-key block, held as MFMA A operands (row R <-> key kw0 + kRowOfReg(R)) so that
 // register r of lane (col, hh) of S^T <-> key kw0 + hh*16 + r, query q0 + sq*32 + col.
 // The 16-bit kernel below splits this work over wavefront pairs; fp32 tiles with
@@ -944,6 +945,298 @@ __global__ __launch_bounds__(256, 1) void coalibi_bwd_dkdv_f32_kernel(BwdArgs ar
   }
 }
 
+
+// Pass 2 (recompute path) of 32 keys per work-group, for fp32 at D <= 64 and 16-bit types at
+// D <= 32 (use_key_form).  Every wavefront holds the 32 keys as MFMA A operands and takes every
+// fourth 32-row query tile, from Q and dO tiles of its own that its own untracked DMA fills, so the
+// four run without a barrier; their sums meet once, at the end.  The 128-key form above has a
+// quarter of the work-groups, each walking four times as many tiles: at B2 H12 n 1000 D64 fp32 its
+// 192 work-groups leave 64 CUs idle and the longest causal block sets the time (213 us; this form
+// 100).  What bounds it: the fp32 products (v_mfma_f32_32x32x2, 64 cycles each) of one
+// wavefront per SIMD, with the next tile's DMA partly exposed (there is no LDS for a second pair of
+// tiles).  At D = 128 in fp32 the operands and compensated sums do not fit the registers beside a
+// tile's state (319 spilled, 3.5 times slower on a full GPU).
+constexpr int kKeyWaves = 4;
+constexpr int kKeyLiveWords = 512;  // LDS bits of the row blocks that processed the keys
+
+template <typename T, int D>
+struct KeyCfg {
+  static constexpr bool kTr = sizeof(T) == 2;
+  static constexpr int CH = 16 / (int)sizeof(T);
+  static constexpr int DP = D < 32 ? 32 : D;
+  static constexpr int LDR = kTr ? DP + 2 * CH : DP + CH;  // Q / dO tile rows
+  using Tile = DmaTile<T, D, kWaveKeys, LDR, 1, false>;
+  static constexpr int LDSP = 32 + (kTr ? 2 : 1) * CH;  // s / dP scratch: [q][key] (fp32: [key][q])
+  static constexpr int LDO = DP + 4;                    // the merged sums (floats): [key][d]
+  static constexpr int kSumBytes = 32 * LDO * 4;
+  // A wavefront's Q tile, dO tile and scratch; at the end dK aliases the first part, dV the second.
+  static constexpr int kTileBytes = Tile::LDS_ELEMS * (int)sizeof(T) > kSumBytes ? Tile::LDS_ELEMS * (int)sizeof(T)
+                                                                                   : kSumBytes;
+  static constexpr int kScratchBytes = 32 * LDSP * (int)sizeof(T);
+  static constexpr int kWaveBytes = 2 * kTileBytes + kScratchBytes;
+  static constexpr int KS = D / 16;
+  static constexpr int DT = DP / 32;
+};
+
+// Which form of the recompute path's pass 2 a launch takes (16-bit types at D >= 64 have their own
+// kernel).  The 32-key form wins where the 128-key blocks are few, and where a wavefront's walk (a
+// tile per row block and query head) is long enough to carry its prologue and merge; in 16-bit types
+// the 128-key form is ahead again once its work-groups fill the GPU.  us, 128-key -> 32-key:
+//   fp32 D 64: B1 H2 n 128 31 -> 12, B2 H12 n 1000 213 -> 100, B4 H16 n 2048 806 -> 755, Hq16/Hkv4
+//     n 2000 1593 -> 388, B8 H32 n 300 137 -> 170;  D 32: B4 H16 n 2048 364 -> 337
+//   fp16 D 32: B8 H8 n 512 (256 blocks) 27 -> 20, B2 H16 n 2048 (512) 101 -> 81, B16 H16 n 256 (512)
+//     17 -> 27, B2 H16 n 3000 (768) 147 -> 157, B4 H16 n 2048 (1024) 112 -> 122
+template <typename T, int D>
+constexpr bool kHasKeyForm = D * sizeof(T) <= (sizeof(T) == 2 ? 64 : 256);
+template <typename T>
+inline bool use_key_form(long long key_blocks, int tiles) {
+  if (key_blocks <= 256) return true;
+  return tiles >= 8 && (sizeof(T) == 4 || key_blocks <= 640);
+}
+
+template <typename T, int D, bool CAUSAL>
+__global__ __launch_bounds__(256, D * sizeof(T) > 128 ? 1 : 2) void coalibi_bwd_dkdv_key_kernel(BwdArgs args) {
+  using C = KeyCfg<T, D>;
+  using M = Mfma<T>;
+  using vec8 = typename M::vec8;
+  __shared__ __align__(16) char smem[kKeyWaves * C::kWaveBytes];
+  __shared__ unsigned sLive[kKeyLiveWords];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31, hh = lane >> 5;
+  const int Sq = args.Sq, Skv = args.Skv;
+  static_assert(sizeof(smem) >= 2 * kMaxBalancedHeads * 4, "the head order is built in smem");
+  const WorkItem item = balanced_item(blockIdx.x, args.B, args.Hkv, args.slopes, args.Hq / args.Hkv,
+                                      reinterpret_cast<float*>(smem), reinterpret_cast<int*>(smem) + kMaxBalancedHeads,
+                                      tid, 256, pass2_rotate(args));
+  const int bhk = item.head;  // b * Hkv + hkv
+  const int kb = item.rank;   // rank 0: key block 0, seen by the most query rows
+  const int b = bhk / args.Hkv, hkv = bhk - b * args.Hkv;
+  const int group = args.Hq / args.Hkv;
+  const size_t kvoff = (size_t)bhk * Skv * D;
+  const int kw0 = kb * kWaveKeys, key0 = kw0 + hh * 16;
+  T* const sQ = reinterpret_cast<T*>(smem + wave * C::kWaveBytes);
+  T* const sdO = reinterpret_cast<T*>(smem + wave * C::kWaveBytes + C::kTileBytes);
+  T* const sSP = reinterpret_cast<T*>(smem + wave * C::kWaveBytes + 2 * C::kTileBytes);
+
+  vec8 ka[C::KS], va[C::KS];
+  {
+    const int key = kw0 + kRowOfReg(col);
+    const bool key_ok = key < Skv;
+    const T* __restrict__ Kr = static_cast<const T*>(args.k) + kvoff + (size_t)key * D;
+    const T* __restrict__ Vr = static_cast<const T*>(args.v) + kvoff + (size_t)key * D;
+#pragma unroll
+    for (int ks = 0; ks < C::KS; ++ks) {
+      ka[ks] = key_ok ? ld_vec8(Kr + ks * 16 + hh * 8) : zero_vec8<T>();
+      // 16-bit types: K pre-scaled by sm_scale*log2(e), so S^T comes out in log2 units.
+      if constexpr (sizeof(T) == 2) ka[ks] = scale_vec8<T>(ka[ks], args.sc2);
+      va[ks] = key_ok ? ld_vec8(Vr + ks * 16 + hh * 8) : zero_vec8<T>();
+    }
+  }
+  const float tile_sc2 = sizeof(T) == 2 ? 1.0f : args.sc2;
+
+  // Row block rb of query head g is live if the forward processed these keys for it: bit rb % 32 of
+  // word g * wph + rb / 32, where the group's words fit; read from kstart otherwise.
+  const int nRB = (Sq + kSkipRows - 1) / kSkipRows, wph = (nRB + 31) / 32;
+  const int* __restrict__ kstart_g = args.kstart + (size_t)(b * args.Hq + hkv * group) * nRB;
+  const bool listed = (long long)group * wph <= kKeyLiveWords;
+  if (listed) {
+    for (int i = wave; i < group * ((wph + 1) / 2); i += kKeyWaves) {
+      const int g = i / ((wph + 1) / 2), w0 = (i - g * ((wph + 1) / 2)) * 2, rb = w0 * 32 + lane;
+      const unsigned long long m = __ballot(rb < nRB && valid_kstart(kstart_g[(size_t)g * nRB + rb], Skv) <= kw0);
+      if (lane == 0) {
+        sLive[g * wph + w0] = (unsigned)m;
+        if (w0 + 1 < wph) sLive[g * wph + w0 + 1] = (unsigned)(m >> 32);
+      }
+    }
+  }
+  __syncthreads();  // sLive; the head-order scratch is free again
+
+  // This wavefront's query tiles: of every live row block of every head of the group, tile
+  // (wave + g) % 4 of its four.
+  struct Pos {
+    int g, qt;  // g == group: none left
+  };
+  const int rb0 = CAUSAL ? kw0 / kSkipRows : 0;  // the first row block that sees the keys
+  auto next = [&](int g, int rb) -> Pos {        // from row block rb of head g on
+    for (; g < group; ++g, rb = rb0) {
+      for (; rb < nRB; ++rb) {
+        if (listed) {  // the next set bit of the word, or the next word
+          const unsigned w = __builtin_amdgcn_readfirstlane(sLive[g * wph + rb / 32]) >> (rb % 32);
+          if (w == 0) {
+            rb |= 31;
+            continue;
+          }
+          rb += __builtin_ctz(w);
+        } else if (kw0 < valid_kstart(kstart_g[(size_t)g * nRB + rb], Skv)) {
+          continue;
+        }
+        const int qt = rb * (kSkipRows / 32) + ((wave + g) & 3);
+        if (qt * 32 < Sq && (!CAUSAL || qt * 32 + 31 >= kw0)) return {g, qt};
+      }
+    }
+    return {group, 0};
+  };
+
+  typename C::Tile dma;
+  dma.init(0, lane);
+  const unsigned lds_q = lds_address(sQ), lds_do = lds_address(sdO);
+  const size_t head0 = (size_t)(b * args.Hq + hkv * group) * Sq;
+  auto issue_do = [&](const Pos& p) {
+    dma.issue_untracked(static_cast<const T*>(args.dout) + (head0 + (size_t)p.g * Sq) * D, p.qt * 32, Sq, lds_do, 0);
+  };
+  auto issue_q = [&](const Pos& p) {
+    dma.issue_untracked(static_cast<const T*>(args.q) + (head0 + (size_t)p.g * Sq) * D, p.qt * 32, Sq, lds_q, 0);
+  };
+  // The row statistics of a tile: lane (col, hh) holds row col's (zero past Sq).
+  struct Rows {
+    float lse2, dsum, zb, cb;
+  };
+  auto load_rows = [&](const Pos& p) {
+    const size_t bh = (size_t)b * args.Hq + hkv * group + p.g;
+    const int q0 = p.qt * 32, rows = min(Sq - q0, 32);
+    auto at = [&](const float* base) {
+      return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(tile_rsrc(base + q0, rows), col * 4, 0, 0));
+    };
+    const size_t blk = (bh * args.nZB + kb) * Sq;
+    return Rows{at(args.lse + bh * Sq) * kLog2e, at(args.dsum + bh * Sq), at(args.zb + blk), at(args.cb + blk)};
+  };
+
+  f32x16 dk[C::DT], dv[C::DT];
+  f32x16 ck[sizeof(T) == 4 ? C::DT : 1], cv[sizeof(T) == 4 ? C::DT : 1];  // fp32: the sums' compensations
+#pragma unroll
+  for (int dt = 0; dt < C::DT; ++dt) {
+    dk[dt] = f32x16{};
+    dv[dt] = f32x16{};
+    if constexpr (sizeof(T) == 4) {
+      ck[dt] = f32x16{};
+      cv[dt] = f32x16{};
+    }
+  }
+
+  Pos cur = next(0, rb0);
+  Rows rows{};
+  if (cur.g < group) {
+    rows = load_rows(cur);
+    issue_do(cur);
+    issue_q(cur);
+  }
+  while (cur.g < group) {
+    const Pos nxt = next(cur.g, cur.qt / 4 + 1);
+    const bool more = nxt.g < group;
+    const float lam = args.slopes[hkv * group + cur.g], lam2 = lam * kLog2e;
+    const int qs0 = cur.qt * 32, row = qs0 + col;
+    const bool masked = (CAUSAL && qs0 < kw0 + 31) || qs0 + 32 > Sq || kw0 + 32 > Skv;
+    wait_vm<0>();  // this tile's Q and dO
+    f32x16 sacc = f32x16{}, dacc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) dacc[r] = -rows.dsum;
+#pragma unroll
+    for (int ks = 0; ks < C::KS; ++ks) {
+      sacc = M::k16(ka[ks], ld_vec8(sQ + col * C::LDR + ks * 16 + hh * 8), sacc);
+      dacc = M::k16(va[ks], ld_vec8(sdO + col * C::LDR + ks * 16 + hh * 8), dacc);
+    }
+    vec8 sb[2], pb[2];
+    float atot, ztot;
+    if (masked)
+      dp_tile<T, true, CAUSAL>(sacc, dacc, rows.zb, rows.cb, rows.lse2, key0, row, hh, Skv, Sq, tile_sc2, lam, lam2,
+                               sb, pb, atot, ztot);
+    else
+      dp_tile<T, false, CAUSAL>(sacc, dacc, rows.zb, rows.cb, rows.lse2, key0, row, hh, Skv, Sq, tile_sc2, lam, lam2,
+                                sb, pb, atot, ztot);
+    if (more) rows = load_rows(nxt);
+    // s, then dP, through the scratch into operands reduced over queries mh*16 + hh*8 + e.
+    auto exchange = [&](const vec8 (&x)[2], vec8 (&op)[2]) {
+      asm volatile("" ::: "memory");
+      if constexpr (C::kTr) {
+        *reinterpret_cast<vec8*>(sSP + col * C::LDSP + hh * 16) = x[0];
+        *reinterpret_cast<vec8*>(sSP + col * C::LDSP + hh * 16 + 8) = x[1];
+      } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sSP[(hh * 16 + r) * C::LDSP + col] = x[r >> 3][r & 7];
+      }
+      asm volatile("" ::: "memory");  // other lanes' values: LDS operations of a wavefront run in order
+#pragma unroll
+      for (int mh = 0; mh < 2; ++mh) {
+        if constexpr (C::kTr)
+          op[mh] = ld_kmajor<T, false>(sSP, C::LDSP, mh * 16, 8, 0, lane);
+        else
+          op[mh] = ld_vec8(sSP + col * C::LDSP + mh * 16 + hh * 8);
+      }
+    };
+    // acc^T[d][key] += x^T[d][q] op[q][key], each tile summed in a fresh accumulator that is then
+    // added to the running one: one rounding at the running sum's magnitude per tile.  fp32:
+    // compensated (Kahan) running sums, so that they stay within a few ulps over any number of tiles.
+    auto reduce = [&](const T* tile, const vec8 (&op)[2], f32x16 (&sum)[C::DT],
+                      f32x16 (&comp)[sizeof(T) == 4 ? C::DT : 1]) {
+#pragma unroll
+      for (int dt = 0; dt < C::DT; ++dt) {
+        f32x16 t = f32x16{};
+#pragma unroll
+        for (int mh = 0; mh < 2; ++mh)
+          t = M::k16(ld_kmajor_any<T, false>(tile, C::LDR, mh * 16, 8, dt * 32, lane), op[mh], t);
+        if constexpr (sizeof(T) == 4) {
+          const f32x16 y = t - comp[dt], n = sum[dt] + y;
+          comp[dt] = (n - sum[dt]) - y;
+          sum[dt] = n;
+        } else {
+          sum[dt] += t;
+        }
+      }
+    };
+    vec8 op[2];
+    exchange(sb, op);
+    reduce(sdO, op, dv, cv);
+    if (more) {  // the dO tile has been read: the next one lands in it during the dK products
+      wait_lds();
+      issue_do(nxt);
+    }
+    exchange(pb, op);
+    reduce(sQ, op, dk, ck);
+    if (more) {
+      wait_lds();
+      issue_q(nxt);
+    }
+    cur = nxt;
+  }
+
+  // The four wavefronts' sums, [key][d] over each wavefront's own tiles.
+  auto sums = [&](int w, int which) {
+    return reinterpret_cast<float*>(smem + w * C::kWaveBytes + which * C::kTileBytes);
+  };
+#pragma unroll
+  for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int at = col * C::LDO + dt * 32 + g * 8 + hh * 4;
+      *reinterpret_cast<f32x4*>(sums(wave, 0) + at) =
+          f32x4{dk[dt][g * 4], dk[dt][g * 4 + 1], dk[dt][g * 4 + 2], dk[dt][g * 4 + 3]};
+      *reinterpret_cast<f32x4*>(sums(wave, 1) + at) =
+          f32x4{dv[dt][g * 4], dv[dt][g * 4 + 1], dv[dt][g * 4 + 2], dv[dt][g * 4 + 3]};
+    }
+  __syncthreads();
+  const int r = tid >> 3;
+  if (kw0 + r < Skv) {
+    using vec4 = typename VecOf<T, 4>::type;
+    const size_t at = kvoff + (size_t)(kw0 + r) * D;
+    for (int c = (tid & 7) * 4; c < D; c += 32) {
+#pragma unroll
+      for (int which = 0; which < 2; ++which) {
+        double s[4] = {};  // four partial sums: a rounding of their own would show in fp32
+#pragma unroll
+        for (int w = 0; w < kKeyWaves; ++w) {
+          const f32x4 v = *reinterpret_cast<const f32x4*>(sums(w, which) + r * C::LDO + c);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) s[e] += (double)v[e];
+        }
+        const float sc = which == 0 ? args.sm_scale : 1.0f;
+        const f32x4 out = {(float)s[0] * sc, (float)s[1] * sc, (float)s[2] * sc, (float)s[3] * sc};
+        *reinterpret_cast<vec4*>(static_cast<T*>(which == 0 ? args.dk : args.dv) + at + c) =
+            __builtin_convertvector(out, vec4);
+      }
+    }
+  }
+}
 
 // Pass 2 for fp16/bf16: dK, dV with wavefront pairs.  A work-group of 4
 // wavefronts owns 64 keys in two key groups kg of 32 and walks query tiles of 64
@@ -1535,8 +1828,17 @@ hipError_t launch_bwd(const BwdArgs& a, int stages, hipStream_t stream) {
                          0, stream, a);
     } else {
       const int nKB = (a.Skv + kBK - 1) / kBK;
-      hipLaunchKernelGGL((coalibi_bwd_dkdv_f32_kernel<T, D, CAUSAL>), dim3(nKB * a.B * a.Hkv), dim3(256), 0,
-                         stream, a);
+      bool key_form = false;
+      if constexpr (kHasKeyForm<T, D>) {
+        key_form = use_key_form<T>(static_cast<long long>(nKB) * a.B * a.Hkv,
+                                   a.Hq / a.Hkv * ((a.Sq + kSkipRows - 1) / kSkipRows));
+        if (key_form)
+          hipLaunchKernelGGL((coalibi_bwd_dkdv_key_kernel<T, D, CAUSAL>),
+                             dim3((a.Skv + kWaveKeys - 1) / kWaveKeys * a.B * a.Hkv), dim3(256), 0, stream, a);
+      }
+      if (!key_form)
+        hipLaunchKernelGGL((coalibi_bwd_dkdv_f32_kernel<T, D, CAUSAL>), dim3(nKB * a.B * a.Hkv), dim3(256), 0,
+                           stream, a);
     }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;

@@ -50,3 +50,21 @@ def test_split_edges(case, dtype, skip):
     ro, _ = ref.forward(qf, kf, vf, lam, causal=causal, scale=scale)
     want = (ro, *ref.backward(dof, qf, kf, vf, lam, causal=causal, scale=scale))
     assert_parity(got, want, TOL[dtype], f"{case}", dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32], ids=["fp16", "fp32"])
+def test_key_form_many_query_heads(dtype):
+    """Pass 2's 32-key form with more query heads per key head than its LDS bits of processed row
+    blocks hold (600 heads, a word each): the bits are read from the forward's record instead."""
+    q, k, v, do = rand_inputs(1, 600, 1, 70, 40, 16, dtype, seed=5)
+    do = do * 0.05
+    lam = torch.linspace(0.001, 2.0, 600).to(dtype).float()
+    qd, kd, vd = (t.to(DEV).requires_grad_() for t in (q, k, v))
+    o = CoALIBIAttention.apply(qd, kd, vd, lam.to(DEV), True, 0.25)
+    o.backward(do.to(DEV))
+    torch.cuda.synchronize()
+    got = tuple(t.detach().float().cpu() for t in (o, qd.grad, kd.grad, vd.grad))
+    qf, kf, vf, dof = (t.float() for t in (q, k, v, do))
+    ro, _ = ref.forward(qf, kf, vf, lam, causal=True, scale=0.25)
+    want = (ro, *ref.backward(dof, qf, kf, vf, lam, causal=True, scale=0.25))
+    assert_parity(got, want, TOL[dtype], "600 heads", dtype)
