@@ -31,7 +31,9 @@ EXPORTS = (
     "co_alibi_fwd",
     "co_alibi_fwd_inference_workspace_bytes",
     "co_alibi_fwd_inference",
+    "co_alibi_fwd_strided",
     "co_alibi_bwd",
+    "co_alibi_bwd_strided",
     "co_alibi_bwd_dq",
     "co_alibi_bwd_dkdv",
     "co_alibi_decode_workspace_bytes",
@@ -46,6 +48,7 @@ _P = ctypes.c_void_p
 _I = ctypes.c_int
 _F = ctypes.c_float
 _Z = ctypes.c_size_t
+_L = ctypes.POINTER(ctypes.c_longlong)
 
 _SIGNATURES = {
     "co_alibi_stats_numel": (_Z, [_I, _I, _I, _I]),
@@ -56,6 +59,14 @@ _SIGNATURES = {
     "co_alibi_fwd": (_I, [_I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _P]),
     "co_alibi_fwd_inference_workspace_bytes": (_Z, [_I, _I, _I, _I]),
     "co_alibi_fwd_inference": (_I, [_I, _P, _P, _P, _P, _P, _P, _Z, _I, _I, _I, _I, _I, _I, _I, _F, _P]),
+    "co_alibi_fwd_strided": (
+        _I,
+        [_I, _P, _P, _P, _P, _P, _L, _P, _P, _P, _Z, _I, _I, _I, _I, _I, _I, _I, _F, _P],
+    ),
+    "co_alibi_bwd_strided": (
+        _I,
+        [_I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L, _P, _Z, _I, _I, _I, _I, _I, _I, _I, _F, _P],
+    ),
     "co_alibi_bwd": (
         _I,
         [_I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _Z, _I, _I, _I, _I, _I, _I, _I, _F, _P],
@@ -96,7 +107,11 @@ def lib() -> ctypes.CDLL:
             raise RuntimeError("co_alibi_attn: native library ABI version mismatch; "
                                "run `python -m co_alibi_attn._build`")
         for name, (res, args) in _SIGNATURES.items():
-            fn = getattr(handle, name)
+            try:
+                fn = getattr(handle, name)
+            except AttributeError:  # built before the symbol was added
+                raise RuntimeError(f"co_alibi_attn: native library lacks {name}; "
+                                   "run `python -m co_alibi_attn._build`") from None
             fn.restype = res
             fn.argtypes = args
         _lib = handle

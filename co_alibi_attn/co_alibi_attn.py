@@ -120,12 +120,32 @@ def co_alibi_attention(q, k, v, causal=True, sm_scale=None, bias_max=8.0):
     """
     if sm_scale is None:
         sm_scale = 1.0 / (q.shape[-1] ** 0.5)
-    q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    needs_grad = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad)
+    if needs_grad:  # what the backward reads are the op's own copies; without one the views are read in place
+        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
     num_q_heads = q.shape[1]
     slopes = _device_slopes(num_q_heads, bias_max, q.dtype, q.device)
     _check_inputs(q, k, v, slopes)
-    needs_grad = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad)
     return ops.fwd(q, k, v, slopes, bool(causal), float(sm_scale), needs_grad)[0]
+
+
+def co_alibi_attention_qkv(qkv, causal=True, sm_scale=None, bias_max=8.0):
+    """``co_alibi_attention`` of a fused projection's output: qkv is (B, S, 3, H, D) (q, k and v of
+    every head), the result (B, S, H, D), both read and written in place by the kernels.  The
+    same values as ``co_alibi_attention`` on the three transposed parts, without their copies, and
+    its gradient is one packed tensor.  The operators are ``co_alibi::fwd_qkv`` and
+    ``co_alibi::bwd_qkv``.  No counterpart in the reference, whose callers pass q, k and v apart."""
+    if qkv.dim() != 5 or qkv.shape[2] != 3:
+        raise ValueError(f"qkv must be (B, S, 3, H, D), got {tuple(qkv.shape)}")
+    if sm_scale is None:
+        sm_scale = 1.0 / (qkv.shape[-1] ** 0.5)
+    assert qkv.is_cuda, "Inputs must be CUDA tensors"
+    if qkv.dtype not in _native.DTYPE_CODES:
+        raise TypeError(f"qkv must be float32/float16/bfloat16, got {qkv.dtype}")
+    _check_head_dim(qkv.shape[4], qkv.dtype)
+    slopes = _device_slopes(qkv.shape[3], bias_max, qkv.dtype, qkv.device)
+    needs_grad = torch.is_grad_enabled() and qkv.requires_grad
+    return ops.fwd_qkv(qkv, slopes, bool(causal), float(sm_scale), needs_grad)[0]
 
 
 def co_alibi_decode(q, k_cache, v_cache, seq_len=None, sm_scale=None, bias_max=8.0, return_lse=False,

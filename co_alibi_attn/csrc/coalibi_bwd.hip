@@ -172,7 +172,9 @@ __device__ __forceinline__ void dp_tile(const f32x16& sacc, f32x16& dacc, float 
 // ---------------------------------------------------------------------------
 // Pass 1: dQ, D, and zb / cb (recompute path) or the score store (STORE).  Per wavefront 32
 // query rows; register r of lane (col, hh) <-> key k0 + hh*16 + r.
-template <typename T, int D, bool CAUSAL, bool STORE>
+// PLAIN: every operand is contiguous, and the strides are constants (with strides in registers the
+// D = 128 kernel spills four more and is 1 to 2 % slower).
+template <typename T, int D, bool CAUSAL, bool STORE, bool PLAIN>
 __global__ __launch_bounds__(256, (sizeof(T) == 4 || D > 128) ? 1 : 2) void coalibi_bwd_dq_kernel(BwdArgs args) {
   using C = BwdCfg<T, D>;
   // K / V tile row stride: 16-bit rows padded by 48 bytes (76 dwords, 12 mod 32), which reads
@@ -205,10 +207,12 @@ __global__ __launch_bounds__(256, (sizeof(T) == 4 || D > 128) ? 1 : 2) void coal
   const int qb = nQB - 1 - item.rank;  // rank 0: the longest causal rows
   const int b = bh / args.Hq, hq = bh - b * args.Hq;
   const int hkv = hq / (args.Hq / args.Hkv);
-  const size_t qoff = (size_t)bh * Sq * D;
-  const size_t kvoff = ((size_t)b * args.Hkv + hkv) * (size_t)Skv * D;
-  const T* __restrict__ Kp = static_cast<const T*>(args.k) + kvoff;
-  const T* __restrict__ Vp = static_cast<const T*>(args.v) + kvoff;
+  const Layout rows_q = contiguous_layout(args.Hq, Sq, D), rows_kv = contiguous_layout(args.Hkv, Skv, D);
+  const Layout ql = PLAIN ? rows_q : args.ql, dol = PLAIN ? rows_q : args.dol, ol = PLAIN ? rows_q : args.ol;
+  const Layout kl = PLAIN ? rows_kv : args.kl, vl = PLAIN ? rows_kv : args.vl, dql = PLAIN ? rows_q : args.dql;
+  const T* __restrict__ Kp = head_at(static_cast<const T*>(args.k), kl, b, hkv);
+  const T* __restrict__ Vp = head_at(static_cast<const T*>(args.v), vl, b, hkv);
+  const int ldk = kl.r, ldv = ldk;  // K and V share a row stride
   const float lam = args.slopes[hq];
   const float lam2 = lam * kLog2e;
   if constexpr (D < C::DP) {  // padding columns of K (read across d by the dQ product) stay zero
@@ -238,17 +242,19 @@ __global__ __launch_bounds__(256, (sizeof(T) == 4 || D > 128) ? 1 : 2) void coal
   float lse2, zhi, zlo;
   {
     const int rows = min(Sq - q0, kBM);
-    const size_t blk = qoff + (size_t)q0 * D;
-    const __amdgpu_buffer_rsrc_t qrs = tile_rsrc(static_cast<const T*>(args.q) + blk, rows * D);
-    const __amdgpu_buffer_rsrc_t dors = tile_rsrc(static_cast<const T*>(args.dout) + blk, rows * D);
-    const __amdgpu_buffer_rsrc_t ors = tile_rsrc(static_cast<const T*>(args.o) + blk, rows * D);
-    const int offb = ((wave * 32 + col) * D + hh * 8) * (int)sizeof(T);
+    auto rows_at = [&](const void* p, const Layout& l) {
+      return tile_rsrc(head_at(static_cast<const T*>(p), l, b, hq) + (size_t)q0 * l.r, row_span(rows, l.r, D));
+    };
+    const __amdgpu_buffer_rsrc_t qrs = rows_at(args.q, ql);
+    const __amdgpu_buffer_rsrc_t dors = rows_at(args.dout, dol);
+    const __amdgpu_buffer_rsrc_t ors = rows_at(args.o, ol);
+    const int r = wave * 32 + col;
 #pragma unroll
     for (int ks = 0; ks < C::KS; ++ks) {
-      const int off = offb + ks * 16 * (int)sizeof(T);
-      qf[ks] = buffer_load_vec8<vec8>(qrs, off);
-      dof[ks] = buffer_load_vec8<vec8>(dors, off);
-      of[ks] = buffer_load_vec8<vec8>(ors, off);
+      const int c = ks * 16 + hh * 8;
+      qf[ks] = buffer_load_vec8<vec8>(qrs, (r * ql.r + c) * (int)sizeof(T));
+      dof[ks] = buffer_load_vec8<vec8>(dors, (r * dol.r + c) * (int)sizeof(T));
+      of[ks] = buffer_load_vec8<vec8>(ors, (r * ol.r + c) * (int)sizeof(T));
     }
     const __amdgpu_buffer_rsrc_t lrs = tile_rsrc(args.lse + (size_t)bh * Sq + q0, rows);
     lse2 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(lrs, (wave * 32 + col) * 4, 0, 0)) * kLog2e;
@@ -267,8 +273,8 @@ __global__ __launch_bounds__(256, (sizeof(T) == 4 || D > 128) ? 1 : 2) void coal
       for (int e = 0; e < 8; ++e) dpart += dof[ks][e] * of[ks][e];
   }
   Tile kregs, vregs;
-  kregs.load(Kp, kt0 * kBN, Skv, tid);
-  vregs.load(Vp, kt0 * kBN, Skv, tid);
+  kregs.template load<!PLAIN>(Kp, kt0 * kBN, Skv, tid, ldk);
+  vregs.template load<!PLAIN>(Vp, kt0 * kBN, Skv, tid, ldv);
   if constexpr (sizeof(T) == 2) {
 #pragma unroll
     for (int ks = 0; ks < C::KS; ++ks) {
@@ -305,8 +311,8 @@ __global__ __launch_bounds__(256, (sizeof(T) == 4 || D > 128) ? 1 : 2) void coal
     vregs.store_rows(sV, LDR1, tid);
     if constexpr (!C::kTr) kregs.store_cols(sKt, C::LDT1, tid);
     lds_barrier();  // the tile is in LDS
-    kregs.load(Kp, (kt + 1) * kBN, Skv, tid);  // past the last tile: zero rows, never used
-    vregs.load(Vp, (kt + 1) * kBN, Skv, tid);
+    kregs.template load<!PLAIN>(Kp, (kt + 1) * kBN, Skv, tid, ldk);  // past the last tile: zero rows, never used
+    vregs.template load<!PLAIN>(Vp, (kt + 1) * kBN, Skv, tid, ldv);
     const int k0 = kt * kBN;
     if constexpr (decltype(tail)::value) {
       // Every key of the tile is above this wavefront's rows, and so are the later tiles'.
@@ -391,7 +397,7 @@ __global__ __launch_bounds__(256, (sizeof(T) == 4 || D > 128) ? 1 : 2) void coal
   for (int kt = kt_main; kt < nkt; ++kt) tile(kt, std::true_type{});
 
   if (row_ok) {
-    T* __restrict__ dQr = static_cast<T*>(args.dq) + qoff + (size_t)row * D;
+    T* __restrict__ dQr = head_at(static_cast<T*>(args.dq), dql, b, hq) + (size_t)row * dql.r;
     using vec4 = typename VecOf<T, 4>::type;
     const float sc = args.sm_scale;
 #pragma unroll
@@ -467,10 +473,9 @@ __global__ __launch_bounds__(256, D * sizeof(T) > 256 ? 1 : 2) void coalibi_bwd_
   if (q0 >= Sq) return;
   const int b = bh / args.Hq, hq = bh - b * args.Hq;
   const int hkv = hq / (args.Hq / args.Hkv);
-  const size_t qoff = (size_t)bh * Sq * D;
-  const size_t kvoff = ((size_t)b * args.Hkv + hkv) * (size_t)Skv * D;
-  const T* __restrict__ Kp = static_cast<const T*>(args.k) + kvoff;
-  const T* __restrict__ Vp = static_cast<const T*>(args.v) + kvoff;
+  const T* __restrict__ Kp = head_at(static_cast<const T*>(args.k), args.kl, b, hkv);
+  const T* __restrict__ Vp = head_at(static_cast<const T*>(args.v), args.vl, b, hkv);
+  const int ldk = args.kl.r, ldv = ldk;  // K and V share a row stride
   T* const sKw = sK + wave * C::K_ELEMS;  // this wavefront's tiles
   T* const sVw = sV + wave * C::V_ELEMS;
   const float lam = args.slopes[hq];
@@ -489,17 +494,19 @@ __global__ __launch_bounds__(256, D * sizeof(T) > 256 ? 1 : 2) void coalibi_bwd_
   double zsum;  // z at the next step's start
   {
     const int rows = min(Sq - q0, kSplitRows);
-    const size_t blk = qoff + (size_t)q0 * D;
-    const __amdgpu_buffer_rsrc_t qrs = tile_rsrc(static_cast<const T*>(args.q) + blk, rows * D);
-    const __amdgpu_buffer_rsrc_t dors = tile_rsrc(static_cast<const T*>(args.dout) + blk, rows * D);
-    const __amdgpu_buffer_rsrc_t ors = tile_rsrc(static_cast<const T*>(args.o) + blk, rows * D);
+    auto rows_at = [&](const void* p, const Layout& l) {
+      return tile_rsrc(head_at(static_cast<const T*>(p), l, b, hq) + (size_t)q0 * l.r, row_span(rows, l.r, D));
+    };
+    const __amdgpu_buffer_rsrc_t qrs = rows_at(args.q, args.ql);
+    const __amdgpu_buffer_rsrc_t dors = rows_at(args.dout, args.dol);
+    const __amdgpu_buffer_rsrc_t ors = rows_at(args.o, args.ol);
     vec8 of[C::KS];
 #pragma unroll
     for (int ks = 0; ks < C::KS; ++ks) {
-      const int off = (col * D + hh * 8 + ks * 16) * (int)sizeof(T);
-      qf[ks] = buffer_load_vec8<vec8>(qrs, off);
-      dof[ks] = buffer_load_vec8<vec8>(dors, off);
-      of[ks] = buffer_load_vec8<vec8>(ors, off);
+      const int c = ks * 16 + hh * 8;
+      qf[ks] = buffer_load_vec8<vec8>(qrs, (col * args.ql.r + c) * (int)sizeof(T));
+      dof[ks] = buffer_load_vec8<vec8>(dors, (col * args.dol.r + c) * (int)sizeof(T));
+      of[ks] = buffer_load_vec8<vec8>(ors, (col * args.ol.r + c) * (int)sizeof(T));
     }
     const size_t nrows = (size_t)args.B * args.Hq * Sq, at = (size_t)bh * Sq + q0;
     auto row_value = [&](const float* p) {
@@ -520,11 +527,11 @@ __global__ __launch_bounds__(256, D * sizeof(T) > 256 ? 1 : 2) void coalibi_bwd_
   // Untracked DMA: the tiles are this wavefront's own, and the waits below order it.
   typename C::KTile kdma;
   typename C::VTile vdma;
-  kdma.init(0, lane);
-  vdma.init(0, lane);
+  kdma.init(0, lane, ldk);
+  vdma.init(0, lane, ldv);
   const unsigned lds_k = lds_address(sKw), lds_v = lds_address(sVw);
-  auto issue_k = [&](int t) { kdma.issue_untracked(Kp, t < nkt ? t * kBN : 0, t < nkt ? Skv : 0, lds_k, 0); };
-  auto issue_v = [&](int t) { vdma.issue_untracked(Vp, t < nkt ? t * kBN : 0, t < nkt ? Skv : 0, lds_v, 0); };
+  auto issue_k = [&](int t) { kdma.issue_untracked(Kp, t < nkt ? t * kBN : 0, t < nkt ? Skv : 0, lds_k, 0, ldk); };
+  auto issue_v = [&](int t) { vdma.issue_untracked(Vp, t < nkt ? t * kBN : 0, t < nkt ? Skv : 0, lds_v, 0, ldv); };
   int t = kt0 + wave;
   if (steps > 0) {
     issue_v(t);
@@ -651,7 +658,7 @@ __global__ __launch_bounds__(256, D * sizeof(T) > 256 ? 1 : 2) void coalibi_bwd_
   const int r = tid >> 3;
   if (q0 + r < Sq) {
     using vec4 = typename VecOf<T, 4>::type;
-    T* __restrict__ dQr = static_cast<T*>(args.dq) + qoff + (size_t)(q0 + r) * D;
+    T* __restrict__ dQr = head_at(static_cast<T*>(args.dq), args.dql, b, hq) + (size_t)(q0 + r) * args.dql.r;
     for (int c = (tid & 7) * 4; c < D; c += 32) {
       f32x4 v = *reinterpret_cast<const f32x4*>(dq_row(0, r) + c);
 #pragma unroll
@@ -1551,7 +1558,8 @@ constexpr int kStoreBQ = 64;  // query rows per tile
 // LISTED: the key block's work items fit kStoreProcessedWords (group * query tiles, checked by
 // the launcher); they are then listed in LDS once, in walk order, each with its row block's
 // processed bit, in place of the per-head bit words and the walk in the loop.
-template <typename T, int D, bool CAUSAL, bool LISTED>
+// PLAIN: as in pass 1, every operand is contiguous.
+template <typename T, int D, bool CAUSAL, bool LISTED, bool PLAIN>
 __global__ __launch_bounds__(256, 2) void coalibi_bwd_dkdv_store_kernel(BwdArgs args) {
   static_assert(sizeof(T) == 2 && (D == 64 || D == 128), "the score store path is 16-bit, D 64 or 128");
   using C = BwdCfg<T, D>;
@@ -1588,7 +1596,6 @@ __global__ __launch_bounds__(256, 2) void coalibi_bwd_dkdv_store_kernel(BwdArgs 
   const int kb = item.rank;   // rank 0: key block 0, seen by the most query rows
   const int b = bhk / args.Hkv, hkv = bhk - b * args.Hkv;
   const int group = args.Hq / args.Hkv;
-  const size_t kvoff = (size_t)bhk * Skv * D;
   const int kwg0 = kb * kStoreBK;
   const int kw0 = kwg0 + kg * 32;  // first key of this wavefront's key group
   const int jb = kw0 / 32;
@@ -1634,19 +1641,20 @@ __global__ __launch_bounds__(256, 2) void coalibi_bwd_dkdv_store_kernel(BwdArgs 
   const int nwork = work.count();
   const int nQ32 = (Sq + 31) / 32;
 
-  Dma dma;
-  dma.init(wave, lane);
+  const Layout rows_q = contiguous_layout(args.Hq, Sq, D), rows_kv = contiguous_layout(args.Hkv, Skv, D);
+  const Layout ql = PLAIN ? rows_q : args.ql, dol = PLAIN ? rows_q : args.dol;
+  Dma qdma, dodma;
+  qdma.init(wave, lane, ql.r);
+  dodma.init(wave, lane, dol.r);
   // Loop invariants kept in scalar registers: the LDS addresses of the tile buffers, the Q / dO
   // of the group's first query head and the head stride.
   const unsigned lds_q = lds_address(sQ[0]), lds_do = lds_address(sdO[0]);
-  const size_t head0 = (size_t)(b * args.Hq + hkv * group) * Sq * D, head_stride = (size_t)Sq * D;
-  const T* __restrict__ q_g = static_cast<const T*>(args.q) + head0;
-  const T* __restrict__ do_g = static_cast<const T*>(args.dout) + head0;
+  const T* __restrict__ q_g = head_at(static_cast<const T*>(args.q), ql, b, hkv * group);
+  const T* __restrict__ do_g = head_at(static_cast<const T*>(args.dout), dol, b, hkv * group);
   auto issue_tile = [&](int gi, int qt, int buf) {
-    const size_t qoff = (size_t)gi * head_stride;
     const unsigned lbuf = (unsigned)(buf * TILE * (int)sizeof(T));
-    dma.issue_untracked(q_g + qoff, qt * BQ, Sq, lds_q + lbuf, wave);
-    dma.issue_untracked(do_g + qoff, qt * BQ, Sq, lds_do + lbuf, wave);
+    qdma.issue_untracked(q_g + (size_t)gi * ql.h, qt * BQ, Sq, lds_q + lbuf, wave, ql.r);
+    dodma.issue_untracked(do_g + (size_t)gi * dol.h, qt * BQ, Sq, lds_do + lbuf, wave, dol.r);
   };
   // A work item: query head gi, query tile qt, and whether the forward processed this key block
   // for the tile's row block.
@@ -1761,7 +1769,8 @@ __global__ __launch_bounds__(256, 2) void coalibi_bwd_dkdv_store_kernel(BwdArgs 
   const int key = kw0 + col;
   if (key < Skv) {
     using vec4 = typename VecOf<T, 4>::type;
-    T* __restrict__ out = static_cast<T*>(qh ? args.dv : args.dk) + kvoff + (size_t)key * D;
+    const Layout ol = PLAIN ? rows_kv : qh ? args.dvl : args.dkl;
+    T* __restrict__ out = head_at(static_cast<T*>(qh ? args.dv : args.dk), ol, b, hkv) + (size_t)key * ol.r;
     const float sc = qh ? 1.0f : args.sm_scale;
 #pragma unroll
     for (int i = 0; i < C::DT; ++i) {
@@ -1787,6 +1796,10 @@ hipError_t launch_bwd(const BwdArgs& a, int stages, hipStream_t stream) {
   // that have it) replaces zb / cb with the records and pass 2 with the store kernel.
   constexpr bool kStore = sizeof(T) == 2 && (D == 64 || D == 128);
   const bool store = kStore && a.scores != nullptr;
+  auto rows_q = [&](const Layout& l) { return is_contiguous(l, a.Hq, a.Sq, D); };
+  auto rows_kv = [&](const Layout& l) { return is_contiguous(l, a.Hkv, a.Skv, D); };
+  const bool plain = rows_q(a.dol) && rows_q(a.ql) && rows_q(a.ol) && rows_q(a.dql) && rows_kv(a.kl) &&
+                     rows_kv(a.vl) && rows_kv(a.dkl) && rows_kv(a.dvl);
   static_assert(kStoreBK == kOrderKeyBlock && kPairBK == kOrderKeyBlock, "key_order numbers 64-key blocks");
   if (stages & 1) {
     const int nQB = (a.Sq + kBM - 1) / kBM, blocks = nQB * a.B * a.Hq;
@@ -1802,10 +1815,14 @@ hipError_t launch_bwd(const BwdArgs& a, int stages, hipStream_t stream) {
       }
     }
     if (!split && store) {
-      if constexpr (kStore)
-        hipLaunchKernelGGL((coalibi_bwd_dq_kernel<T, D, CAUSAL, true>), dim3(blocks), dim3(256), 0, stream, a);
+      if constexpr (kStore) {
+        if (plain)
+          hipLaunchKernelGGL((coalibi_bwd_dq_kernel<T, D, CAUSAL, true, true>), dim3(blocks), dim3(256), 0, stream, a);
+        else
+          hipLaunchKernelGGL((coalibi_bwd_dq_kernel<T, D, CAUSAL, true, false>), dim3(blocks), dim3(256), 0, stream, a);
+      }
     } else if (!split) {
-      hipLaunchKernelGGL((coalibi_bwd_dq_kernel<T, D, CAUSAL, false>), dim3(blocks), dim3(256), 0, stream, a);
+      hipLaunchKernelGGL((coalibi_bwd_dq_kernel<T, D, CAUSAL, false, true>), dim3(blocks), dim3(256), 0, stream, a);
     }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -1815,12 +1832,13 @@ hipError_t launch_bwd(const BwdArgs& a, int stages, hipStream_t stream) {
       if constexpr (kStore) {
         const int nKB = (a.Skv + kStoreBK - 1) / kStoreBK;
         const int nQT = (a.Sq + kStoreBQ - 1) / kStoreBQ;
-        if (static_cast<long long>(a.Hq / a.Hkv) * nQT <= kStoreProcessedWords)
-          hipLaunchKernelGGL((coalibi_bwd_dkdv_store_kernel<T, D, CAUSAL, true>), dim3(nKB * a.B * a.Hkv), dim3(256),
-                             0, stream, a);
-        else
-          hipLaunchKernelGGL((coalibi_bwd_dkdv_store_kernel<T, D, CAUSAL, false>), dim3(nKB * a.B * a.Hkv),
-                             dim3(256), 0, stream, a);
+        const bool listed = static_cast<long long>(a.Hq / a.Hkv) * nQT <= kStoreProcessedWords;
+        auto* const kernel =
+            listed ? (plain ? coalibi_bwd_dkdv_store_kernel<T, D, CAUSAL, true, true>
+                            : coalibi_bwd_dkdv_store_kernel<T, D, CAUSAL, true, false>)
+                   : (plain ? coalibi_bwd_dkdv_store_kernel<T, D, CAUSAL, false, true>
+                            : coalibi_bwd_dkdv_store_kernel<T, D, CAUSAL, false, false>);
+        hipLaunchKernelGGL(kernel, dim3(nKB * a.B * a.Hkv), dim3(256), 0, stream, a);
       }
     } else if constexpr (sizeof(T) == 2 && D >= 64) {  // the pair kernel splits D into 32-row halves
       const int nKB = (a.Skv + kPairBK - 1) / kPairBK;

@@ -72,6 +72,29 @@ int check_shape(const char* fn, int dtype, const Shape& s) {
   return CO_ALIBI_OK;
 }
 
+// The layout of operand `name`: contiguous without strides, else the caller's batch, head and row
+// strides, which must keep every row 16-byte aligned.  A tile's byte offsets are 32-bit in the kernels
+// (at most 256 rows of 4-byte elements).
+constexpr long long kMaxRowStride = 1 << 20;
+// K and V share a row stride: the kernels keep one set of tile offsets for both.
+int check_kv_rows(const char* fn, const coalibi::Layout& k, const coalibi::Layout& v) {
+  return k.r == v.r ? CO_ALIBI_OK : fail(CO_ALIBI_EINVAL, std::string(fn) + ": k and v must have the same row stride");
+}
+int read_layout(const char* fn, const char* name, const long long* strides, int dtype, int H, int S, int D,
+                coalibi::Layout* out) {
+  *out = coalibi::contiguous_layout(H, S, D);
+  if (strides == nullptr) return CO_ALIBI_OK;
+  const long long per16 = dtype == CO_ALIBI_F32 ? 4 : 8;
+  for (int i = 0; i < 3; ++i)
+    if (strides[i] < 0 || strides[i] % per16 != 0)
+      return fail(CO_ALIBI_EINVAL, std::string(fn) + ": the strides of " + name + " must be >= 0 and whole 16-byte units");
+  if (strides[2] < D || strides[2] > kMaxRowStride)
+    return fail(CO_ALIBI_EINVAL, std::string(fn) + ": the row stride of " + name + " must be in [head_dim, " +
+                                     std::to_string(kMaxRowStride) + "]");
+  *out = {strides[0], strides[1], static_cast<int>(strides[2])};
+  return CO_ALIBI_OK;
+}
+
 // Optional outputs may be NULL; when given they must be aligned.
 int check_opt_ptr(const char* fn, const char* name, const void* p, uintptr_t align) {
   if (p != nullptr && !aligned(p, align))
@@ -164,8 +187,9 @@ namespace {
 // without them (lse = stats = NULL: no tail skip), or for inference (knorm scratch only: the
 // tail skip without the backward's statistics).  With the tail skip switched off
 // (co_alibi_set_tail_skip) no key norms are computed and every key is processed.
+// strides: of q, k, v and o (12 values), or NULL.
 int fwd_impl(const char* fn, int dtype, const void* q, const void* k, const void* v, const float* slopes, void* o,
-             float* lse, float* stats, float* knorm_ws, int batch, int heads_q, int heads_kv, int seq_q,
+             const long long* strides, float* lse, float* stats, float* knorm_ws, int batch, int heads_q, int heads_kv, int seq_q,
              int seq_kv, int head_dim, int causal, float sm_scale, void* stream) {
   const Shape s{batch, heads_q, heads_kv, seq_q, seq_kv, head_dim};
   int rc;
@@ -177,6 +201,13 @@ int fwd_impl(const char* fn, int dtype, const void* q, const void* k, const void
   if (!std::isfinite(sm_scale)) return fail(CO_ALIBI_EINVAL, std::string(fn) + ": sm_scale must be finite");
 
   coalibi::FwdArgs a{};
+  const long long* const st4[4] = {strides, strides ? strides + 3 : nullptr, strides ? strides + 6 : nullptr,
+                                   strides ? strides + 9 : nullptr};
+  if ((rc = read_layout(fn, "q", st4[0], dtype, heads_q, seq_q, head_dim, &a.ql)) ||
+      (rc = read_layout(fn, "k", st4[1], dtype, heads_kv, seq_kv, head_dim, &a.kl)) ||
+      (rc = read_layout(fn, "v", st4[2], dtype, heads_kv, seq_kv, head_dim, &a.vl)) ||
+      (rc = read_layout(fn, "o", st4[3], dtype, heads_q, seq_q, head_dim, &a.ol)) || (rc = check_kv_rows(fn, a.kl, a.vl)))
+    return rc;
   a.q = q;
   a.k = k;
   a.v = v;
@@ -226,8 +257,25 @@ extern "C" {
 int co_alibi_fwd(int dtype, const void* q, const void* k, const void* v, const float* slopes, void* o,
                  float* lse, float* stats, int batch, int heads_q, int heads_kv, int seq_q, int seq_kv,
                  int head_dim, int causal, float sm_scale, void* stream) {
-  return fwd_impl("co_alibi_fwd", dtype, q, k, v, slopes, o, lse, stats, nullptr, batch, heads_q, heads_kv, seq_q,
+  return fwd_impl("co_alibi_fwd", dtype, q, k, v, slopes, o, nullptr, lse, stats, nullptr, batch, heads_q, heads_kv, seq_q,
                   seq_kv, head_dim, causal, sm_scale, stream);
+}
+
+int co_alibi_fwd_strided(int dtype, const void* q, const void* k, const void* v, const float* slopes, void* o,
+                         const long long* strides, float* lse, float* stats, void* workspace, size_t workspace_bytes,
+                         int batch, int heads_q, int heads_kv, int seq_q, int seq_kv, int head_dim, int causal,
+                         float sm_scale, void* stream) {
+  const char* fn = "co_alibi_fwd_strided";
+  int rc;
+  if (stats == nullptr) {
+    if ((rc = check_ptr(fn, "workspace", workspace, 256))) return rc;
+    const size_t need = co_alibi_fwd_inference_workspace_bytes(batch, heads_q, seq_q, seq_kv);
+    if (workspace_bytes < need)
+      return fail(CO_ALIBI_EINVAL, std::string(fn) + ": workspace of " + std::to_string(workspace_bytes) +
+                                       " bytes, need " + std::to_string(need));
+  }
+  return fwd_impl(fn, dtype, q, k, v, slopes, o, strides, lse, stats, static_cast<float*>(workspace), batch, heads_q,
+                  heads_kv, seq_q, seq_kv, head_dim, causal, sm_scale, stream);
 }
 
 int co_alibi_fwd_inference(int dtype, const void* q, const void* k, const void* v, const float* slopes, void* o,
@@ -240,8 +288,8 @@ int co_alibi_fwd_inference(int dtype, const void* q, const void* k, const void* 
   if (workspace_bytes < need)
     return fail(CO_ALIBI_EINVAL, std::string(fn) + ": workspace of " + std::to_string(workspace_bytes) +
                                      " bytes, need " + std::to_string(need));
-  return fwd_impl(fn, dtype, q, k, v, slopes, o, nullptr, nullptr, static_cast<float*>(workspace), batch, heads_q,
-                  heads_kv, seq_q, seq_kv, head_dim, causal, sm_scale, stream);
+  return fwd_impl(fn, dtype, q, k, v, slopes, o, nullptr, nullptr, nullptr, static_cast<float*>(workspace), batch,
+                  heads_q, heads_kv, seq_q, seq_kv, head_dim, causal, sm_scale, stream);
 }
 
 }  // extern "C"
@@ -249,7 +297,8 @@ int co_alibi_fwd_inference(int dtype, const void* q, const void* k, const void* 
 namespace {
 
 // stages: 1 = pass 1 (dq, dsum, and zb / cb or the score store), 2 = pass 2 (dk, dv), 3 = both.
-int bwd_impl(const char* fn, int stages, int dtype, const void* dout, const void* q, const void* k,
+// strides: of dout, q, k, v, o, dq, dk and dv (24 values; score-store path only), or NULL.
+int bwd_impl(const char* fn, int stages, const long long* strides, int dtype, const void* dout, const void* q, const void* k,
              const void* v, const void* o, const float* lse, const float* stats, const float* slopes, void* dq,
              void* dk, void* dv, void* workspace, size_t workspace_bytes, int batch, int heads_q,
              int heads_kv, int seq_q, int seq_kv, int head_dim, int causal, float sm_scale, void* stream) {
@@ -268,6 +317,9 @@ int bwd_impl(const char* fn, int stages, int dtype, const void* dout, const void
       co_alibi_bwd_score_store_workspace_bytes(dtype, batch, heads_q, heads_kv, seq_q, seq_kv, head_dim, causal);
   const bool store = need_store != 0 && workspace_bytes >= need_store;
   const size_t need = co_alibi_bwd_workspace_bytes(batch, heads_q, seq_q, seq_kv);
+  if (!store && strides != nullptr)
+    return fail(CO_ALIBI_EINVAL, std::string(fn) + ": strided operands need the score store (a workspace of " +
+                                     std::to_string(need_store) + " bytes; 0: no such path)");
   if (!store && workspace_bytes < need)
     return fail(CO_ALIBI_EINVAL, std::string(fn) + ": workspace of " + std::to_string(workspace_bytes) +
                                      " bytes, need " + std::to_string(need));
@@ -275,6 +327,15 @@ int bwd_impl(const char* fn, int stages, int dtype, const void* dout, const void
 
   const size_t rows = static_cast<size_t>(batch) * heads_q * seq_q;
   coalibi::BwdArgs a{};
+  coalibi::Layout* const layouts[8] = {&a.dol, &a.ql, &a.kl, &a.vl, &a.ol, &a.dql, &a.dkl, &a.dvl};
+  const char* const names[8] = {"dout", "q", "k", "v", "o", "dq", "dk", "dv"};
+  for (int i = 0; i < 8; ++i) {
+    const bool kv = i == 2 || i == 3 || i >= 6;
+    if ((rc = read_layout(fn, names[i], strides ? strides + 3 * i : nullptr, dtype, kv ? heads_kv : heads_q,
+                          kv ? seq_kv : seq_q, head_dim, layouts[i])))
+      return rc;
+  }
+  if ((rc = check_kv_rows(fn, a.kl, a.vl))) return rc;
   a.dout = dout;
   a.q = q;
   a.k = k;
@@ -332,15 +393,24 @@ int co_alibi_bwd(int dtype, const void* dout, const void* q, const void* k, cons
                  const float* lse, const float* stats, const float* slopes, void* dq, void* dk, void* dv,
                  void* workspace, size_t workspace_bytes, int batch, int heads_q, int heads_kv, int seq_q,
                  int seq_kv, int head_dim, int causal, float sm_scale, void* stream) {
-  return bwd_impl("co_alibi_bwd", 3, dtype, dout, q, k, v, o, lse, stats, slopes, dq, dk, dv, workspace,
+  return bwd_impl("co_alibi_bwd", 3, nullptr, dtype, dout, q, k, v, o, lse, stats, slopes, dq, dk, dv, workspace,
                   workspace_bytes, batch, heads_q, heads_kv, seq_q, seq_kv, head_dim, causal, sm_scale, stream);
+}
+
+int co_alibi_bwd_strided(int dtype, const void* dout, const void* q, const void* k, const void* v, const void* o,
+                         const float* lse, const float* stats, const float* slopes, void* dq, void* dk, void* dv,
+                         const long long* strides, void* workspace, size_t workspace_bytes, int batch, int heads_q,
+                         int heads_kv, int seq_q, int seq_kv, int head_dim, int causal, float sm_scale, void* stream) {
+  return bwd_impl("co_alibi_bwd_strided", 3, strides, dtype, dout, q, k, v, o, lse, stats, slopes, dq, dk, dv,
+                  workspace, workspace_bytes, batch, heads_q, heads_kv, seq_q, seq_kv, head_dim, causal, sm_scale,
+                  stream);
 }
 
 int co_alibi_bwd_dq(int dtype, const void* dout, const void* q, const void* k, const void* v, const void* o,
                     const float* lse, const float* stats, const float* slopes, void* dq, void* workspace,
                     size_t workspace_bytes, int batch, int heads_q, int heads_kv, int seq_q, int seq_kv,
                     int head_dim, int causal, float sm_scale, void* stream) {
-  return bwd_impl("co_alibi_bwd_dq", 1, dtype, dout, q, k, v, o, lse, stats, slopes, dq, nullptr, nullptr,
+  return bwd_impl("co_alibi_bwd_dq", 1, nullptr, dtype, dout, q, k, v, o, lse, stats, slopes, dq, nullptr, nullptr,
                   workspace, workspace_bytes, batch, heads_q, heads_kv, seq_q, seq_kv, head_dim, causal,
                   sm_scale, stream);
 }
@@ -349,7 +419,7 @@ int co_alibi_bwd_dkdv(int dtype, const void* dout, const void* q, const void* k,
                       const float* lse, const float* stats, const float* slopes, void* dk, void* dv,
                       void* workspace, size_t workspace_bytes, int batch, int heads_q, int heads_kv,
                       int seq_q, int seq_kv, int head_dim, int causal, float sm_scale, void* stream) {
-  return bwd_impl("co_alibi_bwd_dkdv", 2, dtype, dout, q, k, v, nullptr, lse, stats, slopes, nullptr, dk, dv,
+  return bwd_impl("co_alibi_bwd_dkdv", 2, nullptr, dtype, dout, q, k, v, nullptr, lse, stats, slopes, nullptr, dk, dv,
                   workspace, workspace_bytes, batch, heads_q, heads_kv, seq_q, seq_kv, head_dim, causal,
                   sm_scale, stream);
 }

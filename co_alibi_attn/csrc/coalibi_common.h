@@ -18,6 +18,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "coalibi_kernels.h"
+
 namespace coalibi {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -101,6 +103,14 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const T* p, int elem
   void* base = reinterpret_cast<void*>((static_cast<unsigned long long>(hi) << 32) | lo);
   return __builtin_amdgcn_make_buffer_rsrc(base, (short)0, bytes, kBufferRsrcWord3);
 }
+
+// Head (b, h) of an operand, and the elements from the first to past the last of `rows` of its rows (a
+// buffer resource of that size reads rows from `rows` on as zero, since their offsets are >= rows * ld).
+template <typename T>
+__device__ __forceinline__ T* head_at(T* p, const Layout& l, int b, int h) {
+  return p + ((size_t)b * l.b + (size_t)h * l.h);
+}
+__device__ __forceinline__ int row_span(int rows, int ld, int D) { return rows > 0 ? (rows - 1) * ld + D : 0; }
 
 // Eight consecutive elements at byte offset `off` of a buffer resource (zero past its end):
 // one 16-byte load for 16-bit types, two for fp32.  No branch, so a run of these loads goes
@@ -298,13 +308,14 @@ struct DmaTile {
   static_assert(!PERM || ROWS % 32 == 0, "rows are permuted in blocks of 32");
   int off[SLOTS];
 
-  __device__ __forceinline__ void init(int wave, int lane) {
+  // ld: the matrix's row stride.
+  __device__ __forceinline__ void init(int wave, int lane, int ld = D) {
 #pragma unroll
     for (int m = 0; m < SLOTS; ++m) {
       const int c = (wave + NWAVES * m) * 64 + lane;
       const int r = c / CPR, j = c - r * CPR;
       const int src = PERM ? (r & ~31) + kRowOfReg(r & 31) : r;
-      off[m] = j < D / CH ? (src * D + j * CH) * (int)sizeof(T) : 0x40000000;
+      off[m] = j < D / CH ? (src * ld + j * CH) * (int)sizeof(T) : 0x40000000;
     }
   }
   __device__ __forceinline__ void issue(const T* base, int row0, int nrows, T* lds, int wave) const {
@@ -318,9 +329,10 @@ struct DmaTile {
   // The same through dma16_to_lds_untracked (its rules apply), into the tile at LDS byte
   // address lds_byte (lds_address).  wave < NWAVES, so only the last slot can lie past the
   // tile's instructions.
-  __device__ __forceinline__ void issue_untracked(const T* base, int row0, int nrows, unsigned lds_byte,
-                                                  int wave) const {
-    const __amdgpu_buffer_rsrc_t rsrc = tile_rsrc(base + (size_t)row0 * D, min(max(nrows - row0, 0), ROWS) * D);
+  __device__ __forceinline__ void issue_untracked(const T* base, int row0, int nrows, unsigned lds_byte, int wave,
+                                                  int ld = D) const {
+    const __amdgpu_buffer_rsrc_t rsrc =
+        tile_rsrc(base + (size_t)row0 * ld, row_span(min(max(nrows - row0, 0), ROWS), ld, D));
 #pragma unroll
     for (int m = 0; m < SLOTS; ++m) {
       const int i = wave + NWAVES * m;
@@ -366,16 +378,28 @@ struct TileLoader {
   // Rows row0 .. row0+ROWS-1 of a row-major [nrows][D] array; rows >= nrows read as zero.
   // Buffer loads: the resource covers exactly the tile's valid rows, so the hardware range
   // check zero-fills the rest; per-lane offsets are tile-invariant and the base is uniform.
-  __device__ __forceinline__ void load(const T* __restrict__ base, int row0, int nrows, int tid) {
-    const __amdgpu_buffer_rsrc_t rsrc = tile_rsrc(base + (size_t)row0 * D, min(max(nrows - row0, 0), ROWS) * D);
+  // STRIDED: the array's rows are ld elements apart.
+  template <bool STRIDED = false>
+  __device__ __forceinline__ void load(const T* __restrict__ base, int row0, int nrows, int tid, int ld = D) {
+    if constexpr (!STRIDED) ld = D;
+    const __amdgpu_buffer_rsrc_t rsrc =
+        tile_rsrc(base + (size_t)row0 * ld, row_span(min(max(nrows - row0, 0), ROWS), ld, D));
 #pragma unroll
     for (int i = 0; i < GPT; ++i) {
       const int g = tid + 256 * i;
       if (kPartial && g >= NG) continue;
       const int rr = grp_row(g), cc = grp_col(g);
+      if constexpr (STRIDED && !GROUPED) {
+        // Group i lies i * 256 / CPR rows below group 0: an addition per load (of a step the compiler
+        // cannot see through) in place of an offset register per group across the caller's loop.
+        int step = i * (256 / CPR) * ld * (int)sizeof(T);
+        if (i > 0) asm volatile("" : "+s"(step));
+        r[i][0] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (grp_row(tid) * ld + cc) * (int)sizeof(T) + step, 0, 0);
+      } else {
 #pragma unroll
-      for (int k = 0; k < KG; ++k)
-        r[i][k] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, ((rr + k) * D + cc) * (int)sizeof(T), 0, 0);
+        for (int k = 0; k < KG; ++k)
+          r[i][k] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, ((rr + k) * ld + cc) * (int)sizeof(T), 0, 0);
+      }
     }
   }
 

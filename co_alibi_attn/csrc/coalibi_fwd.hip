@@ -351,9 +351,9 @@ __device__ void schedule_orders(const ScheduleArgs& s, int which, int tid) {
 // non-finite key disables the skip for its head.
 // The first nSched work-groups of the launch write the work orders instead.
 template <typename T, int D>
-__global__ __launch_bounds__(256) void coalibi_key_norm_kernel(const T* __restrict__ k, float* __restrict__ knorm,
-                                                               int Skv, int nKC, int nKeyHeads, int nSched,
-                                                               ScheduleArgs sched) {
+__global__ __launch_bounds__(256) void coalibi_key_norm_kernel(const T* __restrict__ k, Layout kl,
+                                                               float* __restrict__ knorm, int Skv, int nKC,
+                                                               int nKeyHeads, int nSched, ScheduleArgs sched) {
   constexpr int CH = 16 / (int)sizeof(T);  // elements per 16-byte chunk
   constexpr int CPR = D / CH;              // chunks (lanes) per key row: 2 .. 32
   constexpr int RPP = 256 / CPR;           // key rows per pass of the work-group
@@ -373,11 +373,12 @@ __global__ __launch_bounds__(256) void coalibi_key_norm_kernel(const T* __restri
   // chunk's valid rows (rows past Skv read as zero, whose norm 0 leaves the maximum alone).
   constexpr int NP = kNormKeys / RPP;  // passes over the chunk
   const int r0 = c * kNormKeys;
-  const __amdgpu_buffer_rsrc_t rs = tile_rsrc(k + ((size_t)bhk * Skv + r0) * D, min(kNormKeys, Skv - r0) * D);
+  const __amdgpu_buffer_rsrc_t rs = tile_rsrc(
+      head_at(k, kl, bhk / sched.Hkv, bhk % sched.Hkv) + (size_t)r0 * kl.r, row_span(min(kNormKeys, Skv - r0), kl.r, D));
   u32x4 x[NP];
 #pragma unroll
   for (int p = 0; p < NP; ++p)
-    x[p] = __builtin_amdgcn_raw_buffer_load_b128(rs, ((p * RPP + tid / CPR) * D + (tid % CPR) * CH) * (int)sizeof(T),
+    x[p] = __builtin_amdgcn_raw_buffer_load_b128(rs, ((p * RPP + tid / CPR) * kl.r + (tid % CPR) * CH) * (int)sizeof(T),
                                                  0, 0);
   float best = 0.f;
 #pragma unroll
@@ -408,8 +409,9 @@ __global__ __launch_bounds__(256) void coalibi_key_norm_kernel(const T* __restri
 
 // One 128-row block (bh, qb) by a work-group of 4 wavefronts, 32 rows each, over tiles in sK and sV.
 // SKIP: the tail skip (args.knorm holds the key norms); without it every key is processed and
-// the code carries none of the skip's per-tile test.
-template <typename T, int D, bool CAUSAL, bool SKIP>
+// the code carries none of the skip's per-tile test.  PLAIN: every operand is contiguous, and the
+// strides are constants (in registers they cost the grouped-query forward 1.7 %, n 8192 bf16).
+template <typename T, int D, bool CAUSAL, bool SKIP, bool PLAIN>
 __device__ __forceinline__ void fwd_row_block(const FwdArgs& args, int bh, int qb, T* __restrict__ sK,
                                               T* __restrict__ sV) {
   using C = FwdCfg<T, D>;
@@ -424,10 +426,13 @@ __device__ __forceinline__ void fwd_row_block(const FwdArgs& args, int bh, int q
   const int nQB = (Sq + kFwdBM - 1) / kFwdBM;
   const int b = bh / args.Hq, hq = bh - b * args.Hq;
   const int hkv = hq / (args.Hq / args.Hkv);
-  const T* __restrict__ Qp = static_cast<const T*>(args.q) + (size_t)bh * Sq * D;
-  const size_t kvoff = ((size_t)b * args.Hkv + hkv) * (size_t)Skv * D;
-  const T* __restrict__ Kp = static_cast<const T*>(args.k) + kvoff;
-  const T* __restrict__ Vp = static_cast<const T*>(args.v) + kvoff;
+  const Layout rows_q = contiguous_layout(args.Hq, Sq, D), rows_kv = contiguous_layout(args.Hkv, Skv, D);
+  const Layout ql = PLAIN ? rows_q : args.ql, ol = PLAIN ? rows_q : args.ol;
+  const Layout kl = PLAIN ? rows_kv : args.kl, vl = PLAIN ? rows_kv : args.vl;
+  const T* __restrict__ Qp = head_at(static_cast<const T*>(args.q), ql, b, hq);
+  const T* __restrict__ Kp = head_at(static_cast<const T*>(args.k), kl, b, hkv);
+  const T* __restrict__ Vp = head_at(static_cast<const T*>(args.v), vl, b, hkv);
+  const int ldk = kl.r, ldv = ldk;  // K and V share a row stride
   const float lam2 = args.slopes[hq] * kLog2e;
   const float sc2 = args.sc2;
   if constexpr (D < C::DP) {  // the padding columns of V stay zero: tiles only write the D real ones
@@ -447,8 +452,8 @@ __device__ __forceinline__ void fwd_row_block(const FwdArgs& args, int bh, int q
   // Q through a buffer resource over the block's valid rows: rows past Sq read as zero.
   vec8 qf[C::KS];
   {
-    const __amdgpu_buffer_rsrc_t qrs = tile_rsrc(Qp + (size_t)q0 * D, min(Sq - q0, kFwdBM) * D);
-    const int qoffb = ((wave * 32 + col) * D + hh * 8) * (int)sizeof(T);
+    const __amdgpu_buffer_rsrc_t qrs = tile_rsrc(Qp + (size_t)q0 * ql.r, row_span(min(Sq - q0, kFwdBM), ql.r, D));
+    const int qoffb = ((wave * 32 + col) * ql.r + hh * 8) * (int)sizeof(T);
 #pragma unroll
     for (int ks = 0; ks < C::KS; ++ks) qf[ks] = buffer_load_vec8<vec8>(qrs, qoffb + ks * 16 * (int)sizeof(T));
   }
@@ -456,8 +461,8 @@ __device__ __forceinline__ void fwd_row_block(const FwdArgs& args, int bh, int q
   const int nkt = last_key / kFwdBN + 1;
   KTile kt_regs;
   VTile vt_regs;
-  kt_regs.load(Kp, (nkt - 1) * kFwdBN, Skv, tid);
-  vt_regs.load(Vp, (nkt - 1) * kFwdBN, Skv, tid);
+  kt_regs.template load<!PLAIN>(Kp, (nkt - 1) * kFwdBN, Skv, tid, ldk);
+  vt_regs.template load<!PLAIN>(Vp, (nkt - 1) * kFwdBN, Skv, tid, ldv);
   const bool tail_skip = SKIP && lam2 > 0.f;
   float km = 0.f;
   if (tail_skip) {
@@ -529,15 +534,15 @@ __device__ __forceinline__ void fwd_row_block(const FwdArgs& args, int bh, int q
     // registers do not fit beside the tile state, and the loads are issued after it.
     constexpr bool kPrefetchKV = D <= 128;
     if (kPrefetchKV && kt > 0) {
-      kt_regs.load(Kp, (kt - 1) * kFwdBN, Skv, tid);
-      vt_regs.load(Vp, (kt - 1) * kFwdBN, Skv, tid);
+      kt_regs.template load<!PLAIN>(Kp, (kt - 1) * kFwdBN, Skv, tid, ldk);
+      vt_regs.template load<!PLAIN>(Vp, (kt - 1) * kFwdBN, Skv, tid, ldv);
     }
     const int k0 = kt * kFwdBN;
     const bool skip = CAUSAL && k0 > wrow0 + 31;  // every key of the tile is above this wavefront's rows
     if (skip) {
       if (!kPrefetchKV && kt > 0) {
-        kt_regs.load(Kp, (kt - 1) * kFwdBN, Skv, tid);
-        vt_regs.load(Vp, (kt - 1) * kFwdBN, Skv, tid);
+        kt_regs.template load<!PLAIN>(Kp, (kt - 1) * kFwdBN, Skv, tid, ldk);
+        vt_regs.template load<!PLAIN>(Vp, (kt - 1) * kFwdBN, Skv, tid, ldv);
       }
       if (tail_skip && lane == 0) sDone[wave] = Sq <= wrow0;  // no visible key yet: only rows past Sq pass
       continue;
@@ -552,8 +557,8 @@ __device__ __forceinline__ void fwd_row_block(const FwdArgs& args, int bh, int q
     zsum += (double)btot[0];
     zr = (float)zsum;
     if (!kPrefetchKV && kt > 0) {
-      kt_regs.load(Kp, (kt - 1) * kFwdBN, Skv, tid);
-      vt_regs.load(Vp, (kt - 1) * kFwdBN, Skv, tid);
+      kt_regs.template load<!PLAIN>(Kp, (kt - 1) * kFwdBN, Skv, tid, ldk);
+      vt_regs.template load<!PLAIN>(Vp, (kt - 1) * kFwdBN, Skv, tid, ldv);
     }
     if (tail_skip) {
       // Every key left of k0 has z >= zr, so its weight is at most 2^(bound - lam2*zr - m2).
@@ -571,7 +576,7 @@ __device__ __forceinline__ void fwd_row_block(const FwdArgs& args, int bh, int q
   const float ltot = lsum + other_half(lsum);
   const float inv = ltot > 0.f ? 1.0f / ltot : 0.f;
   if (row_ok) {
-    T* __restrict__ Orow = static_cast<T*>(args.o) + ((size_t)bh * Sq + row) * D;
+    T* __restrict__ Orow = head_at(static_cast<T*>(args.o), ol, b, hq) + (size_t)row * ol.r;
     using vec4 = typename VecOf<T, 4>::type;
 #pragma unroll
     for (int dt = 0; dt < C::DT; ++dt) {
@@ -593,7 +598,7 @@ __device__ __forceinline__ void fwd_row_block(const FwdArgs& args, int bh, int q
   }
 }
 
-template <typename T, int D, bool CAUSAL, bool SKIP>
+template <typename T, int D, bool CAUSAL, bool SKIP, bool PLAIN>
 __global__ __launch_bounds__(256, (sizeof(T) == 4 || D > 128) ? 1 : 2) void coalibi_fwd_kernel(FwdArgs args) {
   using C = FwdCfg<T, D>;
   __shared__ __align__(16) T sK[kFwdBN * C::LDK];
@@ -602,7 +607,7 @@ __global__ __launch_bounds__(256, (sizeof(T) == 4 || D > 128) ? 1 : 2) void coal
   const WorkItem item = args.row_order ? table_item(args.row_order, blockIdx.x, args.B * args.Hq, gridDim.x)
                                        : lpt_item(blockIdx.x, args.B * args.Hq, 1);
   // rank 0: the longest causal rows
-  fwd_row_block<T, D, CAUSAL, SKIP>(args, item.head, nQB - 1 - item.rank, sK, sV);
+  fwd_row_block<T, D, CAUSAL, SKIP, PLAIN>(args, item.head, nQB - 1 - item.rank, sK, sV);
 }
 
 // ---------------------------------------------------------------------------
@@ -668,9 +673,9 @@ __device__ __forceinline__ void fwd_split_rows(const FwdArgs& args, int bh, int 
   const int Sq = args.Sq, Skv = args.Skv;
   const int b = bh / args.Hq, hq = bh - b * args.Hq;
   const int hkv = hq / (args.Hq / args.Hkv);
-  const size_t kvoff = ((size_t)b * args.Hkv + hkv) * (size_t)Skv * D;
-  const T* __restrict__ Kp = static_cast<const T*>(args.k) + kvoff;
-  const T* __restrict__ Vp = static_cast<const T*>(args.v) + kvoff;
+  const T* __restrict__ Kp = head_at(static_cast<const T*>(args.k), args.kl, b, hkv);
+  const T* __restrict__ Vp = head_at(static_cast<const T*>(args.v), args.vl, b, hkv);
+  const int ldq = args.ql.r, ldk = args.kl.r, ldv = ldk;
   T* const sKw = sK + wave * C::K_ELEMS;  // this wavefront's tiles
   T* const sVw = sV + wave * C::V_ELEMS;
   const float lam2 = args.slopes[hq] * kLog2e;
@@ -683,18 +688,19 @@ __device__ __forceinline__ void fwd_split_rows(const FwdArgs& args, int bh, int 
   // Untracked DMA: the tiles are this wavefront's own, and the waits below order it.
   typename C::KTile kdma;
   typename C::VTile vdma;
-  kdma.init(0, lane);
-  vdma.init(0, lane);
+  kdma.init(0, lane, ldk);
+  vdma.init(0, lane, ldv);
   const unsigned lds_k = lds_address(sKw), lds_v = lds_address(sVw);
-  auto issue_k = [&](int tt) { kdma.issue_untracked(Kp, max(tt, 0) * kWaveKeys, tt < 0 ? 0 : Skv, lds_k, 0); };
-  auto issue_v = [&](int tt) { vdma.issue_untracked(Vp, max(tt, 0) * kWaveKeys, tt < 0 ? 0 : Skv, lds_v, 0); };
+  auto issue_k = [&](int tt) { kdma.issue_untracked(Kp, max(tt, 0) * kWaveKeys, tt < 0 ? 0 : Skv, lds_k, 0, ldk); };
+  auto issue_v = [&](int tt) { vdma.issue_untracked(Vp, max(tt, 0) * kWaveKeys, tt < 0 ? 0 : Skv, lds_v, 0, ldv); };
   vec8 qf[C::KS];
   {
     const __amdgpu_buffer_rsrc_t qrs =
-        tile_rsrc(static_cast<const T*>(args.q) + ((size_t)bh * Sq + q0) * D, min(Sq - q0, kSplitRows) * D);
+        tile_rsrc(head_at(static_cast<const T*>(args.q), args.ql, b, hq) + (size_t)q0 * ldq,
+                  row_span(min(Sq - q0, kSplitRows), ldq, D));
 #pragma unroll
     for (int ks = 0; ks < C::KS; ++ks)
-      qf[ks] = buffer_load_vec8<vec8>(qrs, (col * D + ks * 16 + hh * 8) * (int)sizeof(T));
+      qf[ks] = buffer_load_vec8<vec8>(qrs, (col * ldq + ks * 16 + hh * 8) * (int)sizeof(T));
   }
   issue_k(t);
   issue_v(t);
@@ -834,7 +840,7 @@ __device__ __forceinline__ void fwd_split_rows(const FwdArgs& args, int bh, int 
   const int r = tid >> 3;
   if (q0 + r < Sq) {
     using vec4 = typename VecOf<T, 4>::type;
-    T* __restrict__ Orow = static_cast<T*>(args.o) + ((size_t)bh * Sq + q0 + r) * D;
+    T* __restrict__ Orow = head_at(static_cast<T*>(args.o), args.ol, b, hq) + (size_t)(q0 + r) * args.ol.r;
     const float inv = sInv[r];
 #pragma unroll
     for (int c = (tid & 7) * 4; c < D; c += 32) {
@@ -870,7 +876,7 @@ __global__ __launch_bounds__(256, D * sizeof(T) > 256 ? 1 : 2) void coalibi_fwd_
     if (part == 0 && args.kstart != nullptr && threadIdx.x == 0) args.kstart[(size_t)item.head * nQB + qb] = 0;
     if (q0 + part * kSplitRows < args.Sq) fwd_split_rows<T, D, CAUSAL>(args, item.head, q0 + part * kSplitRows, sK, sV);
   } else if (part == 0) {
-    fwd_row_block<T, D, CAUSAL, SKIP>(args, item.head, qb, sK, sV);
+    fwd_row_block<T, D, CAUSAL, SKIP, false>(args, item.head, qb, sK, sV);
   }
 }
 
@@ -906,7 +912,7 @@ hipError_t launch_fwd(const FwdArgs& a, hipStream_t stream) {
     // The key table needs the row table's work-group before it (work-group 1 writes it).
     const int nSched = a.row_order == nullptr ? 0 : (a.key_order != nullptr ? 2 : 1);
     hipLaunchKernelGGL((coalibi_key_norm_kernel<T, D>), dim3(nSched + a.nKC * a.B * a.Hq), dim3(256), 0, stream,
-                       static_cast<const T*>(a.k), const_cast<float*>(a.knorm), a.Skv, a.nKC, a.B * a.Hkv, nSched,
+                       static_cast<const T*>(a.k), a.kl, const_cast<float*>(a.knorm), a.Skv, a.nKC, a.B * a.Hkv, nSched,
                        sched);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -932,10 +938,14 @@ hipError_t launch_fwd(const FwdArgs& a, hipStream_t stream) {
       return hipGetLastError();
     }
   }
-  if (a.knorm != nullptr)
-    hipLaunchKernelGGL((coalibi_fwd_kernel<T, D, CAUSAL, true>), dim3(grid), dim3(256), 0, stream, f);
-  else
-    hipLaunchKernelGGL((coalibi_fwd_kernel<T, D, CAUSAL, false>), dim3(grid), dim3(256), 0, stream, f);
+  const bool plain = is_contiguous(a.ql, a.Hq, a.Sq, D) && is_contiguous(a.ol, a.Hq, a.Sq, D) &&
+                     is_contiguous(a.kl, a.Hkv, a.Skv, D) && is_contiguous(a.vl, a.Hkv, a.Skv, D);
+  auto* const kernel = a.knorm != nullptr
+                           ? (plain ? coalibi_fwd_kernel<T, D, CAUSAL, true, true>
+                                    : coalibi_fwd_kernel<T, D, CAUSAL, true, false>)
+                           : (plain ? coalibi_fwd_kernel<T, D, CAUSAL, false, true>
+                                    : coalibi_fwd_kernel<T, D, CAUSAL, false, false>);
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, stream, f);
   return hipGetLastError();
 }
 

@@ -99,7 +99,22 @@ template <typename T>
 constexpr float order_window() {
   return (skip_log2<T>() + 8.0f) / (0.5f * kLog2eHost);
 }
+// Element strides of one (B, H, S, D) operand: from batch to batch, head to head and row to row.  The
+// D elements of a row are consecutive; r >= D.  A model's projections leave (B, S, H, D) memory, whose
+// transposed views the kernels read and write in place this way.
+struct Layout {
+  long long b, h;
+  int r;
+};
+__host__ __device__ inline Layout contiguous_layout(int H, int S, int D) {
+  return {static_cast<long long>(H) * S * D, static_cast<long long>(S) * D, D};
+}
+inline bool is_contiguous(const Layout& l, int H, int S, int D) {
+  const Layout c = contiguous_layout(H, S, D);
+  return l.b == c.b && l.h == c.h && l.r == c.r;
+}
 struct FwdArgs {
+  Layout ql, kl, vl, ol;
   const void* q;
   const void* k;
   const void* v;
@@ -153,6 +168,8 @@ inline size_t score_records_per_head(int Sq, int Skv, bool causal) {
 // dA_ik over the keys k < 32J, written by pass 1 for the blocks it processes.  The score-store
 // path needs neither.
 struct BwdArgs {
+  // Other than contiguous layouts on the score-store path only.
+  Layout dol, ql, kl, vl, ol, dql, dkl, dvl;
   const void* dout;
   const void* q;
   const void* k;

@@ -23,7 +23,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from .co_alibi_attn import co_alibi_attention
+from .co_alibi_attn import co_alibi_attention, co_alibi_attention_qkv
 
 
 @dataclass(frozen=True)
@@ -52,6 +52,10 @@ class CausalCoALiBiAttention(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         B, S, C = x.shape
         qkv = self.qkv(x).view(B, S, 3, self.n_head, self.head_dim)
+        if self.attention is co_alibi_attention and qkv.is_cuda:
+            # The same attention on the packed projection: no copies of its parts, and one packed
+            # gradient in place of three that autograd would zero-fill and add.
+            return self.proj(co_alibi_attention_qkv(qkv, causal=True, bias_max=self.bias_max).reshape(B, S, C))
         q, k, v = (qkv[:, :, i].transpose(1, 2) for i in range(3))  # (B, H, S, D) views
         y = self.attention(q, k, v, causal=True, bias_max=self.bias_max)
         return self.proj(y.transpose(1, 2).reshape(B, S, C))

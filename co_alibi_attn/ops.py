@@ -1,5 +1,5 @@
 """PyTorch operators over the native library: ``co_alibi::fwd``, ``co_alibi::bwd``, ``co_alibi::bwd_dq``,
-``co_alibi::decode``.
+``co_alibi::fwd_qkv``, ``co_alibi::bwd_qkv``, ``co_alibi::decode``.
 
 The operators are defined in C++ (``csrc/torch_ops.cpp``, built into
 ``_lib/libco_alibi_torch.so`` and loaded here): each one is one C-ABI launch
@@ -18,8 +18,11 @@ They replace the reference's two Triton launches with their buffer set-up:
 dK / dV partial buffers and their reduction (:83-133).  ``co_alibi::decode`` has no
 counterpart in the reference (its forward with Sq = 1 over a cache).
 
-Operands are (B, H, S, D) tensors as in include/co_alibi.h; the operators make them
-contiguous and 16-byte aligned (a copy only when they are not).  Argument checking with
+Operands are (B, H, S, D) tensors as in include/co_alibi.h.  The forward, and the backward on
+its score-store path, read them in place in any layout whose rows are consecutive and 16-byte
+aligned (transposed views of (B, S, H, D) memory, parts of a packed QKV tensor); others, and the
+recompute path's, are copied.  ``fwd_qkv`` / ``bwd_qkv`` are the packed form: one (B, S, 3, H, D)
+tensor in, (B, S, H, D) out, one packed gradient.  Argument checking with
 the reference's error types happens in the public functions of co_alibi_attn.py.
 """
 import os
@@ -29,7 +32,7 @@ from torch import Tensor
 
 from . import _native
 
-__all__ = ["fwd", "bwd", "bwd_dq", "backward_for", "decode", "stats_numel", "TORCH_LIB_PATH"]
+__all__ = ["fwd", "bwd", "bwd_dq", "fwd_qkv", "bwd_qkv", "backward_for", "decode", "stats_numel", "TORCH_LIB_PATH"]
 
 TORCH_LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib", "libco_alibi_torch.so")
 
@@ -68,9 +71,11 @@ if _MISSING is None:
     fwd = torch.ops.co_alibi.fwd
     bwd = torch.ops.co_alibi.bwd
     bwd_dq = torch.ops.co_alibi.bwd_dq
+    fwd_qkv = torch.ops.co_alibi.fwd_qkv
+    bwd_qkv = torch.ops.co_alibi.bwd_qkv
     decode = torch.ops.co_alibi.decode
 else:
-    fwd = bwd = bwd_dq = decode = _unavailable
+    fwd = bwd = bwd_dq = fwd_qkv = bwd_qkv = decode = _unavailable
 
 
 def stats_numel(batch: int, heads_q: int, seq_q: int, seq_kv: int) -> int:
@@ -103,7 +108,7 @@ def backward_for(needs_input_grad, do, q, k, v, o, lse, stats, slopes, causal, s
 
 
 def _register_fakes() -> None:
-    """Shape functions of the four operators (FakeTensor / meta tracing, torch.compile)."""
+    """Shape functions of the operators (FakeTensor / meta tracing, torch.compile)."""
 
     @torch.library.register_fake("co_alibi::fwd")
     def _fwd_fake(q, k, v, slopes, causal, sm_scale, with_stats):
@@ -129,6 +134,21 @@ def _register_fakes() -> None:
     def _bwd_dq_fake(do, q, k, v, o, lse, stats, slopes, causal, sm_scale):
         """dq alone (backward pass 1), bit-identical to co_alibi::bwd's dq."""
         return torch.empty_like(q, memory_format=torch.contiguous_format)
+
+    @torch.library.register_fake("co_alibi::fwd_qkv")
+    def _fwd_qkv_fake(qkv, slopes, causal, sm_scale, with_stats):
+        """qkv (B, S, 3, H, D); o (B, S, H, D), and lse and stats as co_alibi::fwd's."""
+        batch, seq, _, heads, head_dim = qkv.shape
+        o = qkv.new_empty((batch, seq, heads, head_dim))
+        if not with_stats:
+            return o, _empty_stats(qkv), _empty_stats(qkv)
+        lse = qkv.new_empty((batch, heads, seq), dtype=torch.float32)
+        return o, lse, qkv.new_empty((stats_numel(batch, heads, seq, seq),), dtype=torch.float32)
+
+    @torch.library.register_fake("co_alibi::bwd_qkv")
+    def _bwd_qkv_fake(do, qkv, o, lse, stats, slopes, causal, sm_scale):
+        """dqkv in qkv's shape and dtype."""
+        return torch.empty_like(qkv, memory_format=torch.contiguous_format)
 
     @torch.library.register_fake("co_alibi::decode")
     def _decode_fake(q, k_cache, v_cache, slopes, seq_lens, max_seq_len, sm_scale, with_lse):

@@ -14,7 +14,7 @@
  * and a decode step the reference does not have, co_alibi_decode: its forward
  * with Sq = 1 over a key / value cache, as one split-K pass over the cache.
  *
- * Tensor layout: contiguous row-major, q / o / dout / dq are (B, Hq, Sq, D),
+ * Tensor layout (except the _strided calls): contiguous row-major, q / o / dout / dq are (B, Hq, Sq, D),
  * k / v / dk / dv are (B, Hkv, Skv, D); query head h attends key/value head
  * h / (Hq / Hkv) (the head mapping of co_alibi_attn.py:143-146, done in-kernel
  * instead of by repeat_interleave).  Element type is selected by `dtype`; all
@@ -109,6 +109,17 @@ int co_alibi_fwd_inference(int dtype, const void* q, const void* k, const void* 
                            int heads_kv, int seq_q, int seq_kv, int head_dim, int causal, float sm_scale,
                            void* stream);
 
+/* Forward on operands in other layouts, as a model's projections leave them ((B, S, H, D) memory,
+ * parts of a packed QKV tensor): strides holds the batch, head and row strides in elements of q, k, v
+ * and o, in this order (12 values).  A row's head_dim elements are consecutive; strides are whole
+ * 16-byte units, row strides at least head_dim and at most 2^20, k's and v's the same.  With stats it is co_alibi_fwd;
+ * without (NULL) it is co_alibi_fwd_inference, with its workspace.  lse and stats keep their layouts.
+ * The reference's kernels take the strides of q, k, v and o too (co_alibi_attn.py:41-57). */
+int co_alibi_fwd_strided(int dtype, const void* q, const void* k, const void* v, const float* slopes, void* o,
+                         const long long* strides, float* lse, float* stats, void* workspace,
+                         size_t workspace_bytes, int batch, int heads_q, int heads_kv, int seq_q, int seq_kv,
+                         int head_dim, int causal, float sm_scale, void* stream);
+
 /* Backward: given dout and the forward's q, k, v, o, lse, stats, writes dq
  * (B,Hq,Sq,D), dk and dv (B,Hkv,Skv,D), all in dtype.  For Hkv < Hq the key /
  * value gradients are summed over the query heads of each group.  workspace
@@ -118,6 +129,15 @@ int co_alibi_bwd(int dtype, const void* dout, const void* q, const void* k, cons
                  void* dk, void* dv, void* workspace, size_t workspace_bytes, int batch, int heads_q,
                  int heads_kv, int seq_q, int seq_kv, int head_dim, int causal, float sm_scale,
                  void* stream);
+
+/* co_alibi_bwd on operands in other layouts (co_alibi_fwd_strided's rules): strides holds those of
+ * dout, q, k, v, o, dq, dk and dv, in this order (24 values).  On the score-store path only: a smaller
+ * workspace than co_alibi_bwd_score_store_workspace_bytes(...) is CO_ALIBI_EINVAL. */
+int co_alibi_bwd_strided(int dtype, const void* dout, const void* q, const void* k, const void* v,
+                         const void* o, const float* lse, const float* stats, const float* slopes, void* dq,
+                         void* dk, void* dv, const long long* strides, void* workspace, size_t workspace_bytes,
+                         int batch, int heads_q, int heads_kv, int seq_q, int seq_kv, int head_dim, int causal,
+                         float sm_scale, void* stream);
 
 /* The two passes of co_alibi_bwd as separate calls, for callers that time or
  * schedule them apart.  co_alibi_bwd_dq writes dq and fills the workspace
