@@ -177,6 +177,7 @@ __device__ __forceinline__ void fwd_tile(const T* __restrict__ sK, const T* __re
 // predicted cost first.
 constexpr int kOrderBuckets = 256;  // cost classes: ceil(extent / 256) keys or rows each
 constexpr int kOrderLdsHeads = 1024;
+constexpr int kOrderLdsItems = 8192;
 
 struct ScheduleArgs {
   const float* slopes;
@@ -203,29 +204,31 @@ __device__ __forceinline__ unsigned long long same_bucket(int b, bool ok) {
 
 // Stable counting sort by one work-group of 256 threads: out[j] is the j-th of the n items in
 // decreasing bucket order, the items of one bucket in index order.  Wavefront w takes the w-th
-// quarter of the items; per wavefront, a chunk of 64 items is counted (and later placed) with
-// one LDS update per distinct bucket, by the lowest lane that holds it.  lds: 5 *
-// kOrderBuckets ints.
+// quarter of the items and places them in chunks of 64, the lowest lane that holds a bucket moving
+// its cursor.  The buckets are computed first, by all threads at once, and kept in LDS as bytes (for
+// the first kOrderLdsItems items; the rest are computed again where they are needed), and counted
+// with LDS atomics: computed chunk by chunk on each wavefront's critical path, twice, they made this
+// work-group the longest of its launch (key-norm launch at the headline 19.5 -> 16.8 us, B1 H8 n
+// 16384 D64 10.6 -> 7.2, B8 H12 n 1024 D64 10.5 -> 6.9).
+// lds: 5 * kOrderBuckets ints.  cls: kOrderLdsItems bytes.
 template <typename F>
-__device__ void sort_items_desc(int n, const F& bucket, int* __restrict__ out, int* lds, int tid) {
+__device__ void sort_items_desc(int n, const F& bucket, int* __restrict__ out, int* lds, unsigned char* cls, int tid) {
   constexpr int K = kOrderBuckets;
-  static_assert(K == 256, "one thread per bucket in the scan");
+  static_assert(K == 256, "one thread per bucket in the scan, a byte per class");
   int* const cur = lds;          // [4][K]: per-wavefront counts, then per-wavefront cursors
   int* const part = lds + 4 * K;  // [4]: per-wavefront scan totals
   const int lane = tid & 63, wave = tid >> 6;
-  for (int j = tid; j < 4 * K; j += 256) cur[j] = 0;
-  __syncthreads();
   const int per = (n + 3) / 4;
   const int lo = min(wave * per, n), hi = min(lo + per, n);
-  int* const mine = cur + wave * K;
-  for (int base = lo; base < hi; base += 64) {
-    const int i = base + lane;
-    const bool ok = i < hi;
-    const int b = ok ? bucket(i) : 0;
-    const unsigned long long peers = same_bucket(b, ok);
-    if (ok && __popcll(peers & ((1ull << lane) - 1)) == 0) mine[b] += __popcll(peers);
+  for (int j = tid; j < 4 * K; j += 256) cur[j] = 0;
+  __syncthreads();
+  for (int i = tid; i < n; i += 256) {
+    const int b = bucket(i);
+    if (i < kOrderLdsItems) cls[i] = (unsigned char)b;
+    atomicAdd(&cur[i / per * K + b], 1);
   }
   __syncthreads();
+  auto bucket_of = [&](int i) { return i < kOrderLdsItems ? (int)cls[i] : bucket(i); };
   // Thread t owns bucket K - 1 - t (descending): its total over the wavefronts, an exclusive
   // scan over the threads, then each wavefront's cursor for the bucket.
   const int bk = K - 1 - tid;
@@ -248,10 +251,12 @@ __device__ void sort_items_desc(int n, const F& bucket, int* __restrict__ out, i
     start += c[w];
   }
   __syncthreads();
+  int* const mine = cur + wave * K;
+  int next = lo + lane < hi ? bucket_of(lo + lane) : 0;  // one chunk ahead
   for (int base = lo; base < hi; base += 64) {
-    const int i = base + lane;
+    const int i = base + lane, b = next;
     const bool ok = i < hi;
-    const int b = ok ? bucket(i) : 0;
+    next = i + 64 < hi ? bucket_of(i + 64) : 0;
     const unsigned long long peers = same_bucket(b, ok);
     if (ok) {
       // LDS operations of the wavefront complete in program order: every lane reads the
@@ -313,6 +318,7 @@ struct KeyCost {
 __device__ void schedule_orders(const ScheduleArgs& s, int which, int tid) {
   __shared__ int lds[5 * kOrderBuckets];
   __shared__ float wlds[kOrderLdsHeads];
+  __shared__ unsigned char cls[kOrderLdsItems];
   for (int h = tid; h < min(s.Hq, kOrderLdsHeads); h += 256) {
     const float lam = s.slopes[h];
     wlds[h] = lam > 0.f ? s.window / lam : __builtin_inff();
@@ -325,7 +331,7 @@ __device__ void schedule_orders(const ScheduleArgs& s, int which, int tid) {
     if (s.rows_sorted) {
       const RowCost cost{win, s.B * s.Hq, s.Hq, nQB, s.Skv, s.causal,
                          (float)((s.Skv + kOrderBuckets - 1) / kOrderBuckets)};
-      sort_items_desc(n, cost, s.row_order, lds, tid);
+      sort_items_desc(n, cost, s.row_order, lds, cls, tid);
     } else {
       for (int i = tid; i < n; i += 256) s.row_order[i] = i;
     }
@@ -335,7 +341,7 @@ __device__ void schedule_orders(const ScheduleArgs& s, int which, int tid) {
     if (s.keys_sorted) {
       const KeyCost cost{win, s.B * s.Hkv, s.Hkv, s.Sq, s.causal,
                          (float)((s.Sq + kOrderBuckets - 1) / kOrderBuckets)};
-      sort_items_desc(n, cost, s.key_order, lds, tid);
+      sort_items_desc(n, cost, s.key_order, lds, cls, tid);
     } else {
       for (int i = tid; i < n; i += 256) s.key_order[i] = i;
     }
@@ -518,7 +524,8 @@ __device__ __forceinline__ void fwd_row_block(const FwdArgs& args, int bh, int q
     // Every wavefront's rows passed the tail test after tile kt + 1: the keys left of it
     // carry weights below 2^-skip_log2<T>() (the vote is uniform, so all wavefronts leave here).
     // Leaving through the loop bound rather than a break keeps the loop's register
-    // allocation as it is without the skip (a break costs 13 spilled registers at D = 128).
+    // allocation as it is without the skip (a break costs 13 spilled registers at D = 128, the
+    // test after the LDS stores 50).
     if (tail_skip && kt < nkt - 1 && (sDone[0] & sDone[1] & sDone[2] & sDone[3])) {
       kfirst = (kt + 1) * kFwdBN;
       kt_end = kt + 1;

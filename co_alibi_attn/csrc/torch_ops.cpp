@@ -60,14 +60,15 @@ Tensor aligned(const Tensor& t) {
   return c;
 }
 
-// Whether the kernels can read a (B, H, S, D) operand in place (co_alibi_fwd_strided's rules; strides of
-// dimensions of size 1 do not matter), and its batch, head and row strides.
+// Whether the kernels can read a (B, H, S, D) operand in place (co_alibi_fwd_strided's rules), and its
+// batch, head and row strides: those of dimensions of size 1 do not matter and are given as if
+// contiguous, which the kernels have faster instantiations for.
 struct Strides {
   long long v[3];
 };
 Strides strides_of(const Tensor& t) {
-  const int64_t D = t.size(3);
-  return {{t.size(0) == 1 ? 0 : t.stride(0), t.size(1) == 1 ? 0 : t.stride(1), t.size(2) == 1 ? D : t.stride(2)}};
+  const int64_t H = t.size(1), S = t.size(2), D = t.size(3);
+  return {{t.size(0) == 1 ? H * S * D : t.stride(0), H == 1 ? S * D : t.stride(1), S == 1 ? D : t.stride(2)}};
 }
 bool readable(const Tensor& t) {
   const int64_t per16 = 16 / t.element_size();

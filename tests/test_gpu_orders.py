@@ -143,3 +143,13 @@ def test_no_tables_without_the_tail_skip(case):
     assert not ints[:4].any()
     assert not ints[4: 4 + B * Hq * nqb].any()
     assert torch.equal(o, o_inf)
+
+
+@pytest.mark.parametrize("case", [(1, 1, 1, 70, 70, 64, torch.float16, True, "alibi"),
+                                  (5, 3, 3, 8200, 40, 32, torch.float16, True, "alibi"),
+                                  (3, 67, 67, 300, 3000, 32, torch.float16, False, "alibi")],
+                         ids=["one_block", "uneven_quarters", "past_the_lds_classes"])
+def test_order_sort_edges(case):
+    """One item, item counts that do not divide over the sorting wavefronts, and more key blocks
+    (9447) than the sort keeps classes of in LDS."""
+    test_orders_are_sorted_permutations(case)
