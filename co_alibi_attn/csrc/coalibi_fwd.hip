@@ -656,14 +656,18 @@ struct SplitCfg {
   static constexpr bool kFits = kLds <= 155 * 1024;
 };
 
-// Whether a row block of a head that has `keys` visible keys is split.  A head that the tail skip
-// stops after about window / slope keys walks at most that many in the whole-block form, which then
-// is the shorter one; the tail skip's record is per 128-row block, so the split form has none and
-// records that it processed every key.  With the skip switched off (window infinite) every
-// block is split.
-__device__ __forceinline__ bool split_row_block(int keys, float slope, float window) {
-  return !(slope > 0.f) || (float)keys <= 3.0f * (window / slope) + 192.0f;
-}
+// Which row blocks a launch splits: those of `keys` visible keys, longer than `longer_than`, of a head
+// that the tail skip stops after about window / slope keys, where that is not much sooner than the
+// split walk's end.  The tail skip's record is per 128-row block, so the split form has no skip
+// and records that it processed every key.  With the skip switched off the window is infinite.
+struct SplitRule {
+  float window;
+  float reach, slack;  // split up to reach * window / slope + slack keys
+  int longer_than;
+  __device__ __forceinline__ bool operator()(int keys, float slope) const {
+    return keys > longer_than && (!(slope > 0.f) || (float)keys <= reach * (window / slope) + slack);
+  }
+};
 
 template <typename T, int D, bool CAUSAL>
 __device__ __forceinline__ void fwd_split_rows(const FwdArgs& args, int bh, int q0, T* __restrict__ sK,
@@ -860,24 +864,35 @@ __device__ __forceinline__ void fwd_split_rows(const FwdArgs& args, int bh, int 
 }
 
 // Work-groups 8j .. 8j + 7 of every 32 run on the 8 XCDs: item (id / 32) * 8 + id % 8, so that the
-// four parts of a row block share their K and V in one XCD's L2.
+// four parts of a row block share their K and V in one XCD's L2.  Within an XCD the ids go to its four
+// shader engines in turn; which part takes which turn rotates, since a block that is not split runs
+// as its part 0 alone (without the rotation all of them share one engine).
 template <typename T, int D, bool CAUSAL, bool SKIP>
 __global__ __launch_bounds__(256, D * sizeof(T) > 256 ? 1 : 2) void coalibi_fwd_split_kernel(FwdArgs args,
-                                                                                               int items, float window) {
+                                                                                               int items, SplitRule rule,
+                                                                                               bool small) {
+  const bool by_head = small && CAUSAL;
   using C = SplitCfg<T, D>;
   __shared__ __align__(16) T sK[kSplitWaves * C::K_ELEMS];
   __shared__ __align__(16) T sV[kSplitWaves * C::V_ELEMS];
-  const int i = (blockIdx.x >> 5) * 8 + (blockIdx.x & 7), part = (blockIdx.x >> 3) & 3;
+  int i = (blockIdx.x >> 5) * 8 + (blockIdx.x & 7), part = ((blockIdx.x >> 3) + (blockIdx.x >> 5)) & 3;
+  if (!small) {
+    // Most blocks are whole, and a work-group that only exits still waits for a slot on its engine,
+    // holding up the ids after it: every part 0 first, then the others.
+    const int first = (items + 7) / 8 * 8, rest = (int)blockIdx.x - first;
+    i = rest < 0 ? (int)blockIdx.x : rest / 24 * 8 + (rest & 7);
+    part = rest < 0 ? 0 : 1 + (rest >> 3) % 3;
+  }
   if (i >= items) return;
-  // Causal: every block of a head on one XCD, where its K and V stay in one L2 (fp32, B2 H12 n 1000:
+  // by_head: every block of a head on one XCD, where its K and V stay in one L2 (fp32, B2 H12 n 1000:
   // 78.3 -> 58.4 us against the sorted order; n 512 to 2048 fp16: 3 to 13 %).  Non-causal heads differ
-  // more in work, and the sorted order is ahead (333 x 2047: 41.2 against 48.8).
-  const WorkItem item = !CAUSAL && args.row_order ? table_item(args.row_order, i, args.B * args.Hq, items)
-                                                  : lpt_item(i, args.B * args.Hq, CAUSAL ? 1 << 30 : 1);
+  // more in work, and the sorted order is ahead (333 x 2047: 41.2 against 48.8), as it is on larger grids.
+  const WorkItem item = !by_head && args.row_order ? table_item(args.row_order, i, args.B * args.Hq, items)
+                                                   : lpt_item(i, args.B * args.Hq, by_head ? 1 << 30 : 1);
   const int nQB = (args.Sq + kFwdBM - 1) / kFwdBM, qb = nQB - 1 - item.rank;
   const int q0 = qb * kFwdBM;
   const float slope = args.slopes[item.head % args.Hq];
-  if (split_row_block(CAUSAL ? min(q0 + kFwdBM, args.Skv) : args.Skv, slope, window)) {
+  if (rule(CAUSAL ? min(q0 + kFwdBM, args.Skv) : args.Skv, slope)) {
     if (blockIdx.x == 0 && args.flags != nullptr && threadIdx.x < kStatsHeader)
       args.flags[threadIdx.x] = threadIdx.x == 0 ? args.order_flags : 0;
     if (part == 0 && args.kstart != nullptr && threadIdx.x == 0) args.kstart[(size_t)item.head * nQB + qb] = 0;
@@ -902,6 +917,16 @@ __global__ __launch_bounds__(256, D * sizeof(T) > 256 ? 1 : 2) void coalibi_fwd_
 //   fp32   D 64: n 1000, 192 blocks 94.7 -> 76.5;  D 128: n 1024, 128 blocks 159.4 -> 105.8
 inline bool split_grid(long long row_blocks, int keys, bool causal) {
   return row_blocks <= std::max(128, causal ? std::min(keys / 4, 384) : std::min(keys / 8, 256));
+}
+
+// Beyond those grids (causal, tail skip on), whether only the longer half of the row blocks is split:
+// the flat heads' last blocks otherwise walk on alone after the rest.  us, whole-block form -> split:
+//   Hq32/Hkv8 n 1741 D128 bf16 (448 blocks) 70.7 -> 59.1; n 2048 D128 H32 (512) 80.9 -> 67.0, D64 62.4 ->
+//   55.3, H48 D64 (768) 65.6 -> 62.7, H64 D128 (1024) 90.1 -> 113.4; n 4096 H16 D128 (512) 142.2 -> 109.1,
+//   H24 D64 (768) 111.2 -> 93.2; n 1024 H64 D64 39.2 -> 40.8; n 8192 H8 D64 (512) 144.1 -> 148.9;
+//   skip off, every head's longer half: n 2048 H32 D128 70.5 -> 97.1
+inline bool split_long_rows(long long row_blocks, int keys) {
+  return row_blocks <= 768 && keys >= 1536 && keys <= 4096;
 }
 
 }  // namespace
@@ -933,15 +958,14 @@ hipError_t launch_fwd(const FwdArgs& a, hipStream_t stream) {
   const int nQB = (a.Sq + kFwdBM - 1) / kFwdBM;
   const int grid = nQB * a.B * a.Hq;
   if constexpr (SplitCfg<T, D>::kFits) {
-    if (split_grid(grid, a.Skv, CAUSAL)) {
+    const float window = a.every_key ? __builtin_inff() : order_window<T>();
+    const bool small = split_grid(grid, a.Skv, CAUSAL);
+    if (small || (CAUSAL && !a.every_key && split_long_rows(grid, a.Skv))) {
       const dim3 parts((grid + 7) / 8 * 32);
-      const float window = a.every_key ? __builtin_inff() : order_window<T>();
-      if (a.knorm != nullptr)
-        hipLaunchKernelGGL((coalibi_fwd_split_kernel<T, D, CAUSAL, true>), parts, dim3(256), 0, stream, f, grid,
-                           window);
-      else
-        hipLaunchKernelGGL((coalibi_fwd_split_kernel<T, D, CAUSAL, false>), parts, dim3(256), 0, stream, f, grid,
-                           window);
+      const SplitRule rule = small ? SplitRule{window, 3.0f, 192.0f, 0} : SplitRule{window, 1.25f, 0.0f, a.Skv / 2};
+      auto* const kernel = a.knorm != nullptr ? coalibi_fwd_split_kernel<T, D, CAUSAL, true>
+                                              : coalibi_fwd_split_kernel<T, D, CAUSAL, false>;
+      hipLaunchKernelGGL(kernel, parts, dim3(256), 0, stream, f, grid, rule, small);
       return hipGetLastError();
     }
   }

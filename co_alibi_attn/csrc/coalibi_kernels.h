@@ -41,7 +41,8 @@ constexpr float kLog2eHost = 1.4426950408889634f;
 // weight is below 2^-skip_log2 of it (the softmax probability s = 2^(a - LSE2) too).
 // The threshold follows the type P is rounded to before it multiplies V:
 //   fp16: 26 -- P < 2^-26 rounds to zero (below half the smallest subnormal, 2^-25), so
-//     the forward's O is bit-identical to the unskipped one;
+//     the forward's O is bit-identical to that of co_alibi_fwd without statistics, which skips
+//     nothing (with the skip switched off, small grids take other forms: coalibi_fwd.hip);
 //   bf16: 32 -- P keeps 8 bits, so each P carries a relative error up to 2^-9; the skipped
 //     weights together are below S * 2^-32 of the row total (1e-6 at S = 4096);
 //   fp32: 64 -- the validation mode stays within S * 2^-64 of the unskipped result.

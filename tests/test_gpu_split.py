@@ -68,3 +68,23 @@ def test_key_form_many_query_heads(dtype):
     ro, _ = ref.forward(qf, kf, vf, lam, causal=True, scale=0.25)
     want = (ro, *ref.backward(dof, qf, kf, vf, lam, causal=True, scale=0.25))
     assert_parity(got, want, TOL[dtype], "600 heads", dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32], ids=["fp16", "fp32"])
+def test_longer_half_split(dtype):
+    """A grid past the small ones (25 heads x 16 row blocks): the longer half of the flat heads' row
+    blocks is split, the rest and the steep heads run whole, in one launch; four heads checked."""
+    H, S, D = 25, 1937, 32
+    q, k, v, do = rand_inputs(1, H, H, S, S, D, dtype, seed=9)
+    do = do * 0.25
+    lam = torch.tensor([2.0, 0.05, 0.01, 0.0] + [0.3] * (H - 4)).to(dtype).float()
+    scale = 1.0 / math.sqrt(D)
+    qd, kd, vd = (t.to(DEV).requires_grad_() for t in (q, k, v))
+    o = CoALIBIAttention.apply(qd, kd, vd, lam.to(DEV), True, scale)
+    o.backward(do.to(DEV))
+    torch.cuda.synchronize()
+    got = tuple(t.detach()[:, :4].float().cpu() for t in (o, qd.grad, kd.grad, vd.grad))
+    qf, kf, vf, dof = (t[:, :4].float() for t in (q, k, v, do))
+    ro, _ = ref.forward(qf, kf, vf, lam[:4], causal=True, scale=scale)
+    want = (ro, *ref.backward(dof, qf, kf, vf, lam[:4], causal=True, scale=scale))
+    assert_parity(got, want, TOL[dtype], "longer half", dtype)
