@@ -906,15 +906,15 @@ __global__ __launch_bounds__(256, D * sizeof(T) > 256 ? 1 : 2) void coalibi_fwd_
 // walks leave more of it (causal: half the work of the longest block on average, and the short
 // blocks' work-groups cost their prologue and merge all the same).  us, whole-block form ->
 // split, fp16 (f = tail skip off):
-//   D 128  n 256: 64 blocks 19.4 -> 13.1 f 13.1 -> 9.2, 128: 19.7 -> 16.5 f 13.3 -> 11.0
-//          n 512: 64 blocks 27.1 -> 20.1 f 20.2 -> 12.2, 128: 27.2 -> 24.4 f 20.3 -> 13.9, 192: 28.2 -> 33.1 f 20.8 -> 22.1
-//          n 1024: 128 blocks 42.6 -> 28.0 f 34.1 -> 21.1, 256: 44.5 -> 44.1 f 35.0 -> 32.8, 320: 46.7 -> 53.2 f 37.5 -> 41.1
-//          n 2048: 128 blocks 73.8 -> 37.6 f 61.5 -> 34.7, 256: 74.9 -> 53.2 f 62.9 -> 52.0, 320: 77.3 -> 61.6 f 66.8 -> 61.9
-//   D 64   n 512: 128 blocks 21.6 -> 19.9 f 14.9 -> 10.4, 192: 22.2 -> 23.1 f 15.2 -> 13.0
-//          n 1024: 256 blocks 34.1 -> 32.7 f 25.3 -> 22.0;  n 2048: 320 blocks 59.5 -> 42.9 f 45.9 -> 40.1
-//   non-causal, D 128: 333 x 2047, 96 blocks 91.0 -> 40.9; 2000 x 3000, 256 blocks 126.2 -> 81.2;
+//   D 128  n 256: 64 blocks 19.5 -> 14.2 f 13.1 -> 9.8, 128: 19.8 -> 16.1 f 13.3 -> 11.6
+//          n 512: 64 blocks 27.1 -> 20.5 f 20.1 -> 13.3, 128: 27.4 -> 22.2 f 20.3 -> 14.9, 192: f 20.8 -> 22.1
+//          n 1024: 128 blocks 43.1 -> 27.4 f 34.2 -> 22.1, 256: 44.5 -> 39.5 f 35.4 -> 34.3, 320: f 37.5 -> 41.1
+//          n 2048: 128 blocks 74.0 -> 40.1 f 61.7 -> 36.5, 256: 75.4 -> 49.7 f 62.6 -> 54.1, 320: 77.7 -> 49.2 f 65.5 -> 65.6
+//   D 64   n 512: 128 blocks 21.5 -> 16.2 f 15.0 -> 10.8
+//          n 1024: 256 blocks 34.2 -> 27.9 f 25.3 -> 22.2;  n 2048: 320 blocks 59.1 -> 36.9 f 46.0 -> 40.9
+//   non-causal, D 128: 333 x 2047, 96 blocks 90.5 -> 41.3; 2000 x 3000, 256 blocks 126.2 -> 69.0;
 //          D 64, 1400 x 1400, 352 blocks 43.8 -> 51.8
-//   fp32   D 64: n 1000, 192 blocks 94.7 -> 76.5;  D 128: n 1024, 128 blocks 159.4 -> 105.8
+//   fp32   D 64: n 1000, 192 blocks 94.7 -> 56.9;  D 128: n 1024, 128 blocks 160.1 -> 73.1
 inline bool split_grid(long long row_blocks, int keys, bool causal) {
   return row_blocks <= std::max(128, causal ? std::min(keys / 4, 384) : std::min(keys / 8, 256));
 }
