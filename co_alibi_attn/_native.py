@@ -37,6 +37,7 @@ EXPORTS = (
     "co_alibi_bwd_dq",
     "co_alibi_bwd_dkdv",
     "co_alibi_decode_workspace_bytes",
+    "co_alibi_decode_splits",
     "co_alibi_decode",
     "co_alibi_decode_noalloc",
     "co_alibi_probe_mfma",
@@ -80,6 +81,7 @@ _SIGNATURES = {
         [_I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _Z, _I, _I, _I, _I, _I, _I, _I, _F, _P],
     ),
     "co_alibi_decode_workspace_bytes": (_Z, [_I, _I, _I, _I]),
+    "co_alibi_decode_splits": (_I, [_I, _I, _I, _I, _I, _I]),
     "co_alibi_decode": (_I, [_I, _P, _P, _P, _P, _P, _P, _P, _P, _Z, _I, _I, _I, _I, _I, _I, _F, _P]),
     "co_alibi_decode_noalloc": (_I, [_I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P]),
     "co_alibi_probe_mfma": (_I, [_P, _P, _I, _I, _P]),

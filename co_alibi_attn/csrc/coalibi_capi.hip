@@ -462,22 +462,68 @@ int device_cus() {
   return n;
 }
 
-// Split count of a decode launch over equal lengths: an equal run of 128-key chunks for each of
-// kDecodeWGsPerCU work-groups per CU (decode_cps), at most decode_splits_max.  One split needs no
-// merge launch, which costs as much as two to three more chunks in one work-group's walk: 8.5
-// against 10.4 us at 2 chunks, 11.2 against 11.9 at 3 and 13.4 against 12.0 at 4 (B1, Hq32/Hkv8,
-// D128, bf16; B16: 9.8 against 13.2 at 2, 14.1 against 15.7 at 4).
-constexpr int kDecodeDirectChunks = 3;
+// How a decode is split, by its type and by units = batch * heads_kv against the `slots` work-groups
+// that the launch is sized for.  Figures: us on the GPU alone, 512 slots, more splits -> fewer.
 constexpr int kDecodeRaggedSplits = 4;
-int decode_splits(int batch, int heads_kv, int seq_kv, int slots) {
-  const int chunks = static_cast<int>(decode_chunks(seq_kv));
-  const long long units = static_cast<long long>(batch) * heads_kv;
-  if (chunks <= kDecodeDirectChunks || units >= slots) return 1;
-  const int cps = coalibi::decode_cps(units * chunks, chunks, slots, coalibi::kMaxDecodeSplits,
-                                      [&](int c) { return units * ((chunks + c - 1) / c); });
-  const int n = (chunks + cps - 1) / cps, own = (chunks + n - 1) / n;
-  return (chunks + own - 1) / own;  // in equal runs
-}
+struct DecodeRule {
+  bool fp32;
+  int head_dim, slots;
+  long long units;
+
+  // Whether a sequence of up to `chunks` chunks is one work-group's (one split, and no merge launch, which
+  // costs as much as one to three more chunks of the walk).  Units 8: D 32 fp16 at 3 chunks 8.2 -> 6.8, D 64 8.8 ->
+  // 8.4, D 128 bf16 at 2 10.3 -> 9.0 (at 3 10.8 -> 10.9, with lengths of 1/8 to all of the bound 10.4 -> 8.7), fp32 D 32
+  // at 2 9.2 -> 7.8; D 256 at 2 13.9 -> 14.1 and fp32 D 64 11.1 -> 11.4 (at 3 14.5 -> 18.3 and 11.3 -> 15.5).  With a
+  // work-group per chunk above half the slots more splits cost more: at 3 chunks, units 100, D 128 12.7 -> 10.8, D 256
+  // 21.8 -> 17.9; units 192 fp32 D 64 22.7 -> 17.6 (units 128 16.8 -> 17.3; ragged, D 256 16.5 -> 18.7).  Above half the slots in units two splits take two rounds: units
+  // 288, 6 chunks, D 128 29.5 -> 28.0, 5 chunks, D 256 61 -> 57 (8: 79 -> 84), 3 chunks, fp32 D 128 62 -> 55 (4: 64 ->
+  // 69); ragged lengths of at most 8 chunks take 5 to 30 % less on average.  From 5/6 of the slots on one split
+  // loses nothing: units 432, D 128, 8 chunks 43.4 -> 38.7, 32 chunks 157 -> 147 (units 384: 124 -> 135), but
+  // D 32 from 16 chunks on (units 448, 32 chunks 65.9 -> 67.6).
+  bool one_split(int chunks, bool ragged) const {
+    if (units >= slots) return true;
+    if (units * 6 >= slots * 5LL) return head_dim > 32 || chunks <= 16;
+    if (units * 2 > slots) return chunks <= (ragged ? 8 : fp32 ? 3 : head_dim <= 128 ? 6 : 5);
+    if (chunks <= 3 && units * chunks * (ragged ? 4 : 6) > slots * 3LL) return true;
+    if (fp32) return chunks <= (head_dim <= 32 ? 2 : 1);
+    return chunks <= (head_dim <= 64 ? 3 : head_dim > 128 ? 1 : ragged ? 3 : 2);
+  }
+
+  // Equal splits: as many per sequence as it takes to give every slot a work-group.
+  int even_splits(int chunks) const {
+    const long long want = (slots + units - 1) / units;
+    const int most = std::min(chunks, coalibi::kMaxDecodeSplits);
+    const int cps = (chunks + static_cast<int>(std::min<long long>(want, most)) - 1) /
+                    static_cast<int>(std::min<long long>(want, most));
+    return (chunks + cps - 1) / cps;
+  }
+
+  // Splits of every sequence of a launch bound by `chunks` chunks.  Equal lengths: where even_splits' last
+  // round is nearly empty, longer splits (decode_cps): units 100, 32 chunks, D 128 48 -> 39; units 36, 100 chunks,
+  // D 256 113 -> 89; short walks of the small types do not gain (units 100, 6 chunks, D 32 10.1 -> 11.3).  Up to half
+  // as long again from D 128 on (units 180, 125 chunks, D 128 294 -> 267; with a quarter 295), a quarter in
+  // the small types (units 210, 100 chunks, D 64 127 -> 133 with a half).
+  int splits(int chunks, bool ragged) const {
+    if (one_split(chunks, ragged)) return 1;
+    const bool small = !fp32 && head_dim <= 64;
+    const int even = even_splits(chunks);
+    if (ragged || (small && chunks < 4 * even)) return even;
+    const int cps = coalibi::decode_cps(units * chunks, chunks, slots, coalibi::kMaxDecodeSplits, small ? 4 : 8, chunks - 1,
+                                        [&](int c) { return units * ((chunks + c - 1) / c); });
+    const int n = (chunks + cps - 1) / cps, own = (chunks + n - 1) / n;
+    return (chunks + own - 1) / own;  // in equal runs
+  }
+
+  // Whether a batch with a length per sequence shares its real chunks out (the kernels' plan) rather than
+  // splitting every sequence by the bound.  The plan costs the two kernels about 3.5 us together, against
+  // the part of a split's walk that it saves.  Lengths of 1/8 to all of the bound, units 128: D 128 at 2 chunks per
+  // split 17.7 -> 20.6, at 4 +2 %, at 6 -17 %, at 16 -8 %; D 64 at 4 +5 %, at 6 -15 %; D 32 at 4 +11 %, at 8 +2 %, at
+  // 12 -12 %; D 256 at 2 +10 %, at 4 -3 %; fp32 D 64 at 2 +17 %, at 4 -9 %.
+  bool plans(int chunks, int splits) const {
+    return splits > 1 && (chunks + splits - 1) / splits >= (fp32 || head_dim > 128 ? 4 : head_dim > 32 ? 5 : 9);
+  }
+  int plan_slack() const { return !fp32 && head_dim <= 64 ? 4 : 6; }
+};
 
 // Bytes of split-K partials for `parts` (batch, query head, split) triples: the maximum, the sum
 // and the sigma total (one 256-byte aligned fp32 array each), then head_dim floats of O per part.
@@ -541,8 +587,10 @@ int decode_impl(const char* fn, bool scratch_ws, int dtype, const void* q, const
                                      std::to_string(coalibi::kMaxDecodeChunks * coalibi::kDecodeChunkKeys));
   // The workspace size first: it depends on the shape only, and a decode whose partials do not fit
   // is refused before any pointer is looked at.
-  const int slots = coalibi::kDecodeWGsPerCU * device_cus();
-  int splits = decode_splits(batch, heads_kv, seq_kv, slots);
+  const DecodeRule rule{dtype == CO_ALIBI_F32, head_dim, coalibi::kDecodeWGsPerCU * device_cus(),
+                        static_cast<long long>(batch) * heads_kv};
+  const int chunks = static_cast<int>(decode_chunks(seq_kv));
+  int splits = rule.splits(chunks, seq_lens != nullptr);
   const size_t rows = static_cast<size_t>(batch) * heads_q;
   size_t parts = rows * (scratch_ws ? static_cast<size_t>(splits) : decode_splits_max(seq_kv));
   const size_t need = decode_partials_bytes(parts, head_dim);
@@ -561,7 +609,8 @@ int decode_impl(const char* fn, bool scratch_ws, int dtype, const void* q, const
     return rc;
   if (!std::isfinite(sm_scale)) return fail(CO_ALIBI_EINVAL, std::string(fn) + ": sm_scale must be finite");
 
-  if (seq_lens != nullptr && splits > 1) {
+  const bool plan = seq_lens != nullptr && rule.plans(chunks, splits);
+  if (plan) {
     // Lengths below seq_kv leave work-groups to the longer sequences, up to kDecodeRaggedSplits
     // times as many splits each, where their partials fit.
     const size_t most = std::min(static_cast<size_t>(splits) * kDecodeRaggedSplits, decode_splits_max(seq_kv));
@@ -593,8 +642,10 @@ int decode_impl(const char* fn, bool scratch_ws, int dtype, const void* q, const
   a.L = seq_kv;
   a.cap = kv_capacity;
   a.nSplits = splits;
-  a.cps = static_cast<int>((decode_chunks(seq_kv) + splits - 1) / splits);
-  a.slots = slots;
+  a.cps = (chunks + splits - 1) / splits;
+  a.slots = rule.slots;
+  a.slack = rule.plan_slack();
+  a.plan = plan;
   a.sc2 = sm_scale * coalibi::kLog2eHost;
   hipStream_t st = static_cast<hipStream_t>(stream);
   hipError_t e;
@@ -614,6 +665,15 @@ extern "C" {
 size_t co_alibi_decode_workspace_bytes(int batch, int heads_q, int seq_kv, int head_dim) {
   if (batch < 1 || heads_q < 1 || seq_kv < 1 || head_dim < 1) return 0;
   return decode_partials_bytes(static_cast<size_t>(batch) * heads_q * decode_splits_max(seq_kv), head_dim);
+}
+
+int co_alibi_decode_splits(int dtype, int batch, int heads_kv, int seq_kv, int head_dim, int ragged) {
+  if (batch < 1 || heads_kv < 1 || seq_kv < 1 || decode_chunks(seq_kv) > static_cast<size_t>(coalibi::kMaxDecodeChunks))
+    return 0;
+  const DecodeRule rule{dtype == CO_ALIBI_F32, head_dim, coalibi::kDecodeWGsPerCU * device_cus(),
+                        static_cast<long long>(batch) * heads_kv};
+  const int chunks = static_cast<int>(decode_chunks(seq_kv)), splits = rule.splits(chunks, ragged != 0);
+  return ragged != 0 && rule.plans(chunks, splits) ? -splits : splits;
 }
 
 int co_alibi_decode(int dtype, const void* q, const void* k_cache, const void* v_cache, const float* slopes,

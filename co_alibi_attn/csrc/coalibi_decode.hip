@@ -34,6 +34,7 @@ namespace coalibi {
 namespace {
 
 constexpr int kDecWaves = 4;
+static_assert(kDecWaves * kWaveKeys == kDecodeChunkKeys, "chunk = the work-group's keys");
 constexpr int kDecMergeThreads = 256;
 
 __device__ __forceinline__ int decode_chunks_of(int len) { return (len + kDecodeChunkKeys - 1) / kDecodeChunkKeys; }
@@ -64,7 +65,8 @@ __device__ __forceinline__ int chunks_per_split(const DecodeArgs& a, int lane) {
   }
   total = wave_reduce(total, [](int x, int y) { return x + y; });
   longest = wave_reduce(longest, [](int x, int y) { return max(x, y); });
-  return decode_cps(static_cast<long long>(total) * a.Hkv, longest, a.slots, a.nSplits, [&](int c) {
+  return decode_cps(static_cast<long long>(total) * a.Hkv, longest, a.slots, a.nSplits, a.slack, longest,
+                    [&](int c) {
     int n = 0;
     for (int b = lane; b < a.B; b += 64) n += (decode_chunks_of(seq_len_of(a, b)) + c - 1) / c;
     return static_cast<long long>(wave_reduce(n, [](int x, int y) { return x + y; })) * a.Hkv;
@@ -131,9 +133,9 @@ struct DecCfg {
                 "O partials alias the tiles");
 };
 
-// How a launch splits its sequences: evenly, by a plan over a length per sequence (RAGGED), or not
-// at all (DIRECT, nSplits == 1): the work-group then writes o and lse itself and no merge is
-// launched.
+// How a launch splits its sequences: into splits of cps chunks, whatever their lengths (kEven), by a
+// plan over a length per sequence (kRagged, a.plan), or not at all (kDirect, nSplits == 1): the
+// work-group then writes o and lse itself and no merge is launched.
 enum class Split { kEven, kRagged, kDirect };
 
 template <typename T, int D, Split SPLIT>
@@ -166,16 +168,24 @@ __global__ __launch_bounds__(kDecWaves * 64, (D > 128 || sizeof(T) == 4) ? 1 : 2
   const int split = item.split, bhk = item.bhk;
   const int G = a.G, nS = a.nSplits;
   const int b = bhk / a.Hkv, hkv = bhk - b * a.Hkv;
-  const int L = SPLIT == Split::kEven ? a.L : seq_len_of(a, b);  // kEven: no lengths
+  const int L = seq_len_of(a, b);
   const int hq0 = hkv * G;  // first query head of the group
   const size_t bh0 = (size_t)b * a.Hq + hq0;
   if constexpr (kRagged) cps = seq_splits(decode_chunks_of(L), cps).cps;
   const int c_first = split * cps;
   const int c_last = min(c_first + cps, decode_chunks_of(L)) - 1;
-  if (c_last < c_first) {  // an empty sequence: no partial (the merge reads none)
-    if constexpr (kDirect) {
+  if (c_last < c_first) {
+    if constexpr (kDirect) {  // an empty sequence
       for (int i = tid; i < G * D; i += kDecWaves * 64) static_cast<T*>(a.o)[bh0 * D + i] = T(0);
       if (tid < G && a.lse != nullptr) a.lse[bh0 + tid] = kNegInf;
+    } else if constexpr (!kRagged) {  // past this sequence's length: an empty partial (a plan's merge reads none)
+      for (int i = tid; i < G * D; i += kDecWaves * 64) a.pout[((bh0 + i / D) * nS + split) * D + i % D] = 0.f;
+      if (tid < G) {
+        const size_t pi = (bh0 + tid) * nS + split;
+        a.pmax[pi] = kNegInf;
+        a.psum[pi] = 0.f;
+        a.psig[pi] = 0.f;
+      }
     }
     return;
   }
@@ -460,7 +470,8 @@ __global__ __launch_bounds__(kDecMergeThreads) void coalibi_decode_merge_kernel(
 #pragma unroll
   for (int w = 0; w < NW; ++w) m = fmaxf(m, sRed[w]);
   __syncthreads();
-  // A sequence of length 0 has no split: O = 0 and LSE = -inf.
+  // Empty splits have maximum -inf and weight 0; a sequence of length 0 has no split with a key:
+  // O = 0 and LSE = -inf.
   const float mref = m == kNegInf ? 0.f : m;
   float l = 0.f;
   for (int c = tid; c < nS; c += kDecMergeThreads) {
@@ -508,7 +519,7 @@ hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream) {
     hipLaunchKernelGGL((coalibi_decode_split_kernel<T, D, Split::kDirect>), even, threads, 0, stream, a);
     return hipGetLastError();
   }
-  if (a.seq_lens == nullptr) {
+  if (!a.plan) {
     hipLaunchKernelGGL((coalibi_decode_split_kernel<T, D, Split::kEven>), even, threads, 0, stream, a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;

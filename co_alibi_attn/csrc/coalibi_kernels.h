@@ -221,8 +221,10 @@ struct DecodeArgs {
   const int* seq_lens;  // (B,) per-sequence cache lengths, or NULL (all L)
   int B, Hq, Hkv, G, L, cap;
   int nSplits;  // most splits of any sequence: the partials' stride
-  int cps;      // chunks per split without seq_lens (with them the kernels share the chunks out)
+  int cps;      // chunks per split (with a plan the kernels share the chunks out)
   int slots;    // resident work-groups the splits are sized for
+  int slack;    // the plan's (decode_cps)
+  bool plan;    // splits sized by the lengths in seq_lens (DecodeRule::plans, coalibi_capi.hip)
   float sc2;
 };
 
@@ -231,14 +233,16 @@ constexpr int kDecodeWGsPerCU = 2;
 
 // Chunks per split of a decode over sequences with `work` chunks in all (summed over the kv heads;
 // `longest` in the longest one): an equal share of `work` per resident work-group, or up to
-// half as much again where that brings groups(c), the work-groups that c chunks per split make,
-// into one round of `slots`.  At most `max_splits` splits per sequence.  The same rule on the host
-// (one length) and in the kernels (a length per sequence), so equal lengths split alike.
+// slack/16 more and one chunk (and at most `most`) where that brings groups(c), the work-groups that c chunks per
+// split make, into one round of `slots`.  At most `max_splits` splits per sequence.  On the host
+// for equal lengths, in the kernels for a length per sequence.
 template <typename F>
-__host__ __device__ inline int decode_cps(long long work, int longest, int slots, int max_splits, const F& groups) {
+__host__ __device__ inline int decode_cps(long long work, int longest, int slots, int max_splits, int slack, int most,
+                                          const F& groups) {
   const int share = static_cast<int>((work + slots - 1) / slots), fit = (longest + max_splits - 1) / max_splits;
   const int c0 = share > fit ? (share > 1 ? share : 1) : (fit > 1 ? fit : 1);
-  for (int c = c0; c <= c0 + c0 / 2 + 1; c += 1 + c / 16)
+  const int c1 = c0 + 1 + static_cast<int>(static_cast<long long>(c0) * slack / 16);
+  for (int c = c0; c <= (c1 < most ? c1 : most); c += 1 + c / 16)
     if (groups(c) <= slots) return c;
   return c0;
 }

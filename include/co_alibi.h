@@ -160,6 +160,12 @@ int co_alibi_bwd_dkdv(int dtype, const void* dout, const void* q, const void* k,
  * split walks one or more 128-key chunks of the cache). */
 size_t co_alibi_decode_workspace_bytes(int batch, int heads_q, int seq_kv, int head_dim);
 
+/* How a decode of this shape is launched: the splits of every sequence, each a work-group per key
+ * head (1: no partials and no merge launch).  With per-sequence lengths (ragged != 0) a negative
+ * value: the lengths decide, in place of that many by the bound seq_kv.  No counterpart in the
+ * reference; it serves tests and measurements. */
+int co_alibi_decode_splits(int dtype, int batch, int heads_kv, int seq_kv, int head_dim, int ragged);
+
 /* Decode: one new query per (batch, query head) against a key / value cache.
  * q and o are (B, Hq, D); k_cache and v_cache are (B, Hkv, kv_capacity, D).  Sequence
  * b has its first len_b rows of every head filled, all of them visible to the query

@@ -1,0 +1,70 @@
+"""Which kernel forms the host's rules choose, at shapes on both sides of their lines (measured at
+256 CUs, the figures stand beside the rules).  The rules are host code: no GPU is needed."""
+import pytest
+
+from co_alibi_attn import _native
+
+F32, F16, BF16 = 0, 1, 2
+
+
+# (dtype, batch, heads_kv, seq_kv, head_dim, lengths per sequence, splits; negative: the lengths decide)
+DECODE = [
+    # short caches: one split, where the type's chunk walk is cheaper than a merge launch
+    (F16, 1, 8, 300, 32, False, 1),
+    (BF16, 1, 8, 200, 128, False, 1),
+    (BF16, 1, 8, 300, 128, False, 3),
+    (BF16, 1, 8, 300, 128, True, 1),
+    (BF16, 1, 8, 300, 256, False, 3),
+    (F32, 1, 8, 300, 64, False, 3),
+    (F32, 1, 8, 200, 64, True, 2),
+    (BF16, 10, 10, 300, 256, False, 1),  # more work-groups than half the slots
+    (BF16, 16, 8, 300, 256, True, 3),
+    # short walks with lengths: the plan would cost more than it shares out
+    (BF16, 1, 8, 500, 128, True, 4),
+    (BF16, 1, 8, 4000, 128, True, 32),
+    (BF16, 8, 8, 1000, 128, True, 8),
+    (BF16, 16, 8, 1000, 128, True, 4),
+    (F16, 16, 8, 1000, 64, True, 4),
+    (F16, 8, 8, 4000, 32, True, 8),
+    (F32, 32, 8, 700, 64, True, 2),
+    # long ones: it pays
+    (BF16, 16, 8, 8192, 128, True, -4),
+    (F16, 16, 8, 8192, 64, True, -4),
+    (F16, 32, 8, 4000, 32, True, -2),
+    (F32, 16, 8, 4000, 64, True, -4),
+    # between half the slots and all of them: two splits unless the walk is short
+    (BF16, 12, 24, 700, 128, False, 1),
+    (BF16, 12, 24, 1000, 128, False, 2),
+    (F32, 12, 24, 500, 64, False, 2),
+    (BF16, 12, 24, 1000, 256, False, 2),
+    (F16, 44, 8, 12780, 64, False, 2),
+    (BF16, 48, 8, 4076, 128, False, 2),
+    (BF16, 48, 8, 1000, 128, True, 1),
+    (BF16, 54, 8, 4000, 128, False, 1),
+    (F16, 63, 8, 16000, 32, False, 2),
+    (BF16, 64, 8, 100000, 128, True, 1),
+    # one sequence: a split per slot, or a chunk per split
+    (BF16, 1, 8, 8192, 128, False, 64),
+    (F16, 10, 10, 700, 32, False, 6),
+]
+
+
+@pytest.mark.parametrize("case", DECODE, ids=str)
+def test_decode_splits(case):
+    assert _native.lib().co_alibi_decode_splits(*case[:5], int(case[5])) == case[6]
+
+
+def test_decode_splits_bounds():
+    """Every split holds a chunk, at most 1024 of them, for any batch and length; what the scratch of
+    co_alibi_decode_noalloc has to hold (the splits of all units) stays under a round and a rest."""
+    lib = _native.lib()
+    for dtype, D in ((F32, 64), (F16, 32), (F16, 64), (BF16, 128), (BF16, 256)):
+        for units in (1, 2, 7, 36, 100, 128, 210, 256, 257, 384, 426, 427, 448, 511, 512, 513, 4096):
+            for chunks in (1, 2, 3, 4, 5, 6, 7, 8, 9, 16, 17, 100, 1024, 1025, 16384):
+                for ragged in (0, 1):
+                    n = lib.co_alibi_decode_splits(dtype, units, 1, chunks * 128, D, ragged)
+                    assert 1 <= abs(n) <= min(chunks, 1024), (dtype, D, units, chunks, ragged, n)
+                    assert n > 0 or ragged
+                    assert abs(n) * units < 512 + units, (dtype, D, units, chunks, ragged, n)
+    assert lib.co_alibi_decode_splits(F16, 0, 1, 128, 64, 0) == 0
+    assert lib.co_alibi_decode_splits(F16, 1, 1, (1 << 21) + 1, 64, 0) == 0

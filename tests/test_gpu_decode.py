@@ -11,7 +11,8 @@ import math
 import pytest
 import torch
 
-from co_alibi_attn import co_alibi_attention, co_alibi_decode
+from co_alibi_attn import _native, co_alibi_attention, co_alibi_decode
+from co_alibi_attn.co_alibi_attn import _device_slopes
 from oracle import co_alibi_ref as ref
 
 pytestmark = pytest.mark.gpu
@@ -261,3 +262,63 @@ def test_decode_equal_lengths_split_alike(L):
     q, k, v = (t.to(DEV) for t in cache_inputs(3, 8, 2, L, L, 64, torch.bfloat16, seed=7))
     seq = torch.full((3,), L, dtype=torch.int64, device=DEV)
     assert torch.equal(co_alibi_decode(q, k, v, seq_len=seq), co_alibi_decode(q, k, v))
+
+
+# (lens, Hq, Hkv, bound, D, dtype, plan): lengths far below the bound, splits sized by the bound (those past a
+# length hold no key) and by the lengths.
+BOUND_CASES = [
+    ([0, 1, 128, 129, 1000, 4000], 8, 2, 4000, 128, torch.bfloat16, False),
+    ([130, 0, 900], 6, 3, 900, 256, torch.float16, False),
+    ([500, 0, 20, 4000], 16, 16, 4000, 64, torch.float32, True),
+    ([2600, 100, 0] * 6, 8, 8, 2600, 64, torch.float16, True),
+]
+
+
+@pytest.mark.parametrize("case", BOUND_CASES, ids=lambda c: "D{}-{}-{}".format(c[4], str(c[5])[6:], c[6]))
+def test_decode_bound_and_plan(case):
+    lens, Hq, Hkv, L, D, dtype, plan = case
+    print(f"case {case}", flush=True)
+    code = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}[dtype]
+    n = _native.lib().co_alibi_decode_splits(code, len(lens), Hkv, L, D, 1)
+    assert n < -1 if plan else n > 1
+    q, k, v = cache_inputs(len(lens), Hq, Hkv, L, L, D, dtype, seed=41)
+    for b, m in enumerate(lens):
+        k[b, :, m:] = 100.0
+        v[b, :, m:] = -1000.0
+    seq = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    o, lse = co_alibi_decode(q.to(DEV), k.to(DEV), v.to(DEV), seq_len=seq, return_lse=True)
+    torch.cuda.synchronize()
+    for b, m in enumerate(lens[:6]):
+        if m == 0:
+            assert not o[b].any() and torch.isneginf(lse[b]).all()
+            continue
+        ro, rlse = oracle_decode(q[b:b + 1], k[b:b + 1], v[b:b + 1], m)
+        check(f"o[{b}] (len {m})", o[b:b + 1], ro, TOL[dtype])
+        check(f"lse[{b}] (len {m})", lse[b:b + 1], rlse, TOL[dtype])
+
+
+def test_decode_noalloc_plan_past_the_scratch():
+    """A plan whose longest sequences may take four times the even split count (16 of 4096 heads at
+    D 128: 34.3 MB of partials) does not fit the 32 MiB scratch of co_alibi_decode_noalloc and takes half
+    as many."""
+    B, Hq, Hkv, L, D, dtype = 16, 256, 8, 2560, 128, torch.bfloat16
+    lib = _native.lib()
+    assert lib.co_alibi_decode_splits(2, B, Hkv, L, D, 1) == -4
+    lens = [L, 300] + [L - 150 * b for b in range(B - 2)]
+    q, k, v = (t.to(DEV) for t in cache_inputs(B, Hq, Hkv, L, L, D, dtype, seed=43))
+    seq = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    slopes = _device_slopes(Hq, 8.0, dtype, DEV)
+    o = torch.full((B, Hq, D), float("nan"), dtype=dtype, device=DEV)
+    print("noalloc", flush=True)
+    rc = lib.co_alibi_decode_noalloc(2, q.data_ptr(), k.data_ptr(), v.data_ptr(), slopes.data_ptr(), seq.data_ptr(),
+                                     o.data_ptr(), 0, B, Hq, Hkv, L, L, D, 1 / math.sqrt(D),
+                                     torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, lib.co_alibi_last_error()
+    whole = co_alibi_decode(q, k, v, seq_len=seq)
+    torch.cuda.synchronize()
+    check("all heads vs the allocating call", o, whole[:, :, 0].cpu(), TOL[dtype])
+    lam = slopes[:32].cpu()
+    for b in (0, 1, 15):
+        ro, _ = ref.forward(q[b:b + 1, :32].float().cpu(), k[b:b + 1, :1, :lens[b]].float().cpu(),
+                            v[b:b + 1, :1, :lens[b]].float().cpu(), lam, causal=False, scale=1 / math.sqrt(D))
+        check(f"o[{b}]", o[b:b + 1, :32].unsqueeze(2), ro, TOL[dtype])
