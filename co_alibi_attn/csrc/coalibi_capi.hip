@@ -2,12 +2,14 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
 #include <mutex>
 #include <string>
+#include <utility>
 
 #include "../../include/co_alibi.h"
 #include "coalibi_kernels.h"
@@ -92,6 +94,20 @@ int read_layout(const char* fn, const char* name, const long long* strides, int 
     return fail(CO_ALIBI_EINVAL, std::string(fn) + ": the row stride of " + name + " must be in [head_dim, " +
                                      std::to_string(kMaxRowStride) + "]");
   *out = {strides[0], strides[1], static_cast<int>(strides[2])};
+  return CO_ALIBI_OK;
+}
+
+// An output's rows must not overlap: different work-groups write them.  Of the dimensions longer than 1,
+// in order of their strides, each must step past all that the smaller ones cover.
+int check_output(const char* fn, const char* name, const coalibi::Layout& l, int B, int H, int S, int D) {
+  std::array<std::pair<long long, long long>, 3> dims = {{{l.b, B}, {l.h, H}, {l.r, S}}};  // stride, length
+  std::sort(dims.begin(), dims.end());
+  __int128 covered = D;
+  for (const auto& [stride, n] : dims) {
+    if (n == 1) continue;
+    if (stride < covered) return fail(CO_ALIBI_EINVAL, std::string(fn) + ": the rows of " + name + " overlap");
+    covered += static_cast<__int128>(stride) * (n - 1);
+  }
   return CO_ALIBI_OK;
 }
 
@@ -206,7 +222,8 @@ int fwd_impl(const char* fn, int dtype, const void* q, const void* k, const void
   if ((rc = read_layout(fn, "q", st4[0], dtype, heads_q, seq_q, head_dim, &a.ql)) ||
       (rc = read_layout(fn, "k", st4[1], dtype, heads_kv, seq_kv, head_dim, &a.kl)) ||
       (rc = read_layout(fn, "v", st4[2], dtype, heads_kv, seq_kv, head_dim, &a.vl)) ||
-      (rc = read_layout(fn, "o", st4[3], dtype, heads_q, seq_q, head_dim, &a.ol)) || (rc = check_kv_rows(fn, a.kl, a.vl)))
+      (rc = read_layout(fn, "o", st4[3], dtype, heads_q, seq_q, head_dim, &a.ol)) ||
+      (rc = check_output(fn, "o", a.ol, batch, heads_q, seq_q, head_dim)) || (rc = check_kv_rows(fn, a.kl, a.vl)))
     return rc;
   a.q = q;
   a.k = k;
@@ -332,7 +349,9 @@ int bwd_impl(const char* fn, int stages, const long long* strides, int dtype, co
   for (int i = 0; i < 8; ++i) {
     const bool kv = i == 2 || i == 3 || i >= 6;
     if ((rc = read_layout(fn, names[i], strides ? strides + 3 * i : nullptr, dtype, kv ? heads_kv : heads_q,
-                          kv ? seq_kv : seq_q, head_dim, layouts[i])))
+                          kv ? seq_kv : seq_q, head_dim, layouts[i])) ||
+        (i >= 5 && (rc = check_output(fn, names[i], *layouts[i], batch, kv ? heads_kv : heads_q, kv ? seq_kv : seq_q,
+                                      head_dim))))
       return rc;
   }
   if ((rc = check_kv_rows(fn, a.kl, a.vl))) return rc;

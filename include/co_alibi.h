@@ -112,8 +112,10 @@ int co_alibi_fwd_inference(int dtype, const void* q, const void* k, const void* 
 /* Forward on operands in other layouts, as a model's projections leave them ((B, S, H, D) memory,
  * parts of a packed QKV tensor): strides holds the batch, head and row strides in elements of q, k, v
  * and o, in this order (12 values).  A row's head_dim elements are consecutive; strides are whole
- * 16-byte units, row strides at least head_dim and at most 2^20, k's and v's the same.  With stats it is co_alibi_fwd;
- * without (NULL) it is co_alibi_fwd_inference, with its workspace.  lse and stats keep their layouts.
+ * 16-byte units, row strides at least head_dim and at most 2^20, k's and v's the same.  An output's rows
+ * must not overlap: of its dimensions longer than 1, in order of their strides, each steps past all that
+ * the smaller ones cover.  With stats it is co_alibi_fwd; without (NULL) it is
+ * co_alibi_fwd_inference, with its workspace.  lse and stats keep their layouts.
  * The reference's kernels take the strides of q, k, v and o too (co_alibi_attn.py:41-57). */
 int co_alibi_fwd_strided(int dtype, const void* q, const void* k, const void* v, const float* slopes, void* o,
                          const long long* strides, float* lse, float* stats, void* workspace,

@@ -227,3 +227,51 @@ def test_decode_python_checks():
         co_alibi_attn.co_alibi_decode(q[:, :, :1], kc, kc)
     with pytest.raises(AssertionError):
         co_alibi_attn.co_alibi_decode(q[:, :, :1], kc, kc[:, :, :8])
+
+
+def _strided_calls(B, Hq, Hkv, Sq, Skv, D, which, layout):
+    """(fwd rc, bwd rc) of the strided entry points with output `which` in `layout` and every other
+    operand contiguous, except that k's and v's row strides differ, which is refused after the outputs were
+    looked at: no call here reaches a launch (its pointers are not memory)."""
+    import ctypes
+
+    lib = _native.lib()
+    q, kv = [Hq * Sq * D, Sq * D, D], [Hkv * Skv * D, Skv * D, D]
+    bad_v = [2 * x for x in kv]
+    p = 4096
+    fwd = (ctypes.c_longlong * 12)(*q, *kv, *bad_v, *(layout if which == "o" else q))
+    rc = [lib.co_alibi_fwd_strided(1, p, p, p, p, p, fwd, None, None, p, 1 << 40, B, Hq, Hkv, Sq, Skv, D, 1, 0.1, None),
+          lib.co_alibi_last_error()]
+    out = {"dq": q, "dk": kv, "dv": kv}
+    if which != "o":
+        out[which] = layout
+    bwd = (ctypes.c_longlong * 24)(*q, *q, *kv, *bad_v, *q, *out["dq"], *out["dk"], *out["dv"])
+    rc += [lib.co_alibi_bwd_strided(1, *[p] * 11, bwd, p, 1 << 40, B, Hq, Hkv, Sq, Skv, D, 1, 0.1, None),
+           lib.co_alibi_last_error()]
+    return rc
+
+
+# (B, Hq, Hkv, Sq, Skv, D), the output, its batch, head and row strides, whether its rows overlap
+OUTPUT_LAYOUTS = [
+    ((2, 4, 4, 10, 10, 64), "o", (2560, 64, 256), False),   # (B, S, H, D) memory
+    ((2, 4, 4, 10, 10, 64), "o", (7680, 64, 768), False),   # a part of packed (B, S, 3, H, D)
+    ((2, 4, 4, 10, 10, 64), "dq", (64, 1280, 128), False),  # (H, S, B, D) memory
+    ((2, 4, 2, 10, 10, 64), "dk", (0, 640, 64), True),      # one batch written by both
+    ((1, 4, 2, 10, 10, 64), "dk", (0, 640, 64), False),     # the stride of a single batch does not matter
+    ((2, 4, 4, 10, 10, 64), "o", (2560, 0, 64), True),      # every head on the same rows
+    ((2, 4, 4, 10, 10, 64), "dq", (2560, 128, 64), True),   # heads that reach into the next one's rows
+    ((2, 4, 4, 10, 10, 64), "dv", (2552, 640, 64), True),   # batches that do
+    ((2, 1, 1, 10, 10, 64), "o", (640, 0, 64), False),
+    ((2, 4, 4, 10, 10, 64), "o", (2560, 64, 200), True),    # rows shorter than the heads inside them
+    ((3, 4, 4, 1, 1, 64), "o", (256, 64, 64), False),       # one row: its stride does not matter
+    ((2, 2, 2, 2, 2, 64), "o", (1 << 62, 1 << 62, 64), True),
+]
+
+
+@pytest.mark.parametrize("shape,which,layout,overlaps", OUTPUT_LAYOUTS, ids=str)
+def test_strided_outputs_must_not_overlap(shape, which, layout, overlaps):
+    fwd, fwd_msg, bwd, bwd_msg = _strided_calls(*shape, which, layout)
+    assert fwd == 1 and bwd == 1
+    overlap, passed = b"the rows of " + which.encode() + b" overlap", b"k and v must have the same row stride"
+    assert (overlap if overlaps and which == "o" else passed) in fwd_msg
+    assert (overlap if overlaps and which != "o" else passed) in bwd_msg
