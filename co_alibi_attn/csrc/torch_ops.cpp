@@ -78,6 +78,9 @@ bool readable(const Tensor& t) {
 }
 // The operand itself where the kernels can read it in place, else a contiguous aligned copy.
 Tensor in_place(const Tensor& t) { return readable(t) ? t : aligned(t); }
+// An output itself where the kernels can write it in place, else a contiguous tensor to copy from (a
+// packed projection's rows can be further apart than the kernels' 2^20 elements).
+Tensor writable(const Tensor& t) { return readable(t) ? t : at::empty(t.sizes(), t.options()); }
 // K and V, whose row strides must agree.
 std::pair<Tensor, Tensor> kv_in_place(const Tensor& k, const Tensor& v) {
   if (readable(k) && readable(v) && strides_of(k).v[2] == strides_of(v).v[2]) return {k, v};
@@ -109,7 +112,7 @@ hipStream_t current_stream(const Tensor& t) { return c10::hip::getCurrentHIPStre
 
 // ---------------------------------------------------------------------------- forward
 
-// The forward into o (B, Hq, Sq, D in any readable layout); returns lse and stats (empty for inference).
+// The forward into o (B, Hq, Sq, D); returns lse and stats (empty for inference).
 std::tuple<Tensor, Tensor> launch_fwd(const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, const Tensor& slopes,
                                       const Tensor& o, bool causal, double sm_scale, bool with_stats) {
   const int64_t batch = q_in.size(0), heads_q = q_in.size(1), seq_q = q_in.size(2), head_dim = q_in.size(3);
@@ -125,13 +128,15 @@ std::tuple<Tensor, Tensor> launch_fwd(const Tensor& q_in, const Tensor& k_in, co
   const size_t ws_bytes = with_stats ? 0 : co_alibi_fwd_inference_workspace_bytes(batch, heads_q, seq_q, seq_kv);
   Tensor ws;
   if (!with_stats) ws = at::empty({static_cast<int64_t>(ws_bytes)}, q.options().dtype(at::kByte));
-  const auto strides = all_strides<4>({q, k, v, o});
+  const Tensor out = writable(o);
+  const auto strides = all_strides<4>({q, k, v, out});
   check(co_alibi_fwd_strided(dtype_code(q.scalar_type()), q.data_ptr(), k.data_ptr(), v.data_ptr(),
-                             sl.data_ptr<float>(), o.data_ptr(), strides.data(),
+                             sl.data_ptr<float>(), out.data_ptr(), strides.data(),
                              with_stats ? lse.data_ptr<float>() : nullptr,
                              with_stats ? stats.data_ptr<float>() : nullptr, with_stats ? nullptr : ws.data_ptr(),
                              ws_bytes, batch, heads_q, heads_kv, seq_q, seq_kv, head_dim, causal ? 1 : 0,
                              static_cast<float>(sm_scale), current_stream(q)));
+  if (!out.is_same(o)) o.copy_(out);
   return {lse, stats};
 }
 
@@ -206,11 +211,15 @@ void launch_bwd(int stages, const Tensor& do_in, const Tensor& q_in, const Tenso
     if (ws.defined()) {
       const Tensor q = in_place(q_in), o = in_place(o_in), dout = in_place(do_t);
       const auto [k, v] = kv_in_place(k_in, v_in);
-      const auto strides = all_strides<8>({dout, q, k, v, o, dq, dk, dv});
+      const std::array<Tensor, 3> to = {dq, dk, dv}, out = {writable(dq), writable(dk), writable(dv)};
+      const auto strides = all_strides<8>({dout, q, k, v, o, out[0], out[1], out[2]});
       check(co_alibi_bwd_strided(code, dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
-                                 lse.data_ptr<float>(), stats.data_ptr<float>(), sl.data_ptr<float>(), dq.data_ptr(),
-                                 dk.data_ptr(), dv.data_ptr(), strides.data(), ws.data_ptr(), store_bytes, batch,
-                                 heads_q, heads_kv, seq_q, seq_kv, head_dim, causal_i, scale, st));
+                                 lse.data_ptr<float>(), stats.data_ptr<float>(), sl.data_ptr<float>(),
+                                 out[0].data_ptr(), out[1].data_ptr(), out[2].data_ptr(), strides.data(),
+                                 ws.data_ptr(), store_bytes, batch, heads_q, heads_kv, seq_q, seq_kv, head_dim,
+                                 causal_i, scale, st));
+      for (int i = 0; i < 3; ++i)
+        if (!out[i].is_same(to[i])) to[i].copy_(out[i]);
       return;
     }
   }

@@ -50,6 +50,16 @@ def test_packed_qkv_equals_contiguous(case):
         assert torch.equal(co_alibi_attention_qkv(qkv, causal=causal), o)
 
 
+@pytest.mark.parametrize("case", [(1, 3, 4200, 256, torch.bfloat16), (2, 2, 2800, 128, torch.float16)],
+                         ids=["output", "gradient"])
+def test_packed_rows_past_the_stride_limit(case):
+    """Packed rows of more elements than the kernels' largest row stride (2^20): the output's (4200 heads of
+    256) or only the gradient's (2800 of 128) are then written through a copy."""
+    B, S, H, D, dtype = case
+    assert 3 * H * D > 1 << 20
+    test_packed_qkv_equals_contiguous((B, S, H, D, dtype, True))
+
+
 def layouts(x):
     """The values of contiguous (B, H, S, D) x in layouts that are read in place, then in ones that are copied."""
     B, H, S, D = x.shape
