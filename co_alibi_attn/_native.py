@@ -36,6 +36,7 @@ EXPORTS = (
     "co_alibi_bwd_strided",
     "co_alibi_bwd_dq",
     "co_alibi_bwd_dkdv",
+    "co_alibi_attention_forms",
     "co_alibi_decode_workspace_bytes",
     "co_alibi_decode_splits",
     "co_alibi_decode",
@@ -80,6 +81,7 @@ _SIGNATURES = {
         _I,
         [_I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _Z, _I, _I, _I, _I, _I, _I, _I, _F, _P],
     ),
+    "co_alibi_attention_forms": (_I, [_I] * 8),
     "co_alibi_decode_workspace_bytes": (_Z, [_I, _I, _I, _I]),
     "co_alibi_decode_splits": (_I, [_I, _I, _I, _I, _I, _I]),
     "co_alibi_decode": (_I, [_I, _P, _P, _P, _P, _P, _P, _P, _P, _Z, _I, _I, _I, _I, _I, _I, _F, _P]),

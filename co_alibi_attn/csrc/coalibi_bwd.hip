@@ -422,9 +422,6 @@ __global__ __launch_bounds__(256, (sizeof(T) == 4 || D > 128) ? 1 : 2) void coal
 // sigmoid totals (z at a tile's start = z at the step's start minus the totals left of it) and
 // their dA totals (C likewise).  Both are taken off / added in tile order, so s, dA, dP and the
 // records are bit for bit those of the whole-block form.  dQ is the sum of the four wavefronts'.
-constexpr int kSplitRows = 32;
-constexpr int kSplitWaves = 4;
-
 template <typename T, int D>
 struct SplitDqCfg {
   static constexpr bool kTr = sizeof(T) == 2;
@@ -443,7 +440,8 @@ struct SplitDqCfg {
   static_assert(16 * LDO * 4 <= K_ELEMS * (int)sizeof(T) && 16 * LDO * 4 <= V_ELEMS * (int)sizeof(T),
                 "dQ partials alias the tiles");
   // fp32 at D = 256 does not fit a CU's LDS.
-  static constexpr bool kFits = (size_t)kSplitWaves * (K_ELEMS + V_ELEMS) * sizeof(T) <= 155 * 1024;
+  static constexpr bool kFits = split_fits(sizeof(T), D);
+  static_assert(!kFits || (size_t)kSplitWaves * (K_ELEMS + V_ELEMS) * sizeof(T) <= 155 * 1024, "the tiles fit a CU");
 };
 
 template <typename T, int D, bool CAUSAL, bool STORE>
@@ -666,25 +664,6 @@ __global__ __launch_bounds__(256, D * sizeof(T) > 256 ? 1 : 2) void coalibi_bwd_
       *reinterpret_cast<vec4*>(dQr + c) = __builtin_convertvector(v * args.sm_scale, vec4);
     }
   }
-}
-
-// Whether pass 1 takes the split form.  As in the forward (split_grid) it wins where the row blocks
-// leave the GPU room.  At D = 128 in 16-bit types a step waits longer for its own K, whose tile the
-// dQ product reads last, and the limit is lower.  us, whole-block form -> split, fp16 (f = tail
-// skip off):
-//   D 64   n 512: 128 blocks 25.0 -> 17.2 f 25.0 -> 14.5, 192: 25.0 -> 22.1, 256: 25.9 -> 26.7
-//          n 1024: 128 blocks 44.1 -> 21.7, 320: 46.2 -> 36.0 f 46.0 -> 42.8, 384: 46.7 -> 41.0 f 46.7 -> 47.3
-//          n 2048: 128 blocks 82.6 -> 36.9, 384: 84.8 -> 52.4 f 88.2 -> 75.5, 512: 86.1 -> 67.7 f 89.3 -> 95.9
-//   D 128  n 512: 128 blocks 31.3 -> 27.8 f 30.1 -> 23.5, 192: 32.4 -> 34.7
-//          n 1024: 128 blocks 53.8 -> 41.3 f 52.3 -> 37.5, 256: 55.2 -> 55.3
-//          n 2048: 128 blocks 98.2 -> 72.7 f 97.1 -> 69.1, 256: 99.3 -> 82.4 f 100.2 -> 84.7, 320: f 103.3 -> 114.0
-//   non-causal, D 128: 333 x 2047, 96 blocks 103.4 -> 67.7; 2000 x 3000, 256 blocks f 158.0 -> 195.3;
-//          D 64, 1400 x 1400, 352 blocks 64.1 -> 49.5
-//   fp32   D 64: n 1000, 192 blocks 133.9 -> 74.6;  D 128: n 1024, 128 blocks 240.5 -> 109.6
-template <typename T, int D>
-inline bool split_dq_grid(long long row_blocks, int keys, bool causal) {
-  if (sizeof(T) == 2 && D >= 128) return row_blocks <= (causal ? std::max(128, std::min(keys / 5, 256)) : 128);
-  return row_blocks <= std::max(128, causal ? std::min(keys / 3, 384) : std::min(keys / 4, 320));
 }
 
 // Pass 2's rotation of the heads over the XCDs (balanced_item): runs of kLptRotateRanks key
@@ -984,22 +963,6 @@ struct KeyCfg {
   static constexpr int KS = D / 16;
   static constexpr int DT = DP / 32;
 };
-
-// Which form of the recompute path's pass 2 a launch takes (16-bit types at D >= 64 have their own
-// kernel).  The 32-key form wins where the 128-key blocks are few, and where a wavefront's walk (a
-// tile per row block and query head) is long enough to carry its prologue and merge; in 16-bit types
-// the 128-key form is ahead again once its work-groups fill the GPU.  us, 128-key -> 32-key:
-//   fp32 D 64: B1 H2 n 128 31 -> 12, B2 H12 n 1000 213 -> 100, B4 H16 n 2048 806 -> 755, Hq16/Hkv4
-//     n 2000 1593 -> 388, B8 H32 n 300 137 -> 170;  D 32: B4 H16 n 2048 364 -> 337
-//   fp16 D 32: B8 H8 n 512 (256 blocks) 27 -> 20, B2 H16 n 2048 (512) 101 -> 81, B16 H16 n 256 (512)
-//     17 -> 27, B2 H16 n 3000 (768) 147 -> 157, B4 H16 n 2048 (1024) 112 -> 122
-template <typename T, int D>
-constexpr bool kHasKeyForm = D * sizeof(T) <= (sizeof(T) == 2 ? 64 : 256);
-template <typename T>
-inline bool use_key_form(long long key_blocks, int tiles) {
-  if (key_blocks <= 256) return true;
-  return tiles >= 8 && (sizeof(T) == 4 || key_blocks <= 640);
-}
 
 template <typename T, int D, bool CAUSAL>
 __global__ __launch_bounds__(256, D * sizeof(T) > 128 ? 1 : 2) void coalibi_bwd_dkdv_key_kernel(BwdArgs args) {
@@ -1805,7 +1768,7 @@ hipError_t launch_bwd(const BwdArgs& a, int stages, hipStream_t stream) {
     const int nQB = (a.Sq + kBM - 1) / kBM, blocks = nQB * a.B * a.Hq;
     bool split = false;
     if constexpr (SplitDqCfg<T, D>::kFits) {
-      split = split_dq_grid<T, D>(blocks, a.Skv, CAUSAL);
+      split = split_dq_grid(sizeof(T), D, blocks, CAUSAL ? std::min(a.Sq, a.Skv) : a.Skv, CAUSAL);
       const dim3 parts((blocks + 7) / 8 * 32);
       if (split && store) {
         if constexpr (kStore)
@@ -1847,9 +1810,9 @@ hipError_t launch_bwd(const BwdArgs& a, int stages, hipStream_t stream) {
     } else {
       const int nKB = (a.Skv + kBK - 1) / kBK;
       bool key_form = false;
-      if constexpr (kHasKeyForm<T, D>) {
-        key_form = use_key_form<T>(static_cast<long long>(nKB) * a.B * a.Hkv,
-                                   a.Hq / a.Hkv * ((a.Sq + kSkipRows - 1) / kSkipRows));
+      if constexpr (has_key_form(sizeof(T), D)) {
+        key_form = use_key_form(sizeof(T), D, static_cast<long long>(nKB) * a.B * a.Hkv,
+                                a.Hq / a.Hkv * ((a.Sq + kSkipRows - 1) / kSkipRows));
         if (key_form)
           hipLaunchKernelGGL((coalibi_bwd_dkdv_key_kernel<T, D, CAUSAL>),
                              dim3((a.Skv + kWaveKeys - 1) / kWaveKeys * a.B * a.Hkv), dim3(256), 0, stream, a);

@@ -173,6 +173,26 @@ size_t co_alibi_bwd_workspace_bytes(int batch, int heads_q, int seq_q, int seq_k
          2 * round_up(block_sums_numel(batch, heads_q, seq_q, seq_kv) * sizeof(float), 256);
 }
 
+int co_alibi_attention_forms(int dtype, int batch, int heads_q, int heads_kv, int seq_q, int seq_kv, int head_dim,
+                             int causal) {
+  if (check_shape("co_alibi_attention_forms", dtype, {batch, heads_q, heads_kv, seq_q, seq_kv, head_dim})) return -1;
+  const int elem = dtype == CO_ALIBI_F32 ? 4 : 2, row_tiles = (seq_q + coalibi::kSkipRows - 1) / coalibi::kSkipRows;
+  const int keys = causal ? std::min(seq_q, seq_kv) : seq_kv;
+  const long long row_blocks = static_cast<long long>(row_tiles) * batch * heads_q;
+  const bool every_key = g_tail_skip.load() == 0, fits = coalibi::split_fits(elem, head_dim);
+  int forms = 0;
+  if (fits && coalibi::split_fwd_grid(elem, head_dim, row_blocks, keys, causal != 0, every_key))
+    forms |= CO_ALIBI_FORM_FWD_SPLIT;
+  else if (fits && causal && !every_key && coalibi::split_fwd_long_rows(elem, head_dim, row_blocks, keys))
+    forms |= CO_ALIBI_FORM_FWD_LONG_ROWS;
+  if (fits && coalibi::split_dq_grid(elem, head_dim, row_blocks, keys, causal != 0)) forms |= CO_ALIBI_FORM_DQ_SPLIT;
+  if (coalibi::has_key_form(elem, head_dim) &&
+      coalibi::use_key_form(elem, head_dim, static_cast<long long>((seq_kv + 127) / 128) * batch * heads_kv,
+                            heads_q / heads_kv * row_tiles))
+    forms |= CO_ALIBI_FORM_DKDV_KEYS;
+  return forms;
+}
+
 int co_alibi_set_tail_skip(int enabled) { return g_tail_skip.exchange(enabled != 0 ? 1 : 0); }
 
 int co_alibi_tail_skip(void) { return g_tail_skip.load(); }

@@ -511,6 +511,9 @@ __device__ __forceinline__ float sum8(f32x8 v, float acc) {
 namespace coalibi {
 
 constexpr int kWaveKeys = 32;  // keys per wavefront: one 32-key MFMA tile
+// The split forms: query rows per work-group, and key tiles (wavefronts) per step.
+constexpr int kSplitRows = 32;
+constexpr int kSplitWaves = 4;
 
 // Buffer-to-LDS DMA of the kWaveKeys rows row0.. of a row-major [nrows][D] matrix into
 // one wavefront's tile (the layout of DmaTile<T, D, kWaveKeys, LD, 1, PERM>): every

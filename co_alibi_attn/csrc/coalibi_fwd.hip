@@ -630,8 +630,6 @@ __global__ __launch_bounds__(256, D * sizeof(T) > 256 ? 1 : 2) void coalibi_fwd_
 //   Per step each wavefront computes its tile's S^T and sigmoids; the tiles' sigmoid totals go
 // through LDS (one barrier), so that z is absolute in every wavefront; the softmax state is a
 // wavefront's own and the four are combined at the end.
-constexpr int kSplitRows = 32;   // rows per work-group
-constexpr int kSplitWaves = 4;   // key tiles per step
 
 template <typename T, int D>
 struct SplitCfg {
@@ -655,7 +653,8 @@ struct SplitCfg {
                 "the 64-key tiles fit");
   static constexpr size_t kLds = (size_t)kSplitWaves * (K_ELEMS + V_ELEMS) * sizeof(T);
   // fp32 at D = 256 takes 266 KB, above a CU's 160.
-  static constexpr bool kFits = kLds <= 155 * 1024;
+  static constexpr bool kFits = split_fits(sizeof(T), D);
+  static_assert(!kFits || kLds <= 155 * 1024, "the tiles fit a CU");
 };
 
 // Which row blocks a launch splits: those of `keys` visible keys, longer than `longer_than`, of a head
@@ -904,33 +903,6 @@ __global__ __launch_bounds__(256, D * sizeof(T) > 256 ? 1 : 2) void coalibi_fwd_
   }
 }
 
-// Whether the split form is launched.  It wins where the row blocks leave the GPU room, and longer
-// walks leave more of it (causal: half the work of the longest block on average, and the short
-// blocks' work-groups cost their prologue and merge all the same).  us, whole-block form ->
-// split, fp16 (f = tail skip off):
-//   D 128  n 256: 64 blocks 19.5 -> 14.2 f 13.1 -> 9.8, 128: 19.8 -> 16.1 f 13.3 -> 11.6
-//          n 512: 64 blocks 27.1 -> 20.5 f 20.1 -> 13.3, 128: 27.4 -> 22.2 f 20.3 -> 14.9, 192: f 20.8 -> 22.1
-//          n 1024: 128 blocks 43.1 -> 27.4 f 34.2 -> 22.1, 256: 44.5 -> 39.5 f 35.4 -> 34.3, 320: f 37.5 -> 41.1
-//          n 2048: 128 blocks 74.0 -> 40.1 f 61.7 -> 36.5, 256: 75.4 -> 49.7 f 62.6 -> 54.1, 320: 77.7 -> 49.2 f 65.5 -> 65.6
-//   D 64   n 512: 128 blocks 21.5 -> 16.2 f 15.0 -> 10.8
-//          n 1024: 256 blocks 34.2 -> 27.9 f 25.3 -> 22.2;  n 2048: 320 blocks 59.1 -> 36.9 f 46.0 -> 40.9
-//   non-causal, D 128: 333 x 2047, 96 blocks 90.5 -> 41.3; 2000 x 3000, 256 blocks 126.2 -> 69.0;
-//          D 64, 1400 x 1400, 352 blocks 43.8 -> 51.8
-//   fp32   D 64: n 1000, 192 blocks 94.7 -> 56.9;  D 128: n 1024, 128 blocks 160.1 -> 73.1
-inline bool split_grid(long long row_blocks, int keys, bool causal) {
-  return row_blocks <= std::max(128, causal ? std::min(keys / 4, 384) : std::min(keys / 8, 256));
-}
-
-// Beyond those grids (causal, tail skip on), whether only the longer half of the row blocks is split:
-// the flat heads' last blocks otherwise walk on alone after the rest.  us, whole-block form -> split:
-//   Hq32/Hkv8 n 1741 D128 bf16 (448 blocks) 70.7 -> 59.1; n 2048 D128 H32 (512) 80.9 -> 67.0, D64 62.4 ->
-//   55.3, H48 D64 (768) 65.6 -> 62.7, H64 D128 (1024) 90.1 -> 113.4; n 4096 H16 D128 (512) 142.2 -> 109.1,
-//   H24 D64 (768) 111.2 -> 93.2; n 1024 H64 D64 39.2 -> 40.8; n 8192 H8 D64 (512) 144.1 -> 148.9;
-//   skip off, every head's longer half: n 2048 H32 D128 70.5 -> 97.1
-inline bool split_long_rows(long long row_blocks, int keys) {
-  return row_blocks <= 768 && keys >= 1536 && keys <= 4096;
-}
-
 }  // namespace
 
 template <typename T, int D, bool CAUSAL>
@@ -961,10 +933,11 @@ hipError_t launch_fwd(const FwdArgs& a, hipStream_t stream) {
   const int grid = nQB * a.B * a.Hq;
   if constexpr (SplitCfg<T, D>::kFits) {
     const float window = a.every_key ? __builtin_inff() : order_window<T>();
-    const bool small = split_grid(grid, a.Skv, CAUSAL);
-    if (small || (CAUSAL && !a.every_key && split_long_rows(grid, a.Skv))) {
+    const int keys = CAUSAL ? std::min(a.Sq, a.Skv) : a.Skv;
+    const bool small = split_fwd_grid(sizeof(T), D, grid, keys, CAUSAL, a.every_key);
+    if (small || (CAUSAL && !a.every_key && split_fwd_long_rows(sizeof(T), D, grid, keys))) {
       const dim3 parts((grid + 7) / 8 * 32);
-      const SplitRule rule = small ? SplitRule{window, 3.0f, 192.0f, 0} : SplitRule{window, 1.25f, 0.0f, a.Skv / 2};
+      const SplitRule rule = small ? SplitRule{window, 3.0f, 192.0f, 0} : SplitRule{window, 1.25f, 0.0f, keys / 2};
       auto* const kernel = a.knorm != nullptr ? coalibi_fwd_split_kernel<T, D, CAUSAL, true>
                                               : coalibi_fwd_split_kernel<T, D, CAUSAL, false>;
       hipLaunchKernelGGL(kernel, parts, dim3(256), 0, stream, f, grid, rule, small);

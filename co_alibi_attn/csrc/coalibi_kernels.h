@@ -1,6 +1,7 @@
 // Launch interface between the C ABI layer and the gfx950 kernels.
 #pragma once
 
+#include <algorithm>
 #include <hip/hip_runtime.h>
 
 namespace coalibi {
@@ -245,6 +246,99 @@ __host__ __device__ inline int decode_cps(long long work, int longest, int slots
   for (int c = c0; c <= (c1 < most ? c1 : most); c += 1 + c / 16)
     if (groups(c) <= slots) return c;
   return c0;
+}
+
+// Which kernel forms a call takes, from its element bytes, head dim, 128-row blocks (batch * heads_q *
+// ceil(seq_q / 128)) and the most keys a row sees (`keys`).  The split forms win where the row blocks leave
+// the GPU room, and longer walks leave more of it (causal: half the work of the longest block on average,
+// and the short blocks' work-groups cost their prologue and merge all the same); they lose K and V reads (four
+// times as many from L2) and, in training, the tail skip's record: both backward passes walk every key of a
+// split block.  `every_key`: the tail skip is switched off.
+//   Types of more than 256 bytes a row (fp32 at D 128, 16 bits at D 256) have one work-group per CU in the split
+// forms, two in the others, so they fill the GPU at half the blocks; their split forms do not fit LDS
+// above 512 bytes.
+//   Figures: us by hipGraph replay, whole-block form -> split, forward alone / forward and backward with the
+// rules' choice for the other launches; f: tail skip off.
+constexpr bool split_fits(int elem, int D) { return D * elem <= 512; }
+
+// Forward.
+//   fp16 D 128  n 64: 64 blocks 12.7 -> 13.1, 128 13.0 -> 15.8;  n 96: 128 15.8 -> 16.0;  n 128: 128 16.8 -> 16.3
+//          n 256: 64 blocks 20.8 -> 15.6 / 52 -> 41, 128 21.0 -> 17.0 / 54 -> 49;  n 512: 128 28.6 -> 23.1 / 78 -> 68
+//          n 1024: 128 blocks 44.0 -> 28.0 / 123 -> 92, 256 45.4 -> 40.8 / 133 -> 130 f 36.7 -> 35.2
+//          n 2048: 128 blocks 75.6 -> 41.0 / 216 -> 146, 384 78.1 -> 60.3 / 235 -> 218 f 68.5 -> 73.2, 320 f 66.7 -> 66.3
+//   fp16 D 64   n 64: 128 blocks 10.4 -> 11.7;  n 512: 128 22.6 -> 17.6 / 61 -> 46;  n 1024: 256 34.5 -> 28.2 / 105 -> 87
+//          n 2048: 384 blocks 60.4 -> 41.9 / 191 -> 148 f 48.0 -> 48.1
+//   fp32 D 64   n 64: 64 blocks 14.7 -> 13.0, 128 15.1 -> 16.3;  n 1024: 256 93.8 -> 76.8;  n 2048: 384 175 -> 156 / 659 -> 619
+//   fp32 D 128  n 1024: 256 blocks 167 -> 144;  n 1536: 288 240 -> 205, 384 243 -> 267;  n 2048: 352 313 -> 226, 384 315 -> 329
+//   fp16 D 256  n 128: 64 blocks 27.1 -> 20.1, 128 29.4 -> 32.0;  n 192: 128 30.2 -> 31.7;  n 256: 128 38.0 -> 34.8
+//          n 1024: 224 blocks 91 -> 81, 256 94 -> 99 / 255 -> 269;  n 1536: 288 128 -> 118 / 345 -> 338, 384 131 -> 154 / 382 -> 422
+//          n 2048: 352 blocks 159 -> 127 f 256: 142 -> 124, 320: 144 -> 159;  n 4096: 384 296 -> 183 f 272 -> 317
+//   non-causal  fp16 D 128 333 x 2047: 96 blocks 89.5 -> 42.1 / 232 -> 154;  n 2048: 128 f 73 -> 48, 192 f 74 -> 74, 256 88 -> 58 f 76 -> 85
+//          fp16 D 64 n 2048: 128 blocks f 46 -> 38, 160 f 47 -> 54, 256 56 -> 41 f 48 -> 67;  fp32 D 128: 192 f 304 -> 292, 224 f 308 -> 381
+//          fp16 D 256 n 2048: 256 blocks 304 -> 163 f 358 -> 209 (the whole-block form spills);  1024 x 64: 128 35 -> 31
+inline bool split_fwd_grid(int elem, int D, long long row_blocks, int keys, bool causal, bool every_key) {
+  const bool fp32 = elem == 4, wide = D * elem > 256;
+  if (wide && !fp32) {
+    const int least = causal && keys < 256 ? 64 : 128;
+    if (!causal) return row_blocks <= std::max(least, std::min(keys / 8, 256));
+    return row_blocks <= std::max(least, std::min(keys / 5, every_key ? 256 : 352));
+  }
+  if (keys <= 64) return row_blocks <= (fp32 ? 64 : 0);
+  const int most = causal ? (wide ? 320 : every_key && D > 64 ? 320 : 384) : every_key ? (fp32 ? 192 : 128) : 256;
+  return row_blocks <= std::max(128, std::min(causal ? keys / 4 : keys / 8, most));
+}
+
+// Forward beyond those grids (causal, tail skip on): whether only the longer half of the row blocks is split.
+// The flat heads' last blocks otherwise walk on alone after the rest.
+//   fp16 D 128  n 1536: 576 blocks 66.7 -> 63.0, 696 68.0 -> 67.7, 768 68.2 -> 75.2 / 234 -> 243;  n 1741 (448, bf16) 70.5 -> 58.6
+//          n 2048: 512 blocks 81.2 -> 68.5 / 251 -> 239, 768 83.7 -> 76.7, 1024 90.1 -> 113.4;  n 4096: 768 144 -> 118 / 451 -> 425
+//   fp16 D 64   n 1536: 576 blocks 50.6 -> 44.4, 768 52.1 -> 56.9;  n 2048: 768 64.0 -> 62.4;  n 4096: 768 110 -> 93;  n 8192: 512 144 -> 149
+//   fp32 D 64   n 1536: 480 blocks 137 -> 130, 576 139 -> 150;  n 2048: 512 180 -> 176, 640 180 -> 192;  n 4096: 640 342 -> 342, 704 342 -> 362
+//   fp16 D 256  n 1536: 336 blocks 130 -> 105;  n 2048: 448 164 -> 136, 512 170 -> 170, 768 175 -> 205;  n 3072: 576 237 -> 186, 768 242 -> 281
+//   fp32 D 128  n 1536: 360 blocks 242 -> 216, 576 248 -> 270;  n 2048: 416 316 -> 262, 512 321 -> 344;  n 3072: 576 470 -> 369, 672 475 -> 495
+inline bool split_fwd_long_rows(int elem, int D, long long row_blocks, int keys) {
+  if (keys < 1536 || keys > 4096) return false;
+  if (D * elem > 256) return row_blocks <= std::min(keys / 5, 768);
+  if (elem == 4 && D > 32) return row_blocks <= std::min(keys / 4, 640);
+  return row_blocks <= std::min(keys * 2 / 5, 768);
+}
+
+// Backward pass 1.  At D = 128 in 16-bit types a step waits longer for its own K, whose tile the dQ product
+// reads last (and reloads spilled registers), and the limit is lower.  Both passes, pass 1 whole -> split:
+//   fp16 D 64   n 64: 64 blocks 11.9 -> 12.7;  n 96: 64 15.5 -> 14.5, 128 16.1 -> 17.6;  n 128: 128 17.8 -> 17.3;  n 256: 128 25.0 -> 21.3
+//          n 1024: 256 blocks 70 -> 57;  n 2048: 384 130 -> 102;  non-causal n 2048: 256 126 -> 114, f 224 134 -> 134
+//   fp16 D 128  n 96: 128 blocks 21.4 -> 25.8;  n 128: 96 24.0 -> 26.6;  n 192: 96 26.0 -> 29.4;  n 256: 128 33.3 -> 32.1;  n 1024: 192 84 -> 74, 256 87 -> 84
+//          n 2048: 256 blocks 149 -> 125, 320 (f) 103 -> 114 (pass 1 alone);  non-causal n 2048: 128 f 141 -> 118, 144 to 256 +13 to 18 %
+//   fp16 D 256  n 128: 96 blocks 41.8 -> 52.1;  n 256: 64 55 -> 47, 128 58 -> 64;  n 512: 128 87 -> 85;  n 1024: 128 150 -> 130, 192 152 -> 151
+//          n 2048: 192 blocks 274 -> 231, 256 278 -> 274, 384 284 -> 320;  non-causal n 2048: 128 294 -> 277, 192 f +6 %
+//   fp32 D 64   n 32: 64 blocks 21.3 -> 23.6;  n 64: 64 26.4 -> 25.0, 128 27.4 -> 32.2;  n 1024: 256 264 -> 218;  n 2048: 384 482 -> 399
+//   fp32 D 128  n 1024: 256 blocks 736 -> 658;  n 2048: 384 1435 -> 1328;  non-causal n 2048: 192 f 1404 -> 1327, 224 f 1409 -> 1458
+inline bool split_dq_grid(int elem, int D, long long row_blocks, int keys, bool causal) {
+  if (elem == 4) {
+    if (keys <= 64) return row_blocks <= (keys <= 32 ? 0 : 64);
+    return row_blocks <= std::max(128, causal ? std::min(keys / 3, 384) : std::min(keys / 4, D > 64 ? 192 : 320));
+  }
+  if (keys <= 64) return false;
+  const int least = keys < (D > 128 ? 512 : D > 64 ? 256 : 128) ? 64 : 128;
+  if (D <= 64) return row_blocks <= std::max(least, causal ? std::min(keys / 3, 384) : std::min(keys / 4, 320));
+  if (!causal) return row_blocks <= least;
+  return row_blocks <= std::max(least, D > 128 ? std::min(keys / 8, 224) : std::min(keys / 5, 256));
+}
+
+// Backward pass 2, recompute path: the 32-key form, for fp32 at D <= 64 and 16-bit types at D <= 32 (16-bit types at
+// D >= 64 have their own kernel).  It wins where the 128-key blocks are few, and where a wavefront's walk (a tile per
+// row block and query head) is long enough to carry its prologue and merge; in 16-bit types the 128-key form
+// is ahead again once its work-groups fill the GPU.  Both passes, 128-key -> 32-key, by key blocks and tiles:
+//   fp32 D 64   128 x 1: 52.6 -> 45.1, 192 x 1 62 -> 74, 256 x 1 65 -> 96, 256 x 2 100 -> 101 (non-causal 99 -> 111), 256 x 4 180 -> 155
+//          384 x 8: 344 -> 308, 512 x 8 397 -> 414, 512 x 4 248 -> 272, 640 x 16 708 -> 645, 1024 x 16 1194 -> 1153, 64 x 64 1761 -> 551
+//   fp32 D 32   192 x 1: 41 -> 44, 256 x 2 64 -> 56, 512 x 8 249 -> 218, 1024 x 16 567 -> 538
+//   fp16 D 32   128 x 1: 17.3 -> 14.2, 192 x 1 23 -> 29, 256 x 2 29.4 -> 28.4, 256 x 4 49 -> 40, 512 x 4 52 -> 59, 512 x 8 89 -> 83
+//          640 x 16: 164 -> 129, 1024 x 16 175 -> 188, 768 x 3 51 -> 64
+constexpr bool has_key_form(int elem, int D) { return D * elem <= (elem == 2 ? 64 : 256); }
+inline bool use_key_form(int elem, int D, long long key_blocks, int tiles) {
+  if (key_blocks <= 128) return true;
+  if (key_blocks <= 256) return tiles >= (elem == 4 && D > 32 ? 3 : 2);
+  return tiles >= 8 && (elem == 4 || key_blocks <= 640);
 }
 
 // Forward; with a.knorm (the tail skip) it first launches the key-norm kernel that fills it.

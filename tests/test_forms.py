@@ -68,3 +68,94 @@ def test_decode_splits_bounds():
                     assert abs(n) * units < 512 + units, (dtype, D, units, chunks, ragged, n)
     assert lib.co_alibi_decode_splits(F16, 0, 1, 128, 64, 0) == 0
     assert lib.co_alibi_decode_splits(F16, 1, 1, (1 << 21) + 1, 64, 0) == 0
+
+
+SPLIT, LONG, DQ, KEYS = 1, 2, 4, 8
+
+
+def _forms(dtype, H, n, m, D, causal, B=1, group=1):
+    return _native.lib().co_alibi_attention_forms(dtype, B, H * group, H, n, m, D, int(causal))
+
+
+# (dtype, heads, seq_q, seq_kv, head_dim, causal, forms with the tail skip, forward's without it)
+ATTENTION = [
+    # the longest walk is one tile: nothing to split
+    (F16, 128, 64, 64, 64, True, 0, 0),
+    (F16, 2, 33, 31, 64, True, 0, 0),
+    (F16, 16, 1024, 64, 128, False, 0, 0),
+    (F32, 64, 64, 64, 64, True, SPLIT | DQ | KEYS, SPLIT),
+    (F32, 128, 64, 64, 64, True, KEYS, 0),
+    (F32, 64, 32, 32, 64, True, SPLIT | KEYS, SPLIT),
+    (BF16, 64, 64, 64, 256, True, SPLIT, SPLIT),
+    # short walks
+    (F16, 128, 128, 128, 128, True, SPLIT, SPLIT),
+    (F16, 64, 128, 128, 128, True, SPLIT | DQ, SPLIT),
+    (F16, 128, 128, 128, 64, True, SPLIT | DQ, SPLIT),
+    (F16, 128, 96, 96, 64, True, SPLIT, SPLIT),
+    (F16, 128, 128, 128, 256, True, 0, 0),
+    (F16, 64, 128, 128, 256, True, SPLIT | DQ, SPLIT),
+    (F16, 64, 256, 256, 256, True, SPLIT, SPLIT),
+    (F16, 64, 256, 256, 128, True, SPLIT | DQ, SPLIT),
+    # one work-group per CU: 16 bits at D 256 and fp32 at D 128
+    (F16, 24, 1024, 1024, 256, True, SPLIT, SPLIT),
+    (F16, 32, 1024, 1024, 256, True, 0, 0),
+    (BF16, 32, 1024, 1024, 256, True, 0, 0),
+    (F16, 32, 1536, 1536, 256, True, 0, 0),
+    (F16, 24, 1536, 1536, 256, True, SPLIT, 0),
+    (F16, 22, 2048, 2048, 256, True, SPLIT, 0),
+    (F16, 24, 2048, 2048, 256, True, LONG, 0),
+    (F16, 48, 2048, 2048, 256, True, 0, 0),
+    (F32, 32, 1024, 1024, 128, True, SPLIT | DQ, SPLIT),
+    (F32, 32, 1536, 1536, 128, True, DQ, 0),
+    (F32, 24, 2048, 2048, 128, True, LONG | DQ, 0),
+    (F32, 32, 2048, 2048, 128, True, 0, 0),
+    (F32, 16, 2048, 2048, 128, False, SPLIT, 0),
+    (F32, 12, 2048, 2048, 128, False, SPLIT | DQ, SPLIT),
+    # two per CU
+    (F16, 32, 1024, 1024, 128, True, SPLIT, SPLIT),
+    (F16, 24, 2048, 2048, 128, True, SPLIT, 0),
+    (F16, 24, 2048, 2048, 64, True, SPLIT | DQ, SPLIT),
+    (F16, 16, 2048, 2048, 64, False, SPLIT | DQ, 0),
+    (F16, 8, 2048, 2048, 64, False, SPLIT | DQ, SPLIT),
+    (F16, 16, 2048, 2048, 128, False, SPLIT, 0),
+    (F32, 16, 2048, 2048, 64, False, SPLIT | DQ | KEYS, 0),
+    # middle grids
+    (F16, 64, 1536, 1536, 128, True, 0, 0),
+    (F16, 48, 1536, 1536, 128, True, LONG, 0),
+    (F16, 48, 2048, 2048, 64, True, LONG, 0),
+    (F32, 48, 1536, 1536, 64, True, KEYS, 0),
+    (F32, 32, 2048, 2048, 64, True, LONG | KEYS, 0),
+    (F32, 40, 2048, 2048, 64, True, KEYS, 0),
+    (F16, 64, 2048, 2048, 128, True, 0, 0),
+    (F16, 8, 8192, 8192, 64, True, 0, 0),
+    # causal rows see at most seq_q keys, however many there are
+    (F16, 32, 1024, 8192, 128, True, SPLIT, SPLIT),
+    (F16, 40, 1024, 8192, 128, True, 0, 0),
+    # pass 2 of the recompute path
+    (F32, 192, 128, 128, 64, True, 0, 0),
+    (F32, 128, 256, 256, 64, False, 0, 0),
+    (F16, 256, 128, 128, 32, True, 0, 0),
+    (F16, 128, 128, 128, 32, True, SPLIT | DQ | KEYS, SPLIT),
+    (F16, 128, 512, 512, 32, True, 0, 0),
+    # nothing is split where the tiles do not fit LDS
+    (F32, 1, 512, 512, 256, True, 0, 0),
+]
+
+
+@pytest.mark.parametrize("case", ATTENTION, ids=str)
+def test_attention_forms(case):
+    *shape, want, fwd_full = case
+    assert _forms(*shape) & (SPLIT | LONG | DQ | KEYS if shape[4] <= 64 else SPLIT | LONG | DQ) == want
+    with _native.tail_skip(False):
+        assert _forms(*shape) & (SPLIT | LONG) == fwd_full
+
+
+def test_attention_forms_grouped_heads_and_errors():
+    """Query heads count in the row blocks, key heads in pass 2's key blocks and the group in its tiles."""
+    assert _forms(BF16, 8, 1741, 1741, 128, True, group=4) == LONG
+    assert _forms(F32, 8, 1024, 1024, 64, True, B=4, group=4) & KEYS
+    assert not _forms(F32, 32, 1024, 1024, 64, True, B=4) & (SPLIT | LONG | DQ)
+    lib = _native.lib()
+    assert lib.co_alibi_attention_forms(3, 1, 1, 1, 1, 1, 64, 1) == -1
+    assert lib.co_alibi_attention_forms(F16, 1, 3, 2, 1, 1, 64, 1) == -1
+    assert lib.co_alibi_attention_forms(F16, 1, 1, 1, 1, 1, 80, 1) == -1
