@@ -25,6 +25,7 @@
 // totals, exactly the totals pass 1 computes (the same sigmoids summed in the same order), so
 // the difference pass 1 takes is exact up to one rounding.
 #include <algorithm>
+#include <type_traits>
 
 #include "coalibi_common.h"
 #include "coalibi_kernels.h"
@@ -605,10 +606,9 @@ __device__ __forceinline__ void fwd_row_block(const FwdArgs& args, int bh, int q
   }
 }
 
-// Two work-groups per CU where the registers allow it: fp32 at D = 64 fits 256 (allowed more it takes 267,
-// which leaves one: B4 H16 D64 n 2048 289 us against 253, n 4096 807 against 690).
-template <typename T, int D, bool CAUSAL, bool SKIP, bool PLAIN>
-__global__ __launch_bounds__(256, D * sizeof(T) > 256 ? 1 : 2) void coalibi_fwd_kernel(FwdArgs args) {
+// PER_CU: work-groups per CU that the registers are to allow.
+template <typename T, int D, bool CAUSAL, bool SKIP, bool PLAIN, int PER_CU>
+__global__ __launch_bounds__(256, PER_CU) void coalibi_fwd_kernel(FwdArgs args) {
   using C = FwdCfg<T, D>;
   __shared__ __align__(16) T sK[kFwdBN * C::LDK];
   __shared__ __align__(16) T sV[C::V_ELEMS];
@@ -946,11 +946,19 @@ hipError_t launch_fwd(const FwdArgs& a, hipStream_t stream) {
   }
   const bool plain = is_contiguous(a.ql, a.Hq, a.Sq, D) && is_contiguous(a.ol, a.Hq, a.Sq, D) &&
                      is_contiguous(a.kl, a.Hkv, a.Skv, D) && is_contiguous(a.vl, a.Hkv, a.Skv, D);
-  auto* const kernel = a.knorm != nullptr
-                           ? (plain ? coalibi_fwd_kernel<T, D, CAUSAL, true, true>
-                                    : coalibi_fwd_kernel<T, D, CAUSAL, true, false>)
-                           : (plain ? coalibi_fwd_kernel<T, D, CAUSAL, false, true>
-                                    : coalibi_fwd_kernel<T, D, CAUSAL, false, false>);
+  constexpr int kPerCU = D * sizeof(T) > 256 ? 1 : 2;
+  auto choose = [&](auto per_cu) {
+    constexpr int N = decltype(per_cu)::value;
+    return a.knorm != nullptr ? (plain ? coalibi_fwd_kernel<T, D, CAUSAL, true, true, N>
+                                       : coalibi_fwd_kernel<T, D, CAUSAL, true, false, N>)
+                              : (plain ? coalibi_fwd_kernel<T, D, CAUSAL, false, true, N>
+                                       : coalibi_fwd_kernel<T, D, CAUSAL, false, false, N>);
+  };
+  auto* kernel = choose(std::integral_constant<int, kPerCU>{});
+  if constexpr (has_roomy_form(sizeof(T), D)) {
+    if (roomy_fwd_grid(grid, CAUSAL ? std::min(a.Sq, a.Skv) : a.Skv, CAUSAL, a.every_key))
+      kernel = choose(std::integral_constant<int, 1>{});
+  }
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, stream, f);
   return hipGetLastError();
 }

@@ -303,6 +303,17 @@ inline bool split_fwd_long_rows(int elem, int D, long long row_blocks, int keys)
   return row_blocks <= std::min(keys * 2 / 5, 768);
 }
 
+// Forward, whole-block form, fp32 at D = 64: asked for one work-group per CU it takes 267 registers, for two 256.
+// The roomier code is the faster one where the tail skip's uneven blocks hardly ever give a CU two.  Two per CU -> one:
+//   n 512: 384 blocks 70.6 -> 71.9;  n 1024: 384 111 -> 96, 576 122 -> 113, 640 122 -> 123, 1024 176 -> 196
+//   n 2048: 448 168 -> 167, 704 205 -> 180, 1024 253 -> 287;  n 4096: 768 378 -> 344, 1024 431 -> 418;  n 8192: 512 700 -> 667
+//   non-causal  n 1024: 384 blocks 107 -> 97, 448 120 -> 124;  n 2048: 448 197 -> 181, 512 216 -> 212, 768 221 -> 237
+//   tail skip off: 2 to 4 % slower everywhere
+constexpr bool has_roomy_form(int elem, int D) { return elem == 4 && D == 64; }
+inline bool roomy_fwd_grid(long long row_blocks, int keys, bool causal, bool every_key) {
+  return !every_key && keys >= 896 && row_blocks <= (causal ? std::min(448 + keys / 8, 1024) : 400);
+}
+
 // Backward pass 1.  At D = 128 in 16-bit types a step waits longer for its own K, whose tile the dQ product
 // reads last (and reloads spilled registers), and the limit is lower.  Both passes, pass 1 whole -> split:
 //   fp16 D 64   n 64: 64 blocks 11.9 -> 12.7;  n 96: 64 15.5 -> 14.5, 128 16.1 -> 17.6;  n 128: 128 17.8 -> 17.3;  n 256: 128 25.0 -> 21.3

@@ -69,5 +69,7 @@ def kernels(tmp_path_factory):
 def test_two_work_groups_per_cu(kernels, kernel, size, dims):
     for D in dims:
         built = kernels[(kernel, size, D)]
+        if (kernel, size, D) == ("fwd", 4, 64):  # also built for one per CU, for grids that give a CU one
+            built = [k for k in built if "Li1EEEv" not in k[0]]
         for name, regs, lds in built:
             assert regs <= 256 and lds <= 80 * 1024, (name, regs, lds)
