@@ -463,8 +463,8 @@ __global__ __launch_bounds__(256, D * sizeof(T) > 256 ? 1 : 2) void coalibi_bwd_
   // The four parts of a row block run on one XCD (ids 8 apart) and share its K and V in L2.
   const int i = (blockIdx.x >> 5) * 8 + (blockIdx.x & 7), part = (blockIdx.x >> 3) & 3;
   if (i >= items) return;
-  // Every block of a head on one XCD: on a grid this small its K and V staying in one L2 counts for
-  // more than an even spread of the heads (n 512 to 2048: up to 15 % faster than the sorted order).
+  // A head's blocks on one XCD (with a multiple of 8 heads; on two with 4 or 12, on four with 2 or 6): on a
+  // grid this small its K and V staying in one L2 counts for more than an even spread of the heads (n 512 to 2048: up to 15 % faster than the sorted order).
   const WorkItem item = lpt_item(i, args.B * args.Hq, 1 << 30);
   const int bh = item.head, qb = nQB - 1 - item.rank;
   const int q0 = qb * kBM + part * kSplitRows;

@@ -517,11 +517,11 @@ constexpr int kSplitWaves = 4;
 
 // Buffer-to-LDS DMA of the kWaveKeys rows row0.. of a row-major [nrows][D] matrix into
 // one wavefront's tile (the layout of DmaTile<T, D, kWaveKeys, LD, 1, PERM>): every
-// instruction reads 64 consecutive 16-byte chunks.  STREAM: non-temporal, for data read once.
+// instruction reads 64 consecutive 16-byte chunks, non-temporal (the decode reads a cache once per step).
 // Rows past nrows, pad chunks and the tail after the last row land as zeros.  The source offsets
 // are recomputed from an opaque copy of the lane index at every issue; hoisted out of the chunk
 // loop they would hold a register per instruction for the whole kernel.
-template <typename T, int D, int LD, bool PERM, bool STREAM>
+template <typename T, int D, int LD, bool PERM>
 __device__ __forceinline__ void dma_wave_rows(const T* base, int row0, int nrows, T* lds, int lane) {
   using Tile = DmaTile<T, D, kWaveKeys, LD, 1, PERM>;
   const __amdgpu_buffer_rsrc_t r = tile_rsrc(base + (size_t)row0 * D, min(max(nrows - row0, 0), kWaveKeys) * D);
@@ -532,11 +532,7 @@ __device__ __forceinline__ void dma_wave_rows(const T* base, int row0, int nrows
     const int ch = m * 64 + ln, row = ch / Tile::CPR, j = ch - row * Tile::CPR;
     const int src = PERM ? (row & ~31) + kRowOfReg(row & 31) : row;
     const bool in_tile = row < kWaveKeys && j < D / Tile::CH;
-    const int off = in_tile ? (src * D + j * Tile::CH) * (int)sizeof(T) : 0x40000000;
-    if constexpr (STREAM)
-      dma16_to_lds_nt(r, lds + m * 64 * Tile::CH, off);
-    else
-      dma16_to_lds(r, lds + m * 64 * Tile::CH, off);
+    dma16_to_lds_nt(r, lds + m * 64 * Tile::CH, in_tile ? (src * D + j * Tile::CH) * (int)sizeof(T) : 0x40000000);
   }
 }
 

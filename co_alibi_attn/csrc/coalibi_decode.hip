@@ -202,10 +202,10 @@ __global__ __launch_bounds__(kDecWaves * 64, (D > 128 || sizeof(T) == 4) ? 1 : 2
   // the rate).  K rows are permuted (LDS row R holds key kRowOfReg(R)) so that register r of
   // lane l of S^T holds key 16*(l/32) + r of the wavefront.
   auto issue_k = [&](int c) {
-    dma_wave_rows<T, D, C::LDK, true, true>(kbase, c * kDecodeChunkKeys + wave * kWaveKeys, L, sKw, lane);
+    dma_wave_rows<T, D, C::LDK, true>(kbase, c * kDecodeChunkKeys + wave * kWaveKeys, L, sKw, lane);
   };
   auto issue_v = [&](int c) {
-    dma_wave_rows<T, D, C::LDV, false, true>(vbase, c * kDecodeChunkKeys + wave * kWaveKeys, L, sVw, lane);
+    dma_wave_rows<T, D, C::LDV, false>(vbase, c * kDecodeChunkKeys + wave * kWaveKeys, L, sVw, lane);
   };
   issue_k(c_last);
   issue_v(c_last);

@@ -885,7 +885,8 @@ __global__ __launch_bounds__(256, D * sizeof(T) > 256 ? 1 : 2) void coalibi_fwd_
     part = rest < 0 ? 0 : 1 + (rest >> 3) % 3;
   }
   if (i >= items) return;
-  // by_head: every block of a head on one XCD, where its K and V stay in one L2 (fp32, B2 H12 n 1000:
+  // by_head: a head's blocks on one XCD where the heads are a multiple of 8 (on two with 4 or 12, on four
+  // with 2 or 6), where its K and V stay in one L2 (fp32, B2 H12 n 1000:
   // 78.3 -> 58.4 us against the sorted order; n 512 to 2048 fp16: 3 to 13 %).  Non-causal heads differ
   // more in work, and the sorted order is ahead (333 x 2047: 41.2 against 48.8), as it is on larger grids.
   const WorkItem item = !by_head && args.row_order ? table_item(args.row_order, i, args.B * args.Hq, items)
