@@ -59,7 +59,9 @@ STORE_KERNELS = ("coalibi_fwd_kernel", "coalibi_bwd_dq_kernel", "coalibi_bwd_dkd
 DECODE_KERNELS = ("coalibi_decode_split_kernel", "coalibi_decode_merge_kernel")
 # co_alibi_fwd launches the key-norm kernel (max |k| per key chunk, for the tail skip) before
 # the forward kernel; per-launch timings of "coalibi_fwd_kernel" through the C ABI include it.
-NAMED_KERNELS = KERNELS + STORE_KERNELS[2:] + DECODE_KERNELS + ("coalibi_key_norm_kernel",)
+FORM_KERNELS = ("coalibi_fwd_split_kernel", "coalibi_bwd_dq_split_kernel", "coalibi_bwd_dkdv_key_kernel",
+                "coalibi_bwd_dkdv_f32_kernel")
+NAMED_KERNELS = KERNELS + STORE_KERNELS[2:] + FORM_KERNELS + DECODE_KERNELS + ("coalibi_key_norm_kernel",)
 # The two --pmc passes of the counter summary: at most 8 SQ and 2 GRBM counters each.
 COUNTER_PASSES = (
     ("SQ_INSTS_VALU", "SQ_INSTS_VALU_TRANS_F32", "SQ_INSTS_MFMA", "SQ_INSTS_LDS", "SQ_INSTS_SALU", "SQ_WAVES",
@@ -402,8 +404,8 @@ FULL_WORK = " (full work)"
 
 def _mode_split(trace_rows):
     """Per-dispatch rows of a kernel trace, in time order, with each attention kernel named by the
-    tail-skip mode it ran in: the forward's template says it (its last argument, the skip), and
-    the backward kernels take the mode of the latest forward before them.  Returns
+    tail-skip mode it ran in: the forward's template says it (its second truth value, after the
+    causal mask), and the backward kernels take the mode of the latest forward before them.  Returns
     {name: [duration ns, ...]}."""
     import re
 
@@ -412,12 +414,11 @@ def _mode_split(trace_rows):
     for r in sorted(trace_rows, key=lambda r: int(r["Start_Timestamp"])):
         name = r["Kernel_Name"]
         short = _short(name)
-        if short == "coalibi_fwd_kernel":  # the last template argument, demangled or mangled
-            m = re.search(r"coalibi_fwd_kernel<[^>]*?,\s*(true|false)\s*>", name) or \
-                re.search(r"coalibi_fwd_kernelI.*Lb([01])E", name)
+        if short in ("coalibi_fwd_kernel", "coalibi_fwd_split_kernel"):  # demangled or mangled
+            m = re.search(short + r"<[^>]*?(?:true|false),\s*(true|false)\s*[,>]", name) or \
+                re.search(short + r"I.*?Lb[01]ELb([01])E", name)
             full = m is not None and m.group(1) in ("false", "0")
-        if short in ("coalibi_fwd_kernel", "coalibi_bwd_dq_kernel", "coalibi_bwd_dkdv_kernel",
-                     "coalibi_bwd_dkdv_store_kernel") and full:
+        if full and (short in FORM_KERNELS or short in KERNELS or short in STORE_KERNELS):
             short += FULL_WORK
         out[short].append(int(r["End_Timestamp"]) - int(r["Start_Timestamp"]))
     return out

@@ -160,3 +160,30 @@ def test_issued_products_match_the_kernel_loops():
     fwd, _ = profiling.attention_flops(4, 16, 4096, 4096, 128)
     issued = 64 * per_head * 32 * profiling.K16_FLOPS
     assert 1.0 < issued / fwd < 1.03
+
+
+def test_trace_rows_name_the_skip_mode():
+    """The forward's second truth value is the tail skip, whatever arguments follow it; the backward kernels
+    take the latest forward's mode, in every form."""
+    anon = "void coalibi::(anonymous namespace)::"
+    names = [
+        (anon + "coalibi_fwd_kernel<_Float16, 128, true, true, false, 2>(coalibi::FwdArgs)", False),
+        (anon + "coalibi_bwd_dq_kernel<_Float16, 128, true, true, false>(coalibi::BwdArgs)", False),
+        (anon + "coalibi_fwd_kernel<_Float16, 128, false, false, true, 2>(coalibi::FwdArgs)", True),
+        (anon + "coalibi_bwd_dkdv_store_kernel<_Float16, 128, false, true, true>(coalibi::BwdArgs)", True),
+        ("_ZN7coalibi12_GLOBAL__N_118coalibi_fwd_kernelIDF16bLi64ELb1ELb1ELb0ELi2EEEvNS_7FwdArgsE", False),
+        ("_ZN7coalibi12_GLOBAL__N_118coalibi_fwd_kernelIDF16bLi64ELb1ELb0ELb1ELi2EEEvNS_7FwdArgsE", True),
+        (anon + "coalibi_bwd_dq_split_kernel<float, 64, true, false>(coalibi::BwdArgs, int)", True),
+        (anon + "coalibi_bwd_dkdv_key_kernel<float, 64, true>(coalibi::BwdArgs)", True),
+        ("_ZN7coalibi12_GLOBAL__N_124coalibi_fwd_split_kernelIDF16_Li64ELb1ELb1EEEvNS_7FwdArgsEiNS0_9SplitRuleEb", False),
+        (anon + "coalibi_fwd_split_kernel<float, 64, false, false>(coalibi::FwdArgs, int, SplitRule, bool)", True),
+        (COPY, False),
+    ]
+    for i, (name, full) in enumerate(names):  # one row more at a time: the last one's name
+        rows = [dict(Start_Timestamp=str(j), End_Timestamp=str(j + 1), Kernel_Name=n) for j, (n, _) in
+                enumerate(names[:i + 1])]
+        before = profiling._mode_split(rows[:-1])
+        after = profiling._mode_split(rows)
+        (added,) = [k for k in after if len(after[k]) > len(before.get(k, []))]
+        assert added.endswith(profiling.FULL_WORK) == full, (name, added)
+        assert name == COPY or added.split(" ")[0] in name and "..." not in added
