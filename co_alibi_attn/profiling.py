@@ -224,10 +224,18 @@ class KernelSet:
         return self.stats[4:4 + n].view(torch.int32).view(w.batch * w.heads_q, -1).cpu().numpy()
 
     def issued_flops(self, name: str, kstart=None) -> float | None:
-        """Flops the MFMA units execute in one launch of a kernel, from the recorded kstart."""
+        """Flops the MFMA units execute in one launch of a kernel, from the recorded kstart; None where the
+        launch takes a split form, whose work issued_k16 does not count."""
+        from co_alibi_attn import _native
+
         w = self.w
         if name == "coalibi_fwd_kernel (inference)":
             name = "coalibi_fwd_kernel"
+        split = {"coalibi_fwd_kernel": 3, "coalibi_bwd_dq_kernel": 4}.get(name, 0)
+        with _native.tail_skip(self.skip):
+            if _native.lib().co_alibi_attention_forms(_native.DTYPE_CODES[w.dtype], w.batch, w.heads_q, w.heads_kv,
+                                                      w.seq, w.seq, w.head_dim, int(w.causal)) & split:
+                return None
         n = issued_k16(name, self.kstart() if kstart is None else kstart, w.batch, w.heads_q, w.heads_kv, w.seq,
                        w.seq, w.head_dim, w.causal)
         return None if n is None else n * K16_FLOPS

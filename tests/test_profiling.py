@@ -187,3 +187,15 @@ def test_trace_rows_name_the_skip_mode():
         (added,) = [k for k in after if len(after[k]) > len(before.get(k, []))]
         assert added.endswith(profiling.FULL_WORK) == full, (name, added)
         assert name == COPY or added.split(" ")[0] in name and "..." not in added
+
+
+def test_issued_flops_of_split_launches_are_not_counted():
+    """The validation workload's grid is split (its products are not those of whole blocks); the headline's is not."""
+    from co_alibi_attn.workloads import WORKLOADS
+
+    for name, split in (("cpu", True), ("headline", False)):
+        ks = object.__new__(profiling.KernelSet)
+        ks.w, ks.skip = WORKLOADS[name], True
+        zeros = np.zeros((ks.w.batch * ks.w.heads_q, (ks.w.seq + 127) // 128), dtype=np.int32)
+        for kernel in ("coalibi_fwd_kernel", "coalibi_bwd_dq_kernel"):
+            assert (ks.issued_flops(kernel, zeros) is None) == split
