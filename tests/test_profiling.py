@@ -191,6 +191,8 @@ def test_trace_rows_name_the_skip_mode():
 
 def test_issued_flops_of_split_launches_are_not_counted():
     """The validation workload's grid is split (its products are not those of whole blocks); the headline's is not."""
+    import numpy as np
+
     from co_alibi_attn.workloads import WORKLOADS
 
     for name, split in (("cpu", True), ("headline", False)):
