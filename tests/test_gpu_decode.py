@@ -322,3 +322,36 @@ def test_decode_noalloc_plan_past_the_scratch():
         ro, _ = ref.forward(q[b:b + 1, :32].float().cpu(), k[b:b + 1, :1, :lens[b]].float().cpu(),
                             v[b:b + 1, :1, :lens[b]].float().cpu(), lam, causal=False, scale=1 / math.sqrt(D))
         check(f"o[{b}]", o[b:b + 1, :32].unsqueeze(2), ro, TOL[dtype])
+
+
+# The split plan's edges at bounds where it decides (asserted): as PLAN_CASES, (name, lens, Hq, Hkv, cap, D).
+LONG_PLAN_CASES = [
+    ("B70", [0] + [170 * i % 2500 for i in range(68)] + [0], 8, 2, 2500, 64),
+    ("one_long", [0, 0, 34000, 0, 0], 8, 2, 34000, 64),
+    ("chunk_edges", [127, 128, 129, 255, 256, 257, 384, 385], 6, 3, 26000, 32),
+    ("all_empty", [0, 0, 0], 4, 4, 28000, 64),
+    ("equal", [2304, 2304, 2304], 128, 64, 2304, 64),
+    ("past_the_bound", [5000, 2560, 1, -3], 256, 64, 2560, 32),
+]
+
+
+@pytest.mark.parametrize("case", LONG_PLAN_CASES, ids=lambda c: c[0])
+def test_decode_length_plan(case):
+    name, lens, Hq, Hkv, cap, D = case
+    assert _native.lib().co_alibi_decode_splits(1, len(lens), Hkv, cap, D, 1) < -1
+    print(f"case {name}", flush=True)
+    q, k, v = cache_inputs(len(lens), Hq, Hkv, cap, cap, D, torch.float16, seed=37)
+    held = [min(max(n, 0), cap) for n in lens]
+    for b, n in enumerate(held):
+        k[b, :, n:] = 100.0
+        v[b, :, n:] = -1000.0
+    seq = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    o, lse = co_alibi_decode(q.to(DEV), k.to(DEV), v.to(DEV), seq_len=seq, return_lse=True)
+    torch.cuda.synchronize()
+    for b, n in enumerate(held):
+        if n == 0:
+            assert not o[b].any() and torch.isneginf(lse[b]).all()
+            continue
+        ro, rlse = oracle_decode(q[b:b + 1], k[b:b + 1], v[b:b + 1], n)
+        check(f"o[{b}] (len {n})", o[b:b + 1], ro, TOL[torch.float16])
+        check(f"lse[{b}] (len {n})", lse[b:b + 1], rlse, TOL[torch.float16])
