@@ -185,6 +185,8 @@ int co_alibi_attention_forms(int dtype, int batch, int heads_q, int heads_kv, in
     forms |= CO_ALIBI_FORM_FWD_SPLIT;
   else if (fits && causal && !every_key && coalibi::split_fwd_long_rows(elem, head_dim, row_blocks, keys))
     forms |= CO_ALIBI_FORM_FWD_LONG_ROWS;
+  else if (coalibi::has_roomy_form(elem, head_dim) && coalibi::roomy_fwd_grid(row_blocks, keys, causal != 0, every_key))
+    forms |= CO_ALIBI_FORM_FWD_ROOMY;
   if (fits && coalibi::split_dq_grid(elem, head_dim, row_blocks, keys, causal != 0)) forms |= CO_ALIBI_FORM_DQ_SPLIT;
   if (coalibi::has_key_form(elem, head_dim) &&
       coalibi::use_key_form(elem, head_dim, static_cast<long long>((seq_kv + 127) / 128) * batch * heads_kv,

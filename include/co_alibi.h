@@ -160,12 +160,13 @@ int co_alibi_bwd_dkdv(int dtype, const void* dout, const void* q, const void* k,
 /* Which kernel forms calls of this shape take under the current tail-skip setting, or -1 for an
  * unsupported one: on small grids the forward and backward pass 1 split a row block over four
  * work-groups (which rounds sums in another order), the forward also the longer half of the row blocks on
- * middle grids, and the recompute path's pass 2 works on 32 keys per work-group.  No counterpart in the
- * reference; it serves tests and measurements. */
+ * middle grids, the fp32 forward at head dim 64 has two register budgets, and the recompute path's pass 2
+ * works on 32 keys per work-group.  No counterpart in the reference; it serves tests and measurements. */
 #define CO_ALIBI_FORM_FWD_SPLIT 1
 #define CO_ALIBI_FORM_FWD_LONG_ROWS 2
 #define CO_ALIBI_FORM_DQ_SPLIT 4
 #define CO_ALIBI_FORM_DKDV_KEYS 8
+#define CO_ALIBI_FORM_FWD_ROOMY 16
 int co_alibi_attention_forms(int dtype, int batch, int heads_q, int heads_kv, int seq_q, int seq_kv,
                              int head_dim, int causal);
 

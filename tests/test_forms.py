@@ -159,3 +159,14 @@ def test_attention_forms_grouped_heads_and_errors():
     assert lib.co_alibi_attention_forms(3, 1, 1, 1, 1, 1, 64, 1) == -1
     assert lib.co_alibi_attention_forms(F16, 1, 3, 2, 1, 1, 64, 1) == -1
     assert lib.co_alibi_attention_forms(F16, 1, 1, 1, 1, 1, 80, 1) == -1
+
+
+def test_roomy_forward():
+    """fp32 at head dim 64: the register budget of one work-group per CU on grids that give a CU one."""
+    for H, n, causal, B, want in ((36, 1024, True, 2, 16), (40, 1024, True, 2, 0), (22, 2048, True, 2, 16),
+                                  (32, 2048, True, 2, 0), (24, 1024, False, 2, 16), (32, 1024, False, 2, 0),
+                                  (48, 512, True, 2, 0), (16, 1024, True, 2, 0)):
+        assert _forms(F32, H, n, n, 64, causal, B=B) & 16 == want, (H, n, causal)
+        assert not _forms(F16, H, n, n, 64, causal, B=B) & 16 and not _forms(F32, H, n, n, 32, causal, B=B) & 16
+        with _native.tail_skip(False):
+            assert not _forms(F32, H, n, n, 64, causal, B=B) & 16

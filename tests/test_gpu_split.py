@@ -138,6 +138,25 @@ def test_forward_record_shows_the_form(slope, split):
     assert kstart[0].any() != split, kstart
 
 
+@pytest.mark.parametrize("H,S,causal", [(36, 1000, True), (20, 900, False)], ids=["causal", "full"])
+def test_roomy_fp32_forward(H, S, causal):
+    """The fp32 forward at head dim 64 under the register budget of one work-group per CU; four heads checked, and
+    the backward that follows its record."""
+    assert _native.lib().co_alibi_attention_forms(0, 1, H, H, S, S, 64, int(causal)) & 19 == 16
+    q, k, v, do = rand_inputs(1, H, H, S, S, 64, torch.float32, seed=17)
+    do = do * 0.25
+    lam = torch.tensor([2.0, 0.05, 0.01, 0.0] + [0.3] * (H - 4))
+    qd, kd, vd = (t.to(DEV).requires_grad_() for t in (q, k, v))
+    o = CoALIBIAttention.apply(qd, kd, vd, lam.to(DEV), causal, 0.125)
+    o.backward(do.to(DEV))
+    torch.cuda.synchronize()
+    got = tuple(t.detach()[:, :4].float().cpu() for t in (o, qd.grad, kd.grad, vd.grad))
+    ins = [t[:, :4] for t in (q, k, v)]
+    ro, _ = ref.forward(*ins, lam[:4], causal=causal, scale=0.125)
+    want = (ro, *ref.backward(do[:, :4], *ins, lam[:4], causal=causal, scale=0.125))
+    assert_parity(got, want, TOL[torch.float32], "roomy", torch.float32)
+
+
 # (Hq, S, D, dtype, causal): a batch of 17 of these takes the whole-block pass 1, one of them alone the split form.
 PASS1_CASES = [
     (4, 250, 64, torch.float16, True),
