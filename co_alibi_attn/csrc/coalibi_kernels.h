@@ -341,7 +341,7 @@ inline bool split_dq_grid(int elem, int D, long long row_blocks, int keys, bool 
 // row block and query head) is long enough to carry its prologue and merge; in 16-bit types the 128-key form
 // is ahead again once its work-groups fill the GPU.  Both passes, 128-key -> 32-key, by key blocks and tiles:
 //   fp32 D 64   128 x 1: 52.6 -> 45.1, 192 x 1 62 -> 74, 256 x 1 65 -> 96, 256 x 2 100 -> 101 (non-causal 99 -> 111), 256 x 4 180 -> 155
-//          384 x 8: 344 -> 308, 512 x 8 397 -> 414, 512 x 4 248 -> 272, 640 x 16 708 -> 645, 1024 x 16 1194 -> 1153, 64 x 64 1761 -> 551
+//          384 x 8: 344 -> 308, 512 x 8 397 -> 414, 1024 x 8 734 -> 746, 512 x 4 248 -> 272, 640 x 16 708 -> 645, 1024 x 16 1194 -> 1153, 64 x 64 1761 -> 551
 //   fp32 D 32   192 x 1: 41 -> 44, 256 x 2 64 -> 56, 512 x 8 249 -> 218, 1024 x 16 567 -> 538
 //   fp16 D 32   128 x 1: 17.3 -> 14.2, 192 x 1 23 -> 29, 256 x 2 29.4 -> 28.4, 256 x 4 49 -> 40, 512 x 4 52 -> 59, 512 x 8 89 -> 83
 //          640 x 16: 164 -> 129, 1024 x 16 175 -> 188, 768 x 3 51 -> 64
@@ -349,7 +349,7 @@ constexpr bool has_key_form(int elem, int D) { return D * elem <= (elem == 2 ? 6
 inline bool use_key_form(int elem, int D, long long key_blocks, int tiles) {
   if (key_blocks <= 128) return true;
   if (key_blocks <= 256) return tiles >= (elem == 4 && D > 32 ? 3 : 2);
-  return tiles >= 8 && (elem == 4 || key_blocks <= 640);
+  return tiles >= (elem == 4 && D > 32 && key_blocks > 448 ? 12 : 8) && (elem == 4 || key_blocks <= 640);
 }
 
 // Forward; with a.knorm (the tail skip) it first launches the key-norm kernel that fills it.

@@ -137,6 +137,8 @@ ATTENTION = [
     (F16, 256, 128, 128, 32, True, 0, 0),
     (F16, 128, 128, 128, 32, True, SPLIT | DQ | KEYS, SPLIT),
     (F16, 128, 512, 512, 32, True, 0, 0),
+    (F32, 64, 1024, 1024, 64, True, 0, 0),
+    (F32, 48, 1024, 1024, 64, True, KEYS | 16, 0),
     # nothing is split where the tiles do not fit LDS
     (F32, 1, 512, 512, 256, True, 0, 0),
 ]
@@ -145,7 +147,7 @@ ATTENTION = [
 @pytest.mark.parametrize("case", ATTENTION, ids=str)
 def test_attention_forms(case):
     *shape, want, fwd_full = case
-    assert _forms(*shape) & (SPLIT | LONG | DQ | KEYS if shape[4] <= 64 else SPLIT | LONG | DQ) == want
+    assert _forms(*shape) & (31 if want & 16 else SPLIT | LONG | DQ | KEYS) == want
     with _native.tail_skip(False):
         assert _forms(*shape) & (SPLIT | LONG) == fwd_full
 
