@@ -516,16 +516,16 @@ struct DecodeRule {
   // 8.4, D 128 bf16 at 2 10.3 -> 9.0 (at 3 10.8 -> 10.9, with lengths of 1/8 to all of the bound 10.4 -> 8.7), fp32 D 32
   // at 2 9.2 -> 7.8; D 256 at 2 13.9 -> 14.1 and fp32 D 64 11.1 -> 11.4 (at 3 14.5 -> 18.3 and 11.3 -> 15.5).  With a
   // work-group per chunk above half the slots more splits cost more: at 3 chunks, units 100, D 128 12.7 -> 10.8, D 256
-  // 21.8 -> 17.9; units 192 fp32 D 64 22.7 -> 17.6 (units 128 16.8 -> 17.3; ragged, D 256 16.5 -> 18.7).  Above half the slots in units two splits take two rounds: units
-  // 288, 6 chunks, D 128 29.5 -> 28.0, 5 chunks, D 256 61 -> 57 (8: 79 -> 84), 3 chunks, fp32 D 128 62 -> 55 (4: 64 ->
-  // 69); ragged lengths of at most 8 chunks take 5 to 30 % less on average.  From 5/6 of the slots on one split
-  // loses nothing: units 432, D 128, 8 chunks 43.4 -> 38.7, 32 chunks 157 -> 147 (units 384: 124 -> 135), but
-  // D 32 from 16 chunks on (units 448, 32 chunks 65.9 -> 67.6).
+  // 21.8 -> 17.9; units 192 fp32 D 64 22.7 -> 17.6 (units 128 16.8 -> 17.3; ragged, D 256 16.5 -> 18.7).  Above half
+  // the slots in units two splits take two rounds: units 288, 6 chunks, D 128 29.5 -> 28.0, 5 chunks, D 256 61 -> 57
+  // (8: 79 -> 84), 3 chunks, fp32 D 128 62 -> 55 (4: 64 -> 69); ragged lengths of at most 8 chunks take 5 to 30 % less
+  // on average.  From 5/6 of the slots on one split loses nothing: units 432, D 128, 8 chunks 43.4 -> 38.7, 32 chunks
+  // 157 -> 147 (units 384: 124 -> 135), but D 32 from 16 chunks on (units 448, 32 chunks 65.9 -> 67.6).
   bool one_split(int chunks, bool ragged) const {
     if (units >= slots) return true;
     if (units * 6 >= slots * 5LL) return head_dim > 32 || chunks <= 16;
     if (units * 2 > slots) return chunks <= (ragged ? 8 : fp32 ? 3 : head_dim <= 128 ? 6 : 5);
-    if (chunks <= 3 && units * chunks * (ragged ? 4 : 6) > slots * 3LL) return true;
+    if (chunks <= 3 && units * chunks * (ragged || fp32 ? 4 : 6) > slots * 3LL) return true;
     if (fp32) return chunks <= (head_dim <= 32 ? 2 : 1);
     return chunks <= (head_dim <= 64 ? 3 : head_dim > 128 ? 1 : ragged ? 3 : 2);
   }
@@ -541,14 +541,14 @@ struct DecodeRule {
 
   // Splits of every sequence of a launch bound by `chunks` chunks.  Equal lengths: where even_splits' last
   // round is nearly empty, longer splits (decode_cps): units 100, 32 chunks, D 128 48 -> 39; units 36, 100 chunks,
-  // D 256 113 -> 89; short walks of the small types do not gain (units 100, 6 chunks, D 32 10.1 -> 11.3).  Up to half
-  // as long again from D 128 on (units 180, 125 chunks, D 128 294 -> 267; with a quarter 295), a quarter in
-  // the small types (units 210, 100 chunks, D 64 127 -> 133 with a half).
+  // D 256 113 -> 89.  Up to half as long again from D 128 on (units 180, 125 chunks, D 128 294 -> 267; with a quarter
+  // 295).  The small types gain from a quarter on few units (units 110, 32 chunks, D 64 33 -> 29), not on short
+  // walks (units 100, 6 chunks, D 32 10.1 -> 11.3) or more units (units 210, 125 chunks, D 32 122 -> 133).
   int splits(int chunks, bool ragged) const {
     if (one_split(chunks, ragged)) return 1;
     const bool small = !fp32 && head_dim <= 64;
     const int even = even_splits(chunks);
-    if (ragged || (small && chunks < 4 * even)) return even;
+    if (ragged || (small && (chunks < 4 * even || units * 4 >= slots))) return even;
     const int cps = coalibi::decode_cps(units * chunks, chunks, slots, coalibi::kMaxDecodeSplits, small ? 4 : 8, chunks - 1,
                                         [&](int c) { return units * ((chunks + c - 1) / c); });
     const int n = (chunks + cps - 1) / cps, own = (chunks + n - 1) / n;

@@ -46,6 +46,11 @@ DECODE = [
     # one sequence: a split per slot, or a chunk per split
     (BF16, 1, 8, 8192, 128, False, 64),
     (F16, 10, 10, 700, 32, False, 6),
+    (F16, 11, 10, 4076, 64, False, 4),
+    (F16, 21, 10, 16000, 32, False, 3),
+    (BF16, 18, 10, 16000, 128, False, 2),
+    (F32, 10, 10, 300, 64, False, 3),
+    (F32, 18, 10, 300, 64, False, 1),
 ]
 
 
